@@ -629,42 +629,50 @@ __host__ __device__ inline bool collision_box(const Vec3<T>& A, const Vec3<T>& B
 }
 
 // ---------------------------------------------------------------- underestimation
+// Normal of the plane of nearest points (R, O): normalize(R - O).  Eigen's
+// normalized() divides by the norm and leaves a zero vector as is.
+template <typename T>
+__host__ __device__ inline Vec3<T> plane_normal(const Vec3<T>& R, const Vec3<T>& O) {
+    const Vec3<T> RO = R - O;
+    const T z = sqnorm(RO);
+    Vec3<T> n = RO;
+    if (z > 0) {
+        const T s = vsqrt(z);
+        n = Vec3<T>{RO.x / s, RO.y / s, RO.z / s};
+    }
+    return n;
+}
+
 // One (link, obstacle) term of computeDistanceUnderestimation,
 // RealVectorSpace.cpp:420-427: min over the link's end points of the signed
-// distance to the plane through O with normal normalize(R - O), minus radius.
-// Eigen's normalized() divides by the norm and leaves a zero vector as is.
+// distance to the plane through O with normal n, minus radius.
+template <typename T>
+__host__ __device__ inline T plane_value(const Vec3<T>& P0, const Vec3<T>& P1, const Vec3<T>& O, const Vec3<T>& n,
+                                         T radius) {
+    return smin(dot(P0 - O, n), dot(P1 - O, n)) - radius;
+}
 template <typename T>
 __host__ __device__ inline T plane_term(const Vec3<T>& P0, const Vec3<T>& P1, const Vec3<T>& R, const Vec3<T>& O,
                                         T radius) {
-    const Vec3<T> RO = R - O;
-    const T z = sqnorm(RO);
-    Vec3<T> n = RO;
-    if (z > 0) {
-        const T s = vsqrt(z);
-        n = Vec3<T>{RO.x / s, RO.y / s, RO.z / s};
-    }
-    return smin(dot(P0 - O, n), dot(P1 - O, n)) - radius;
+    return plane_value(P0, P1, O, plane_normal(R, O), radius);
 }
 
-// The same term after the plane has moved towards the robot for delta_t at
-// the obstacle's maximal speed (AbstractTrajectory::
+// The plane after it has moved towards the robot for delta_t at the
+// obstacle's maximal speed (AbstractTrajectory::
 // computeDistanceUnderestimation, AbstractTrajectory.cpp:295-306): both
-// points shift by normalize(R - O) * max_vel * delta_t, then the plane is
-// rebuilt from the shifted points.
+// points shift by normalize(R - O) * max_vel * delta_t.
 template <typename T>
-__host__ __device__ inline T plane_term_moving(const Vec3<T>& P0, const Vec3<T>& P1, const Vec3<T>& R, const Vec3<T>& O,
-                                               T radius, T max_vel, T delta_t) {
-    const Vec3<T> RO = R - O;
-    const T z = sqnorm(RO);
-    Vec3<T> n = RO;
-    if (z > 0) {
-        const T s = vsqrt(z);
-        n = Vec3<T>{RO.x / s, RO.y / s, RO.z / s};
-    }
+__host__ __device__ inline void plane_move(Vec3<T>& R, Vec3<T>& O, T max_vel, T delta_t) {
+    const Vec3<T> n = plane_normal(R, O);
     const Vec3<T> dl{n.x * max_vel * delta_t, n.y * max_vel * delta_t, n.z * max_vel * delta_t};
-    const Vec3<T> R2{R.x + dl.x, R.y + dl.y, R.z + dl.z};
-    const Vec3<T> O2{O.x + dl.x, O.y + dl.y, O.z + dl.z};
-    return plane_term(P0, P1, R2, O2, radius);
+    R = Vec3<T>{R.x + dl.x, R.y + dl.y, R.z + dl.z};
+    O = Vec3<T>{O.x + dl.x, O.y + dl.y, O.z + dl.z};
+}
+template <typename T>
+__host__ __device__ inline T plane_term_moving(const Vec3<T>& P0, const Vec3<T>& P1, Vec3<T> R, Vec3<T> O, T radius,
+                                               T max_vel, T delta_t) {
+    plane_move(R, O, max_vel, delta_t);
+    return plane_term(P0, P1, R, O, radius);
 }
 
 }  // namespace rvs

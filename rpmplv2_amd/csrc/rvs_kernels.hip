@@ -562,6 +562,83 @@ __global__ __launch_bounds__(kBlock) void k_under(RobotDev rb, EnvDev env, Query
     if (stored) stored[c] = neg ? 0 : 1;
 }
 
+// The same against one nearest-point set shared by every configuration.  Bound
+// by VALU issue.  The planes (O and the unit normal, with its square root and
+// three divisions) depend on the set alone, so each workgroup computes them
+// once, a plane per thread, for as many links as a 32 KB tile of LDS holds
+// (all 102 of the xArm6 scene in 3 KB), and the lanes of a wave read them as
+// LDS broadcasts, about 21 instructions a plane; worked out again in every
+// lane, as k_under does for sets of their own, a plane takes about 75
+// (1,048,576 xArm6 configurations against 102 planes: 310 us a call so, 110 us
+// with the tile).  A pair the reference skips (|O| = MAX_DISTANCE) gets a NaN normal: its term is NaN
+// and never enters a minimum.  The running minimum starts at infinity, so
+// that its sign alone says whether any term was negative; MAX_DISTANCE, the
+// reference's start, enters last.
+constexpr int kPlaneTile = 1024;   // planes of a tile
+struct alignas(16) Plane {
+    Vec3<float> O;
+    float nx, ny, nz;
+    float pad[2];
+};
+static_assert(sizeof(Plane) == 32, "two 16-byte LDS reads per plane");
+
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_under_shared(
+    RobotDev rb, EnvDev env, QueryParams qp, const float* __restrict__ q, int64_t n, const float* __restrict__ np_ref,
+    float* d_out, float* prof_out, uint8_t* stored, const float* __restrict__ max_vel, float delta_t, int tile) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    Plane* planes = reinterpret_cast<Plane*>(smem);   // [tile][M]
+    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const bool live = g < n;
+    const int64_t c = live ? g : n - 1;   // every thread stages and meets the barriers
+    const int M = env.num_obj;
+    const int L = rb.num_links;
+    const float* qc = q + c * rb.num_dofs;
+    const float maxd = qp.maxd;
+    FKStream fk;
+    fk_init(fk);
+    Vec3<float> P0 = skel_point<float>(fk, rb, qc, 0);
+    float d = maxd;
+    bool neg = false;
+    for (int i0 = 0; i0 < L; i0 += tile) {
+        const int i1 = min(L, i0 + tile);
+        if (i0 > 0) __syncthreads();
+        for (int k = threadIdx.x; k < (i1 - i0) * M; k += blockDim.x) {
+            const int i = i0 + k / M, j = k % M;
+            const float* e = np_ref + ((int64_t)j * L + i) * 6;
+            Vec3<float> R{e[0], e[1], e[2]}, O{e[3], e[4], e[5]};
+            const bool skip = vnorm(O) == maxd;
+            if (max_vel) plane_move(R, O, max_vel[j], delta_t);
+            const Vec3<float> nv = plane_normal(R, O);
+            planes[k] = Plane{O, skip ? NAN : nv.x, skip ? NAN : nv.y, skip ? NAN : nv.z, {0.0f, 0.0f}};
+        }
+        __syncthreads();
+        for (int i = i0; i < i1; ++i) {
+            if (!__any(!neg)) break;   // a wave whose lanes are all settled waits at the tiles' barriers
+            const Vec3<float> P1 = skel_point<float>(fk, rb, qc, i + 1);
+            const float r = rb.radius[i];
+            const Plane* row = planes + (i - i0) * M;
+            float low = INFINITY;
+#pragma unroll 2
+            for (int j = 0; j < M; ++j) {
+                const Plane pl = row[j];
+                low = smin(low, plane_value(P0, P1, pl.O, Vec3<float>{pl.nx, pl.ny, pl.nz}, r));
+            }
+            neg = neg || low < 0;
+            const float prof = smin(maxd, low);
+            if (live && !neg && prof_out) prof_out[c * L + i] = prof;
+            d = smin(d, prof);
+            P0 = P1;
+        }
+    }
+    if (!live) return;
+    if (neg) {
+        if (prof_out) for (int k = 0; k < L; ++k) prof_out[c * L + k] = 0.0f;
+        d = 0.0f;
+    }
+    d_out[c] = d;
+    if (stored) stored[c] = neg ? 0 : 1;
+}
+
 // ---------------------------------------------------------------- self distance
 // Capsule-capsule distance of the robot's listed link pairs:
 // distanceLineSegToLineSeg - r_a - r_b (xArm6::computeCapsulesDistance,
@@ -897,22 +974,38 @@ hipError_t launch_is_valid(const RobotDev& rb, const EnvDev& env, const QueryPar
     return hipGetLastError();
 }
 
+namespace {
+
+// One shared set goes through the tiled planes, a set per configuration
+// through the lane's own.
+hipError_t launch_under(const RobotDev& rb, const EnvDev& env, const QueryParams& qp, const float* q, int64_t n,
+                        const float* np_ref, int64_t np_stride, const float* max_vel, float delta_t, float* d,
+                        float* profile, uint8_t* stored, hipStream_t st) {
+    if (n <= 0) return hipSuccess;
+    if (np_stride == 0) {
+        const int M = std::max(1, (int)env.num_obj);
+        const int tile = std::max(1, std::min((int)rb.num_links, kPlaneTile / M));
+        hipLaunchKernelGGL(k_under_shared, grid_for(n, kBlock), dim3(kBlock), (size_t)tile * M * sizeof(Plane), st, rb,
+                           env, qp, q, n, np_ref, d, profile, stored, max_vel, delta_t, tile);
+    } else {
+        hipLaunchKernelGGL(k_under, grid_for(n, kBlock), dim3(kBlock), 0, st, rb, env, qp, q, n, np_ref, np_stride, d,
+                           profile, stored, nullptr, 0, max_vel, delta_t);
+    }
+    return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_underestimation(const RobotDev& rb, const EnvDev& env, const QueryParams& qp, const float* q,
                                   int64_t n, const float* np_ref, int64_t np_stride, float* d, float* profile,
                                   uint8_t* stored, hipStream_t st) {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_under, grid_for(n, kBlock), dim3(kBlock), 0, st, rb, env, qp, q, n, np_ref, np_stride, d,
-                       profile, stored, nullptr, 0, nullptr, 0.0f);
-    return hipGetLastError();
+    return launch_under(rb, env, qp, q, n, np_ref, np_stride, nullptr, 0.0f, d, profile, stored, st);
 }
 
 hipError_t launch_underestimation_moving(const RobotDev& rb, const EnvDev& env, const QueryParams& qp, const float* q,
                                          int64_t n, const float* np_ref, int64_t np_stride, const float* max_vel,
                                          float delta_t, float* d, float* profile, uint8_t* stored, hipStream_t st) {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_under, grid_for(n, kBlock), dim3(kBlock), 0, st, rb, env, qp, q, n, np_ref, np_stride, d,
-                       profile, stored, nullptr, 0, max_vel, delta_t);
-    return hipGetLastError();
+    return launch_under(rb, env, qp, q, n, np_ref, np_stride, max_vel, delta_t, d, profile, stored, st);
 }
 
 hipError_t launch_underestimation_seg(const RobotDev& rb, const EnvDev& env, const QueryParams& qp, const float* q,

@@ -114,6 +114,41 @@ def test_underestimation(oracle, engine):
     assert ulps(d2, ud2).max() <= 2
 
 
+@pytest.mark.parametrize("dofs,boxes,n,far", [(6, 1, 1, False), (6, 16, 255, False), (10, 40, 257, False),
+                                              (22, 100, 300, False), (22, 1000, 65, False), (6, 17, 257, True),
+                                              (22, 100, 300, True), (22, 1000, 65, True)])
+def test_underestimation_shared_set_sizes(oracle, engine, dofs, boxes, n, far):
+    """One nearest-point set for all, from a single plane per link to sets
+    of several tiles (2,200 and 22,000 planes), ragged batches, a NaN joint,
+    a missing (NaN) pair and pairs the reference skips: stored flags equal,
+    values within 2 ulp (the device's double sine and cosine), profiles of
+    unstored configurations 0.  far: boxes out of the robot's reach, so that
+    the configurations are stored."""
+    rng = np.random.default_rng(90 + boxes)
+    rb = R.xarm6() if dofs == 6 else R.chain(rng.uniform(0.05, 0.1, dofs), radius=0.02, ground_included=1)
+    sc = W._boxes(rng, boxes, 0.02, 0.1, 2.5)
+    if far:
+        u = rng.normal(size=(boxes, 3))
+        sc = W.Scene(sc.dim, 4.0 * u / np.linalg.norm(u, axis=1, keepdims=True), sc.quat, sc.is_ground,
+                     sc.min_dist_tol)
+    q = rng.uniform(-0.3, 0.3, (n, dofs)).astype(np.float32)
+    q[n // 2, 1] = np.nan
+    P = R.skeleton_np(rb, np.zeros(dofs))[0]
+    ref = np.zeros((boxes, rb.num_links, 6), np.float32)
+    ref[..., :3] = 0.5 * (P[:-1] + P[1:])
+    ref[..., 3:] = np.clip(ref[..., :3], sc.aabb[:, None, :3], sc.aabb[:, None, 3:])
+    ref[0, 0] = np.nan
+    ref[-1, 1] = (0, 0, 0, 0, 0, -1000.0)
+    rid, eid = engine.load_robot(rb), engine.create_env(sc)
+    d, prof, st = engine.underestimation(rid, eid, q, ref)
+    od, oprof, ost = oracle.underestimation(rb, oracle.scene_of(sc), q, ref)
+    assert (st == ost).all()
+    assert ulps(d, od).max() <= 2
+    ok = st == 1
+    assert (ok.mean() > 0.9) if far else True
+    assert (prof[~ok] == 0).all() and (not ok.any() or ulps(prof[ok], oprof[ok]).max() <= 2)
+
+
 def test_self_distance(oracle, engine):
     rb = R.chain(np.random.default_rng(5).uniform(0.1, 0.3, 22), radius=0.04, self_collision=True)
     q = np.random.default_rng(6).uniform(-np.pi, np.pi, (8192, 22)).astype(np.float32)
