@@ -570,17 +570,8 @@ __global__ __launch_bounds__(kBlock) void k_under(RobotDev rb, EnvDev env, Query
 // LDS broadcasts, about 21 instructions a plane; worked out again in every
 // lane, as k_under does for sets of their own, a plane takes about 75
 // (1,048,576 xArm6 configurations against 102 planes: 310 us a call so, 110 us
-// with the tile).  A pair the reference skips (|O| = MAX_DISTANCE) gets a NaN normal: its term is NaN
-// and never enters a minimum.  The running minimum starts at infinity, so
-// that its sign alone says whether any term was negative; MAX_DISTANCE, the
-// reference's start, enters last.
+// with the tile).
 constexpr int kPlaneTile = 1024;   // planes of a tile
-struct alignas(16) Plane {
-    Vec3<float> O;
-    float nx, ny, nz;
-    float pad[2];
-};
-static_assert(sizeof(Plane) == 32, "two 16-byte LDS reads per plane");
 
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_under_shared(
     RobotDev rb, EnvDev env, QueryParams qp, const float* __restrict__ q, int64_t n, const float* __restrict__ np_ref,
@@ -602,27 +593,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     for (int i0 = 0; i0 < L; i0 += tile) {
         const int i1 = min(L, i0 + tile);
         if (i0 > 0) __syncthreads();
-        for (int k = threadIdx.x; k < (i1 - i0) * M; k += blockDim.x) {
-            const int i = i0 + k / M, j = k % M;
-            const float* e = np_ref + ((int64_t)j * L + i) * 6;
-            Vec3<float> R{e[0], e[1], e[2]}, O{e[3], e[4], e[5]};
-            const bool skip = vnorm(O) == maxd;
-            if (max_vel) plane_move(R, O, max_vel[j], delta_t);
-            const Vec3<float> nv = plane_normal(R, O);
-            planes[k] = Plane{O, skip ? NAN : nv.x, skip ? NAN : nv.y, skip ? NAN : nv.z, {0.0f, 0.0f}};
-        }
+        stage_planes(planes, np_ref, M, L, i0, i1, maxd, max_vel, delta_t);
         __syncthreads();
         for (int i = i0; i < i1; ++i) {
             if (!__any(!neg)) break;   // a wave whose lanes are all settled waits at the tiles' barriers
             const Vec3<float> P1 = skel_point<float>(fk, rb, qc, i + 1);
             const float r = rb.radius[i];
-            const Plane* row = planes + (i - i0) * M;
-            float low = INFINITY;
-#pragma unroll 2
-            for (int j = 0; j < M; ++j) {
-                const Plane pl = row[j];
-                low = smin(low, plane_value(P0, P1, pl.O, Vec3<float>{pl.nx, pl.ny, pl.nz}, r));
-            }
+            const float low = planes_min(planes + (i - i0) * M, M, P0, P1, r);
             neg = neg || low < 0;
             const float prof = smin(maxd, low);
             if (live && !neg && prof_out) prof_out[c * L + i] = prof;

@@ -31,10 +31,13 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "rvs_fk.hpp"
 #include "rvs_geometry.hpp"
 #include "rvs_internal.hpp"
 #include "rvs_radii.hpp"
+#include "rvs_stage.hpp"
 
 namespace rvs {
 
@@ -44,8 +47,8 @@ constexpr int32_t kAdvanced = 1, kTrapped = 2, kReached = 3;
 
 // Floats of one lane's LDS slice: skeleton of the start state and of the
 // current state (3 (D+1) each), radii column, current state, clearance
-// losses (D each).
-__host__ __device__ inline int spine_slice(int D) { return 6 * (D + 1) + 3 * D; }
+// losses, joint distances to the target (D each).
+__host__ __device__ inline int spine_slice(int D) { return 6 * (D + 1) + 4 * D; }
 
 // One lane's view of its LDS slice.
 struct SpineLane {
@@ -54,6 +57,7 @@ struct SpineLane {
     float* ac;
     float* qt;
     float* rp;
+    float* dl;
     int B, t;
     __device__ SpineLane(float* base, int D, int B_, int t_) : B(B_), t(t_) {
         sk0 = base;
@@ -61,15 +65,14 @@ struct SpineLane {
         ac = sk + (size_t)3 * (D + 1) * B;
         qt = ac + (size_t)D * B;
         rp = qt + (size_t)D * B;
+        dl = rp + (size_t)D * B;
     }
     __device__ float& Q(int k) const { return qt[k * B + t]; }
     __device__ float& RP(int k) const { return rp[k * B + t]; }
+    __device__ float& DL(int k) const { return dl[k * B + t]; }
     __device__ float& acc(int i) const { return ac[i * B + t]; }
     __device__ Vec3<float> P0(int k) const {
         return Vec3<float>{sk0[(3 * k) * B + t], sk0[(3 * k + 1) * B + t], sk0[(3 * k + 2) * B + t]};
-    }
-    __device__ Vec3<float> P(int k) const {
-        return Vec3<float>{sk[(3 * k) * B + t], sk[(3 * k + 1) * B + t], sk[(3 * k + 2) * B + t]};
     }
     __device__ void set_P(float* s, int k, const Vec3<float>& v) const {
         s[(3 * k) * B + t] = v.x;
@@ -78,32 +81,30 @@ struct SpineLane {
     }
 };
 
-// extendSpine from the state in the lane's Q (distance dq, link profile
-// pc(i)) towards qe; Q holds q_new afterwards.  Returns the status.
+// extendSpine from the state in the lane's Q, whose skeleton is in sk0
+// (distance dq, link profile pc(i)), towards qe; Q holds q_new afterwards.
+// Returns the status.
 template <typename PC>
 __device__ int32_t spine_run(const RobotDev& rb, const SpineLane& s, float dq, PC pc, const float* qe,
                              int num_iter, int expanded) {
     const int D = rb.num_dofs;
     if (dq <= 0.0f) return kTrapped;
-    {
-        FKStream fk;
-        fk_init(fk);
-        for (int k = 0; k <= D; ++k) {
-            const Vec3<float> v = skel_point<float>(fk, rb, s.qt + s.t, k, s.B);
-            s.set_P(s.sk0, k, v);
-            s.set_P(s.sk, k, v);
-        }
-    }
     for (int k = 0; k < D; ++k) s.RP(k) = 0.0f;
     float rho = 0.0f;
     int32_t status = kAdvanced;
-    auto P = [&](int k) { return s.P(k); };
+    const float* skel = s.sk0;   // the start state's skeleton, later the current state's
+    auto P = [&](int k) {
+        return Vec3<float>{skel[(3 * k) * s.B + s.t], skel[(3 * k + 1) * s.B + s.t], skel[(3 * k + 2) * s.B + s.t]};
+    };
     auto acc = [&](int i) -> float& { return s.acc(i); };
     for (int it = 1;; ++it) {
-        for (int i = 0; i < D; ++i) s.acc(i) = 0.0f;
+        for (int i = 0; i < D; ++i) {
+            s.acc(i) = 0.0f;
+            s.DL(i) = fabsf(qe[i] - s.Q(i));
+        }
         // covered distance of skeleton point j: R.col(j).dot(|q_e - q_temp|)
         auto covered = [&]() {
-            return eigen_dyn_sum([&](int i) { return s.acc(i) * fabsf(qe[i] - s.Q(i)); }, D);
+            return eigen_dyn_sum([&](int i) { return s.acc(i) * s.DL(i); }, D);
         };
         float step = INFINITY;
         for (int j = 1; j <= D; ++j) {
@@ -122,6 +123,7 @@ __device__ int32_t spine_run(const RobotDev& rb, const SpineLane& s, float dq, P
         FKStream fk;
         fk_init(fk);
         s.set_P(s.sk, 0, skel_point<float>(fk, rb, s.qt + s.t, 0, s.B));
+        skel = s.sk;
         float prev = 0.0f;
         for (int k = 1; k <= D; ++k) {
             const Vec3<float> v = skel_point<float>(fk, rb, s.qt + s.t, k, s.B);
@@ -146,6 +148,9 @@ __global__ __launch_bounds__(64) void k_spines(RobotDev rb, SpineArgs a, int64_t
     const float* pc = a.profile + c * a.profile_stride;
     // q_new may alias q (in-place layers): read the whole state first
     for (int k = 0; k < D; ++k) s.Q(k) = qc[k];
+    FKStream fk;
+    fk_init(fk);
+    for (int k = 0; k <= D; ++k) s.set_P(s.sk0, k, skel_point<float>(fk, rb, s.qt + s.t, k, s.B));
     const int32_t status =
         spine_run(rb, s, a.d[c * a.d_stride], [&](int i) { return pc[i]; }, a.q_e + c * D, a.num_iter, a.expanded);
     float* qn = a.q_new + c * D;
@@ -158,61 +163,87 @@ __global__ __launch_bounds__(64) void k_spines(RobotDev rb, SpineArgs a, int64_t
 // computeDistanceUnderestimation of its end state against the root's
 // nearest points, stop below D_CRIT or when the spine did not advance.  The
 // profile of the current layer's start state sits in the lane's slice after
-// the spine part.
-__global__ __launch_bounds__(64) void k_gen_spines_under(RobotDev rb, GenSpineArgs g, int64_t n) {
+// the spine part, the root's planes after the slices.
+//
+// Bound by the latency and issue of one wave per SIMD (65,536 spines are
+// 1,024 waves).  The planes are worked out once per workgroup (in every lane
+// at every layer they were three quarters of the instructions), as many links
+// at a time as fit; one tile holds all 102 of the xArm6 scene and is staged
+// once, more tiles are staged again in every layer.  The skeleton that the
+// underestimation computes is the next layer's start skeleton, so a layer
+// runs the kinematics once (65,536 xArm6 spines of 5 layers, the root's
+// distance included: 354 to 153 us a call).
+// A workgroup is one wave; its lanes go through the layers together, finished
+// ones masked off, so that all of them stage.
+__global__ __launch_bounds__(64) void k_gen_spines_under(RobotDev rb, GenSpineArgs g, int64_t n, int tile) {
     extern __shared__ __align__(16) unsigned char smem[];
-    const int D = rb.num_dofs, L = rb.num_links;
+    const int D = rb.num_dofs, L = rb.num_links, M = g.num_obj;
     const int B = blockDim.x, t = threadIdx.x;
-    float* base = reinterpret_cast<float*>(smem);
+    Plane* planes = reinterpret_cast<Plane*>(smem);   // [tile][M]
+    float* base = reinterpret_cast<float*>(smem + (size_t)tile * M * sizeof(Plane));
     const SpineLane s(base, D, B, t);
     float* pr = base + (size_t)spine_slice(D) * B;    // [L][B]
     auto PR = [&](int k) -> float& { return pr[k * B + t]; };
     const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= n) return;
-    const float* qe = g.q_e + c * D;
+    const bool live = c < n;
+    const float* qe = g.q_e + (live ? c : 0) * D;
     const float d0 = g.d_root[0];
     for (int k = 0; k < D; ++k) s.Q(k) = g.q_root[k];
     for (int k = 0; k < L; ++k) PR(k) = g.profile_root[k];
     int32_t status = kTrapped;
     float d_out = d0;
-    float dq = d0;
-    if (d0 > 0.0f) {
-        for (int layer = 0; layer < g.num_layers; ++layer) {
-            status = spine_run(rb, s, dq, [&](int i) { return PR(i); }, qe, g.num_iter, g.expanded);
-            // computeDistanceUnderestimation(q_new, root nearest points)
-            FKStream fk;
-            fk_init(fk);
-            Vec3<float> P0 = skel_point<float>(fk, rb, s.qt + t, 0, B);
-            float d = g.maxd;
-            bool neg = false;
-            for (int i = 0; i < L && !neg; ++i) {
+    bool on = live && d0 > 0.0f;   // still extending
+    if (on) {
+        FKStream fk;
+        fk_init(fk);
+        for (int k = 0; k <= D; ++k) s.set_P(s.sk0, k, skel_point<float>(fk, rb, s.qt + t, k, B));
+    }
+    const bool one_tile = tile >= L;
+    if (one_tile) {
+        stage_planes(planes, g.np_root, M, L, 0, L, g.maxd, nullptr, 0.0f);
+        __syncthreads();
+    }
+    for (int layer = 0; layer < g.num_layers; ++layer) {
+        if (!__any(on)) break;   // uniform: the workgroup is one wave
+        if (on) status = spine_run(rb, s, d_out, [&](int i) { return PR(i); }, qe, g.num_iter, g.expanded);
+        // computeDistanceUnderestimation(q_new, root nearest points)
+        FKStream fk;
+        fk_init(fk);
+        Vec3<float> P0{0.0f, 0.0f, 0.0f};
+        if (on) {
+            P0 = skel_point<float>(fk, rb, s.qt + t, 0, B);
+            s.set_P(s.sk0, 0, P0);
+        }
+        float d = g.maxd;
+        bool neg = false;
+        for (int i0 = 0; i0 < L; i0 += tile) {
+            const int i1 = min(L, i0 + tile);
+            if (!one_tile) {
+                __syncthreads();
+                stage_planes(planes, g.np_root, M, L, i0, i1, g.maxd, nullptr, 0.0f);
+                __syncthreads();
+            }
+            for (int i = i0; on && !neg && i < i1; ++i) {
                 const Vec3<float> P1 = skel_point<float>(fk, rb, s.qt + t, i + 1, B);
-                float prof = g.maxd;
-                for (int j = 0; j < g.num_obj; ++j) {
-                    const float* e = g.np_root + ((int64_t)j * L + i) * 6;
-                    const Vec3<float> O{e[3], e[4], e[5]};
-                    if (vnorm(O) == g.maxd) continue;
-                    const Vec3<float> R{e[0], e[1], e[2]};
-                    const float tm = plane_term(P0, P1, R, O, rb.radius[i]);
-                    if (tm < 0.0f) {
-                        neg = true;
-                        break;
-                    }
-                    prof = min_std(prof, tm);
-                }
+                s.set_P(s.sk0, i + 1, P1);
+                const float low = planes_min(planes + (i - i0) * M, M, P0, P1, rb.radius[i]);
+                neg = low < 0.0f;
+                const float prof = min_std(g.maxd, low);
                 PR(i) = prof;
                 d = min_std(d, prof);
                 P0 = P1;
             }
+        }
+        if (on) {
             if (neg) {   // returned early: no profile stored
                 d = 0.0f;
                 for (int k = 0; k < L; ++k) PR(k) = 0.0f;
             }
             d_out = d;
-            dq = d;
-            if (d < g.d_crit || status != kAdvanced) break;
+            on = !(d < g.d_crit || status != kAdvanced);
         }
     }
+    if (!live) return;
     float* qn = g.q_new + c * D;
     for (int k = 0; k < D; ++k) qn[k] = s.Q(k);
     g.status[c] = status;
@@ -372,10 +403,16 @@ hipError_t launch_spines(const RobotDev& rb, const SpineArgs& a, int64_t n, hipS
 
 hipError_t launch_gen_spines_under(const RobotDev& rb, const GenSpineArgs& g, int64_t n, hipStream_t st) {
     if (n <= 0) return hipSuccess;
+    // 64 KB of LDS: the lanes' slices (fewer lanes for long chains), beside
+    // at least one link's planes and as many links' as fit
     const size_t per = spine_lds_per_lane(rb) + (size_t)rb.num_links * sizeof(float);
+    const size_t link = (size_t)std::max(1, (int)g.num_obj) * sizeof(Plane);
+    const size_t room = 64 * 1024;
     int B = 64;
-    while (B > 16 && per * B > 64 * 1024) B /= 2;
-    hipLaunchKernelGGL(k_gen_spines_under, dim3((unsigned)((n + B - 1) / B)), dim3(B), per * B, st, rb, g, n);
+    while (B > 1 && per * B + link > room) B /= 2;
+    const int tile = (int)std::min<size_t>((size_t)rb.num_links, std::max<size_t>(1, (room - per * B) / link));
+    hipLaunchKernelGGL(k_gen_spines_under, dim3((unsigned)((n + B - 1) / B)), dim3(B),
+                       (size_t)tile * g.num_obj * sizeof(Plane) + per * B, st, rb, g, n, tile);
     return hipGetLastError();
 }
 

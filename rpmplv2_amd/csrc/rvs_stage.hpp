@@ -136,6 +136,47 @@ __device__ __attribute__((always_inline)) inline void seg_bounds(const Vec3<T>& 
     hi = Vec3<T>{A.x < B.x ? B.x : A.x, A.y < B.y ? B.y : A.y, A.z < B.z ? B.z : A.z};
 }
 
+// The planes of one nearest-point set ([M][L][6], RealVectorSpace.cpp:402-446)
+// in LDS, links i0 .. i1 - 1 as [i1 - i0][M]: O and the unit normal of each
+// (obstacle, link) pair, worked out by the threads of the workgroup (all of
+// them call; the caller synchronizes before the planes are read and before
+// they are staged again).  A pair the reference skips (|O| = maxd) gets a NaN
+// normal: its term is NaN and never enters a minimum.  With max_vel [M] the
+// planes first move towards the robot for delta_t.
+struct alignas(16) Plane {
+    Vec3<float> O;
+    float nx, ny, nz;
+    float pad[2];
+};
+static_assert(sizeof(Plane) == 32, "two 16-byte LDS reads per plane");
+
+__device__ inline void stage_planes(Plane* planes, const float* __restrict__ set, int M, int L, int i0, int i1,
+                                    float maxd, const float* __restrict__ max_vel, float delta_t) {
+    for (int k = threadIdx.x; k < (i1 - i0) * M; k += blockDim.x) {
+        const int i = i0 + k / M, j = k % M;
+        const float* e = set + ((int64_t)j * L + i) * 6;
+        Vec3<float> R{e[0], e[1], e[2]}, O{e[3], e[4], e[5]};
+        const bool skip = vnorm(O) == maxd;
+        if (max_vel) plane_move(R, O, max_vel[j], delta_t);
+        const Vec3<float> nv = plane_normal(R, O);
+        planes[k] = Plane{O, skip ? NAN : nv.x, skip ? NAN : nv.y, skip ? NAN : nv.z, {0.0f, 0.0f}};
+    }
+}
+
+// Smallest term of one link (P0, P1) over its row of M staged planes, from
+// infinity: its sign alone says whether any term was negative, and
+// MAX_DISTANCE, the start of the reference's minimum, enters afterwards.
+__device__ __attribute__((always_inline)) inline float planes_min(const Plane* row, int M, const Vec3<float>& P0,
+                                                                  const Vec3<float>& P1, float r) {
+    float low = INFINITY;
+#pragma unroll 2
+    for (int j = 0; j < M; ++j) {
+        const Plane pl = row[j];
+        low = smin(low, plane_value(P0, P1, pl.O, Vec3<float>{pl.nx, pl.ny, pl.nz}, r));
+    }
+    return low;
+}
+
 template <typename T> __device__ inline T rnew_of(const RobotDev& rb, int i);
 template <> __device__ inline float rnew_of<float>(const RobotDev& rb, int i) { return rb.rnew32[i]; }
 template <> __device__ inline double rnew_of<double>(const RobotDev& rb, int i) { return rb.rnew64[i]; }

@@ -798,6 +798,27 @@ def test_extend_gen_spines(oracle, engine, use_real_dist, num_iter):
     assert (st == 2).all() and (qn == root_bad[None]).all() and (dd == 0).all()
 
 
+@pytest.mark.parametrize("dofs,boxes,n,num_iter", [(6, 1, 1, 1), (10, 250, 65, 5), (22, 90, 70, 1), (22, 1000, 33, 2)])
+def test_extend_gen_spines_plane_tiles(oracle, engine, dofs, boxes, n, num_iter):
+    """Underestimation layers against plane sets of one tile and of several
+    (down to one link a tile and fewer lanes a workgroup), ragged batches:
+    identical to the oracle's composition."""
+    rng = np.random.default_rng(95 + boxes)
+    rb = R.xarm6() if dofs == 6 else R.chain(rng.uniform(0.05, 0.1, dofs), radius=0.02)
+    u = rng.normal(size=(boxes, 3))
+    sc = W._boxes(rng, boxes, 0.02, 0.1, 2.5)
+    sc = W.Scene(sc.dim, 2.6 * u / np.linalg.norm(u, axis=1, keepdims=True), sc.quat, sc.is_ground, sc.min_dist_tol)
+    root = np.zeros(dofs, np.float32)
+    v = rng.normal(size=(n, dofs))
+    q_e = (np.pi * v / np.linalg.norm(v, axis=1, keepdims=True)).astype(np.float32)
+    rid, eid = engine.load_robot(rb), engine.create_env(sc)
+    got = engine.extend_gen_spines(rid, eid, root, q_e, num_layers=4, num_iter=num_iter, d_crit=0.03)
+    want = oracle.extend_gen_spines(rb, oracle.scene_of(sc), root, q_e, num_layers=4, num_iter=num_iter, d_crit=0.03)
+    for g, o in zip(got, want):
+        assert (g == o).all()
+    assert (got[2] > 0).any()
+
+
 @pytest.mark.parametrize("eps_step", [0.1, 0.02])
 def test_edge_self_collision(oracle, engine, eps_step):
     """Capsule part of xArm6::checkSelfCollision(q1, q2) for 16384 edges
