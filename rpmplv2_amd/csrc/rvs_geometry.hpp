@@ -140,6 +140,7 @@ __host__ __device__ inline T seg_seg(const Vec3<T>& A, const Vec3<T>& B, const V
     const T opt2 = MP::div(dot(AC, DC), alpha3);
     const T opt3 = MP::div(dot(BC, DC), alpha3);
     if (WANT_NP) np->valid = false;
+    T sq = T(INFINITY);   // smallest squared candidate (a NaN one never enters)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const T o = (i == 0) ? opt0 : (i == 1) ? opt1 : (i == 2) ? opt2 : opt3;
@@ -158,13 +159,20 @@ __host__ __device__ inline T seg_seg(const Vec3<T>& A, const Vec3<T>& B, const V
             p0 = (i == 2) ? A : B;
             p1 = lerp(C, D, o);
         }
-        const T d_tmp = vnorm<T, MP>(p1 - p0);
-        if (d_tmp < d_c) {
-            d_c = d_tmp;
-            if (WANT_NP) { np->r = p0; np->o = p1; np->valid = true; }
+        if (WANT_NP) {
+            const T d_tmp = vnorm<T, MP>(p1 - p0);
+            if (d_tmp < d_c) {
+                d_c = d_tmp;
+                np->r = p0; np->o = p1; np->valid = true;
+            }
+        } else {
+            sq = smin(sq, sqnorm(p1 - p0));
         }
     }
-    return d_c;
+    // without the points one square root serves all four candidates: a
+    // correctly rounded square root is monotone, so the root of the smallest
+    // square is the smallest root
+    return WANT_NP ? d_c : smin(d_c, MP::root(sq));
 }
 
 // ---------------------------------------------------------------- seg-pt
@@ -291,10 +299,9 @@ __host__ __device__ inline T capsule_box(const Vec3<T>& A, const Vec3<T>& B, T r
             }
         }
     }
-    if (inside) {
-        if (WANT_NP) np->valid = false;
-        return T(0);
-    }
+    // no points until a case finds some (a NaN end point finds none)
+    if (WANT_NP) np->valid = false;
+    if (inside) return T(0);
 
     // --- work list
     T d_c = p.maxd;
@@ -367,6 +374,7 @@ __host__ __device__ inline T capsule_box(const Vec3<T>& A, const Vec3<T>& B, T r
     bool hit = false;
     if (nfaces == 1) hit = face_crossed<T, MP>(A, B, b, face1, p);
     else if (nfaces == 6)
+#pragma clang loop unroll(disable)
         for (int f = 0; f < 6; ++f) hit = hit || face_crossed<T, MP>(A, B, b, f, p);
 
     if (hit) {
@@ -379,6 +387,7 @@ __host__ __device__ inline T capsule_box(const Vec3<T>& A, const Vec3<T>& B, T r
         d_c = seg_pt<T, WANT_NP, MP>(A, B, b.corner(corner), p, &t);
         if (WANT_NP) *np = t;
     } else {
+#pragma clang loop unroll(disable)
         for (int e = 0; e < nedges; ++e) {
             const int ed = list_edge(kind, param, e);
             NP<T> t;
@@ -528,31 +537,49 @@ __host__ __device__ inline float flat_capsule_box(const Vec3<float>& A, const Ve
 }
 
 // ---------------------------------------------------------------- collision
-// checkCases, CollisionAndDistance.cpp:113-148: distance of AB to the one or
-// two rectangle edges on the side of point 'pt' (2-D coordinates u, v).
+// The collision tree's segment-segment tests all ask whether AB comes closer
+// than the radius to some edge of the box, and any one that does makes the
+// capsule collide (a minimum below the radius is a value below the radius; the
+// one early stop, at a distance of 0, already collides).  So the face tests
+// below only collect the edges they would measure, as a 12-bit mask, and
+// collision_box measures each edge once, through a single copy of seg_seg: the
+// tree with a copy per call site (24 of them) was 63 KB of kernel code, as
+// large as the instruction cache that two CUs share; now 21 KB (isValid of
+// 1,000,003 xArm6 configurations, 17 boxes: 304 to 234 us a call; 65,536 edges
+// of ten states: 237 to 200 us).
+// Edge (axis a, corner c with bit a clear) runs from corner c to c | 1 << a, as
+// every edge of checkCases does; its bit is 4 a + the corner's other two bits.
+__host__ __device__ inline int box_edge_bit(int axis, int corner) {
+    const int b1 = axis == 0 ? 1 : 0, b2 = axis == 2 ? 1 : 2;
+    return 1 << (4 * axis + ((corner >> b1) & 1) + 2 * ((corner >> b2) & 1));
+}
+__host__ __device__ inline int box_edge_corner(int bit) {
+    const int axis = bit >> 2, b1 = axis == 0 ? 1 : 0, b2 = axis == 2 ? 1 : 2;
+    return ((bit & 1) << b1) | (((bit >> 1) & 1) << b2);
+}
+
+// checkCases, CollisionAndDistance.cpp:113-148: the one or two edges of face
+// 'face' on the side of a point with in-face coordinates (u, v).
 template <typename T>
-__host__ __device__ inline T check_cases(const Vec3<T>& A, const Vec3<T>& B, const Box<T>& b, int face, T u, T v,
-                                         const Params<T>& p) {
+__host__ __device__ inline int check_cases_edges(const Box<T>& b, int face, T u, T v) {
     const int c = face % 3;
     const int fix = (face >= 3) ? (1 << c) : 0;
     const int a1 = (c == 0) ? 1 : 0, a2 = (c == 2) ? 1 : 2;
-    const int b1 = 1 << a1, b2 = 1 << a2;
-    T d1 = p.maxd, d2 = p.maxd;
-    int e = -1;
-    if (u < b.lo_at(a1)) e = edge_of(fix, fix | b2);
-    else if (u > b.hi_at(a1)) e = edge_of(fix | b1, fix | b1 | b2);
-    if (e >= 0) d1 = seg_seg<T, false>(A, B, b.corner(e & 7), b.corner(e >> 3), p, nullptr);
-    e = -1;
-    if (d1 > 0 && v < b.lo_at(a2)) e = edge_of(fix, fix | b1);
-    else if (d1 > 0 && v > b.hi_at(a2)) e = edge_of(fix | b2, fix | b1 | b2);
-    if (e >= 0) d2 = seg_seg<T, false>(A, B, b.corner(e & 7), b.corner(e >> 3), p, nullptr);
-    return smin(d1, d2);
+    int m = 0;
+    if (u < b.lo_at(a1)) m |= box_edge_bit(a2, fix);
+    else if (u > b.hi_at(a1)) m |= box_edge_bit(a2, fix | 1 << a1);
+    if (v < b.lo_at(a2)) m |= box_edge_bit(a1, fix);
+    else if (v > b.hi_at(a2)) m |= box_edge_bit(a1, fix | 1 << a2);
+    return m;
 }
 
-// collisionCapsuleToRectangle, CollisionAndDistance.cpp:46-111, general radius
+// collisionCapsuleToRectangle, CollisionAndDistance.cpp:46-111, general
+// radius: true when the face test itself collides; otherwise the edges whose
+// distance decides are added to 'edges' ('checked' is set when a checkCases
+// would run, whose minimum starts from MAX_DISTANCE).
 template <typename T>
 __host__ __device__ inline bool rect_collision(const Vec3<T>& A, const Vec3<T>& B, T radius, const Box<T>& b,
-                                               int face, const Params<T>& p) {
+                                               int face, const Params<T>& p, int& edges, bool& checked) {
     const int c = face % 3;
     const int o1 = (c == 0) ? 1 : 0, o2 = (c == 2) ? 1 : 2;
     const T v = b.f(face);
@@ -584,13 +611,11 @@ __host__ __device__ inline bool rect_collision(const Vec3<T>& A, const Vec3<T>& 
     if (radius > 0) {
         const bool a_in = Au > r0 && Au < r2 && Av > r1 && Av < r3;
         const bool b_in = Bu > r0 && Bu < r2 && Bv > r1 && Bv < r3;
-        if (a_in) {
-            if (b_in) return smin(nA, nB) < radius;
-            return smin(check_cases(A, B, b, face, Bu, Bv, p), nA) < radius;
-        }
-        if (b_in) return smin(check_cases(A, B, b, face, Au, Av, p), nB) < radius;
-        if (check_cases(A, B, b, face, Au, Av, p) < radius) return true;
-        return check_cases(A, B, b, face, Bu, Bv, p) < radius;
+        if (a_in && b_in) return smin(nA, nB) < radius;
+        if (!b_in) edges |= check_cases_edges(b, face, Bu, Bv);
+        if (!a_in) edges |= check_cases_edges(b, face, Au, Av);
+        checked = true;
+        return (a_in && nA < radius) || (b_in && nB < radius);
     }
     return false;
 }
@@ -617,13 +642,23 @@ __host__ __device__ inline bool collision_box(const Vec3<T>& A, const Vec3<T>& B
         (B.x > b.lo[0] - r_new && B.y > b.lo[1] - r_new && B.z > b.lo[2] - r_new &&
          B.x < b.hi[0] + r_new && B.y < b.hi[1] + r_new && B.z < b.hi[2] + r_new))
         return true;
-    // one face per axis, chosen by A's position, tested in x, y, z order
+    // one face per axis, chosen by A's position; then the edges they ask for
+    int edges = 0;
+    bool checked = false;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         int face = -1;
         if (A[k] < b.lo[k]) face = k;
         else if (A[k] > b.hi[k]) face = k + 3;
-        if (face >= 0 && rect_collision(A, B, radius, b, face, p)) return true;
+        if (face >= 0 && rect_collision(A, B, radius, b, face, p, edges, checked)) return true;
+    }
+    if (checked && p.maxd < radius) return true;
+#pragma clang loop unroll(disable)
+    while (edges) {
+        const int e = __builtin_ctz(edges);
+        const int c0 = box_edge_corner(e);
+        if (seg_seg<T, false>(A, B, b.corner(c0), b.corner(c0 | 1 << (e >> 2)), p, nullptr) < radius) return true;
+        edges &= edges - 1;
     }
     return false;
 }

@@ -96,6 +96,12 @@ int run(long n, uint64_t seed, const char* tag) {
             for (int k = 0; k < 6 && ok; ++k) ok = same(g6[k], onp[k]);
             if (!ok) { if (bad_np < 5) printf("[%s] nearest-point mismatch it=%ld path=%d\n", tag, it, opath); bad_np++; }
         }
+        // without nearest points (one square root for the segment candidates)
+        const T gd0 = capsule_box<T, false>(a, bb, r, b, p, nullptr, nullptr);
+        if (!same(gd0, od)) {
+            if (bad_cb < 5) printf("[%s] capsule_box (no points) mismatch it=%ld path=%d gpu=%.9g oracle=%.9g\n", tag, it, opath, (double)gd0, (double)od);
+            bad_cb++;
+        }
         if constexpr (sizeof(T) == 4) {
             // the flat evaluation of the per-lane walk: where it does not flag
             // the pair, the contact outputs (0 inside, -r crossing) are the
@@ -137,6 +143,8 @@ int run(long n, uint64_t seed, const char* tag) {
         NP<T> t{};
         T gs = seg_seg<T, true>(a, bb, c, dd, p, &t);
         if (!same(gs, os)) { if (bad_ss < 5) printf("[%s] seg_seg mismatch it=%ld %.9g %.9g\n", tag, it, (double)gs, (double)os); bad_ss++; }
+        const T gs0 = seg_seg<T, false>(a, bb, c, dd, p, nullptr);
+        if (!same(gs0, os)) { if (bad_ss < 5) printf("[%s] seg_seg (no points) mismatch it=%ld %.9g %.9g\n", tag, it, (double)gs0, (double)os); bad_ss++; }
         T opnt;
         if constexpr (sizeof(T) == 4) opnt = orc_seg_pt32(A, B, C, &op, snp, &sv);
         else opnt = orc_seg_pt64(A, B, C, &op, snp, &sv);
