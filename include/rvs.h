@@ -417,13 +417,14 @@ rvs_status rvs_get_tuning(rvs_context* ctx, int32_t robot, int32_t env, rvs_tuni
 
 /* Batches of reference-arithmetic distances (RVS_PREC_REF32 calls, calls
  * with nearest points, the distances inside generalized-spine and served
- * underestimation calls) up to max_configs configurations run one wave per
- * configuration, lanes over the obstacles: lower latency for small batches,
+ * underestimation calls) up to max_configs configurations spread each
+ * configuration's pairs over 16 to 64 lanes: lower latency for small batches,
  * the same results bit for bit.
  * Larger batches run one lane per configuration.  0 disables; default
- * 16384 (measured crossover on MI355X: 1 configuration 37 us vs 42 us per
- * call, 2048: 58 us vs 267 us, 32768: 429 us vs 218 us).  No counterpart in
- * the reference (a launch-shape choice). */
+ * 16384 (MI355X, xArm6 and 17 boxes, spread against one lane: 1 configuration
+ * 24 us vs 78 us per call, 4096: 46 us vs 294 us, 16384: 67 us vs 255 us,
+ * 65536: 149 us vs 203 us, 131072: 257 us vs 202 us).  No counterpart in the
+ * reference (a launch-shape choice). */
 rvs_status rvs_set_small_batch(rvs_context* ctx, int64_t max_configs);
 
 /* Launch shape of the persistent first-collision kernel: resident waves per

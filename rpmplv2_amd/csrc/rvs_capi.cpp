@@ -346,6 +346,7 @@ rvs_status rvs_robot_load(rvs_context* c, const rvs_robot_desc* d, int32_t* robo
         rpy_to_matrix(j.rpy, s.R);
         for (int i = 0; i < 3; ++i) s.o[i] = j.xyz[i];
         s.rev = (j.type == RVS_JOINT_REVOLUTE) ? 1 : 0;
+        s.joint = ndof;
         ndof += s.rev;
         double a[3];
         for (int i = 0; i < 3; ++i) a[i] = s.R[3 * i] * j.axis[0] + s.R[3 * i + 1] * j.axis[1] + s.R[3 * i + 2] * j.axis[2];

@@ -38,7 +38,7 @@ struct SegDev {
     double axis[3];   // rotation axis in the parent frame, unit length
     double o[3];      // joint origin translation
     int32_t rev;      // 1 revolute, 0 fixed
-    int32_t pad;
+    int32_t joint;    // revolute: its joint coordinate, the number of revolute segments before it
 };
 
 // The FP32 bulk pass's copy of a segment, in float: the origin rotation R

@@ -265,6 +265,14 @@ hipError_t launch_distance_refine(const RobotDev& rb, const EnvDev& env, const Q
                                   int64_t n, const DistOut& out, const int32_t* idx, const uint32_t* count,
                                   hipStream_t st, uint32_t* count_out = nullptr);
 hipError_t launch_zero_u32(uint32_t* p, int n, hipStream_t st);
+// Exact distances with a few lanes per configuration, the pairs of a
+// configuration spread over them: the n configurations of a direct call (idx
+// null), or the *count entries of a refinement list.  Whether the robot's
+// links x the scene's obstacles fit its rows:
+bool pairs_fit(const RobotDev& rb, const EnvDev& env);
+hipError_t launch_distance_pairs(const RobotDev& rb, const EnvDev& env, const QueryParams& qp, const float* q,
+                                 const DistOut& out, const int32_t* idx, const uint32_t* count, int64_t n,
+                                 int64_t max_waves, hipStream_t st, uint32_t* count_out = nullptr);
 
 
 // One lane per configuration; with perm, lane g takes configuration perm[g]

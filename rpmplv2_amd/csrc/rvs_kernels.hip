@@ -159,26 +159,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // ends after the first round with a hit.
 constexpr int kRefineWaves = 4;   // waves per workgroup of the refinement kernel (they share the staged obstacles)
 
-// Entry k of the refinement's work: configuration c and the first link to
-// recompute, k0 (entry k itself and k0 = 0 for a direct call, idx null; k0
-// = 0 too without a profile, which holds the values of the links before it).
-__device__ __attribute__((always_inline)) inline void flag_decode(const int32_t* idx, int64_t k, const QueryParams& qp,
-                                                                  const DistOut& out, int64_t& c, int& k0) {
-    if (!idx) {
-        c = k;
-        k0 = 0;
-        return;
-    }
-    const int64_t e = (int64_t)idx[k];
-    if (qp.flag_link) {
-        c = e & (((int64_t)1 << kFlagLinkShift) - 1);
-        k0 = out.profile ? (int)(e >> kFlagLinkShift) : 0;
-    } else {
-        c = e;
-        k0 = 0;
-    }
-}
-
 // With idx null the kernel serves a direct call: wave k takes configuration
 // k < n (latency-bound small batches: one wave per configuration instead of
 // one lane).  With nearest points every pair is evaluated (no broad phase)
@@ -330,124 +310,6 @@ __global__ __launch_bounds__(64 * kRefineWaves) void k_distance_refine(RobotDev 
             if (out.d) out.d[c] = hit ? 0.0f : d;
             if (out.verdict) out.verdict[c] = hit ? 0 : 1;
         }
-    }
-}
-
-// Exact recomputation for small obstacle sets (links x obstacles <=
-// kPairsMax, fewer than 64 links): one wave per configuration evaluates all
-// of its (link, obstacle) pairs at once, lane t taking pairs t, t + 64, ...
-// of pair = link * M + obstacle, instead of one link per round.  Lane m
-// computes joint m's sine and cosine, every lane runs the same forward
-// kinematics on them and lane k keeps skeleton point k; a pair fetches its
-// end points by lane shuffles.  The filtered pair distances go to
-// the wave's LDS row, lane i then walks link i's obstacles in order as the
-// reference's loop does (running std::min from MAX_DISTANCE, stop at the
-// first value <= 0), and the links combine in order: the first link with a
-// hit ends the configuration (later links 0, distance 0), otherwise the
-// distance is the smallest link value (a minimum of non-NaN floats, exact in
-// any order).  Every pair is evaluated (no broad phase, no early exit), which
-// changes no result: the per-link walk over the stored values is the
-// reference's loop.  The workgroup's waves step through the configurations
-// together so that the LDS row can be handed over with a workgroup barrier.
-constexpr int kPairsMax = 256;
-
-__host__ __device__ inline size_t pairs_row_off(const EnvDev& env) {
-    return (staged_bytes<float>(env) + 15) & ~size_t(15);
-}
-
-inline bool refine_pairs_fit(const RobotDev& rb, const EnvDev& env) {
-    return rb.num_links < 64 && rb.num_dofs <= 64 && (int64_t)rb.num_links * env.num_obj <= kPairsMax;
-}
-
-template <bool OBB>
-__global__ __launch_bounds__(64 * kRefineWaves) void k_distance_refine_pairs(RobotDev rb, EnvDev env,
-                                                                             QueryParams qp,
-                                                                             const float* __restrict__ q, DistOut out,
-                                                                             const int32_t* __restrict__ idx,
-                                                                             const uint32_t* __restrict__ count,
-                                                                             int64_t n_direct, uint32_t* count_out) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    const Staged<float> s = stage_env<float, OBB>(env, smem);
-    const int M = env.num_obj, L = rb.num_links;
-    const int npairs = L * M;
-    const int t = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    float* row = reinterpret_cast<float*>(smem + pairs_row_off(env)) + wave * kPairsMax;
-    const Params<float> p{qp.eq, qp.maxd};
-    const int64_t total = idx ? (int64_t)*count : n_direct;
-    if (count_out && blockIdx.x == 0 && threadIdx.x == 0) *count_out = (uint32_t)total;
-    for (int64_t kb = (int64_t)blockIdx.x * kRefineWaves; kb < total; kb += (int64_t)gridDim.x * kRefineWaves) {
-        const int64_t k = kb + wave;
-        const bool live = k < total;   // uniform over the wave
-        int64_t c = 0;
-        int k0 = 0;   // the first link to recompute; the pairs of the links before it are not evaluated
-        if (live) {
-            flag_decode(idx, k, qp, out, c, k0);
-            const float* qc = q + c * rb.num_dofs;
-            // lane m computes the sine and cosine of joint m (the same
-            // function of the same value as a serial stream); the FK stream
-            // then takes them by shuffles
-            double my_s = 0.0, my_c = 1.0;
-            if (t < rb.num_dofs) sincos((double)qc[t], &my_s, &my_c);
-            const auto sc = [&](int m, double* st, double* ct) {
-                *st = __shfl(my_s, m, 64);
-                *ct = __shfl(my_c, m, 64);
-            };
-            FKStream fk;
-            fk_init(fk);
-            Vec3<float> mine{0.0f, 0.0f, 0.0f};
-            for (int pt = 0; pt <= L; ++pt) {
-                const Vec3<float> P = skel_point_sc<float>(fk, rb, pt, sc);
-                if (t == pt) mine = P;
-            }
-            for (int base = k0 * M; base < npairs; base += 64) {   // uniform rounds: the shuffles see every lane
-                const int pp = base + t;
-                const int i = pp < npairs ? pp / M : 0;
-                const int j = pp - i * M;
-                const Vec3<float> A{__shfl(mine.x, i, 64), __shfl(mine.y, i, 64), __shfl(mine.z, i, 64)};
-                const Vec3<float> B{__shfl(mine.x, i + 1, 64), __shfl(mine.y, i + 1, 64), __shfl(mine.z, i + 1, 64)};
-                if (pp < npairs) {
-                    float dt;
-                    if (s.gnd[j] && i < rb.ground_included) {
-                        dt = p.maxd;
-                    } else if (OBB) {
-                        const float* x = s.xf + 12 * j;
-                        dt = capsule_box<float, false>(to_box(x, A), to_box(x, B), rb.radius[i], s.box[j], p, nullptr,
-                                                       nullptr);
-                    } else {
-                        dt = capsule_box<float, false>(A, B, rb.radius[i], s.box[j], p, nullptr, nullptr);
-                    }
-                    if (dt > s.tol[j]) dt = p.maxd;
-                    row[pp] = dt;
-                }
-            }
-        }
-        __syncthreads();
-        if (live) {
-            float prof = p.maxd;
-            bool hit = false;
-            if (t < k0) {
-                prof = out.profile[c * L + t];   // a link before k0: the bulk pass's value, no hit
-            } else if (t < L) {
-                for (int j = 0; j < M; ++j) {
-                    prof = smin(prof, row[t * M + j]);
-                    if (prof <= 0) {
-                        hit = true;
-                        break;
-                    }
-                }
-            }
-            const uint64_t hm = __ballot(hit);
-            const int first_hit = hm ? __ffsll((unsigned long long)hm) - 1 : L;
-            float d = (t < first_hit && t < L) ? prof : p.maxd;
-            for (int o = 32; o > 0; o >>= 1) d = smin(d, __shfl_xor(d, o, 64));
-            if (t >= k0 && t < L && out.profile) out.profile[c * L + t] = t <= first_hit ? prof : 0.0f;
-            if (t == 0) {
-                if (out.d) out.d[c] = hm ? 0.0f : d;
-                if (out.verdict) out.verdict[c] = hm ? 0 : 1;
-            }
-        }
-        __syncthreads();   // the row is rewritten by the next round
     }
 }
 
@@ -871,22 +733,13 @@ hipError_t launch_distance_fp64(const RobotDev& rb, const EnvDev& env, const Que
 hipError_t launch_distance_ref32_waves(const RobotDev& rb, const EnvDev& env, const QueryParams& qp, const float* q,
                                        int64_t n, const DistOut& out, hipStream_t st) {
     if (n <= 0) return hipSuccess;
+    if (pairs_fit(rb, env)) return launch_distance_pairs(rb, env, qp, q, out, nullptr, nullptr, n, 65536, st);
     const unsigned grid = (unsigned)std::min<int64_t>((n + kRefineWaves - 1) / kRefineWaves, 65536);
     const size_t sm = staged_bytes<float>(env);
     const dim3 b(64 * kRefineWaves);
     const int32_t* no_idx = nullptr;
     const uint32_t* no_count = nullptr;
     uint32_t* no_out = nullptr;
-    if (!out.nearest && refine_pairs_fit(rb, env)) {
-        const size_t smp = pairs_row_off(env) + (size_t)kRefineWaves * kPairsMax * sizeof(float);
-        if (env.use_obb)
-            hipLaunchKernelGGL((k_distance_refine_pairs<true>), dim3(grid), b, smp, st, rb, env, qp, q, out, no_idx,
-                               no_count, n, no_out);
-        else
-            hipLaunchKernelGGL((k_distance_refine_pairs<false>), dim3(grid), b, smp, st, rb, env, qp, q, out, no_idx,
-                               no_count, n, no_out);
-        return hipGetLastError();
-    }
     if (env.use_obb) {
         if (out.nearest)
             hipLaunchKernelGGL((k_distance_refine<true, true>), dim3(grid), b, sm, st, rb, env, qp, q, out, no_idx,
@@ -911,21 +764,12 @@ hipError_t launch_distance_refine(const RobotDev& rb, const EnvDev& env, const Q
     if (n <= 0) return hipSuccess;
     QueryParams rq = qp;   // the entries' form, as the bulk pass's launch chose it
     rq.flag_link = flags_carry_link(n) ? 1 : 0;
-    // enough waves to cover a typical flagged set in one round; the kernel
-    // loops when more configurations are flagged
+    // enough waves to cover a typical flagged set in one round; the kernels
+    // loop when more configurations are flagged
+    if (pairs_fit(rb, env)) return launch_distance_pairs(rb, env, rq, q, out, idx, count, n, 2048, st, count_out);
     const unsigned grid = (unsigned)std::min<int64_t>((n + kRefineWaves - 1) / kRefineWaves, 2048);
     const size_t sm = staged_bytes<float>(env);
     const dim3 b(64 * kRefineWaves);
-    if (refine_pairs_fit(rb, env)) {
-        const size_t smp = pairs_row_off(env) + (size_t)kRefineWaves * kPairsMax * sizeof(float);
-        if (env.use_obb)
-            hipLaunchKernelGGL((k_distance_refine_pairs<true>), dim3(grid), b, smp, st, rb, env, rq, q, out, idx, count,
-                               (int64_t)0, count_out);
-        else
-            hipLaunchKernelGGL((k_distance_refine_pairs<false>), dim3(grid), b, smp, st, rb, env, rq, q, out, idx,
-                               count, (int64_t)0, count_out);
-        return hipGetLastError();
-    }
     if (env.use_obb)
         hipLaunchKernelGGL((k_distance_refine<true, false>), dim3(grid), b, sm, st, rb, env, rq, q, out, idx, count,
                            (int64_t)0, count_out);

@@ -98,9 +98,11 @@ __device__ __attribute__((always_inline)) inline Vec3<T> from_box(const float* x
 // Compares squared values (no square root); a NaN end point never culls.
 constexpr float kCullMargin = 1e-5f;
 
+// Squared gap between the segment's bounding box and the box cb (0 on an
+// axis where they overlap or a coordinate is NaN).
 template <typename T>
-__device__ __attribute__((always_inline)) inline bool cull_pair(const float* __restrict__ cb, const Vec3<T>& slo,
-                                                                 const Vec3<T>& shi, T bound) {
+__device__ __attribute__((always_inline)) inline T gap_squared(const float* __restrict__ cb, const Vec3<T>& slo,
+                                                               const Vec3<T>& shi) {
     T g2 = T(0);
     {
         T g = (T)cb[0] - shi.x;
@@ -120,7 +122,13 @@ __device__ __attribute__((always_inline)) inline bool cull_pair(const float* __r
         g = g1 > g ? g1 : g;
         g2 = g > T(0) ? g2 + g * g : g2;
     }
-    return g2 > bound * bound;
+    return g2;
+}
+
+template <typename T>
+__device__ __attribute__((always_inline)) inline bool cull_pair(const float* __restrict__ cb, const Vec3<T>& slo,
+                                                                 const Vec3<T>& shi, T bound) {
+    return gap_squared(cb, slo, shi) > bound * bound;
 }
 
 template <typename T>
@@ -175,6 +183,26 @@ __device__ __attribute__((always_inline)) inline float planes_min(const Plane* r
         low = smin(low, plane_value(P0, P1, pl.O, Vec3<float>{pl.nx, pl.ny, pl.nz}, r));
     }
     return low;
+}
+
+// Entry k of the refinement's work: configuration c and the first link to
+// recompute, k0 (entry k itself and k0 = 0 for a direct call, idx null; k0
+// = 0 too without a profile, which holds the values of the links before it).
+__device__ __attribute__((always_inline)) inline void flag_decode(const int32_t* idx, int64_t k, const QueryParams& qp,
+                                                                  const DistOut& out, int64_t& c, int& k0) {
+    if (!idx) {
+        c = k;
+        k0 = 0;
+        return;
+    }
+    const int64_t e = (int64_t)idx[k];
+    if (qp.flag_link) {
+        c = e & (((int64_t)1 << kFlagLinkShift) - 1);
+        k0 = out.profile ? (int)(e >> kFlagLinkShift) : 0;
+    } else {
+        c = e;
+        k0 = 0;
+    }
 }
 
 template <typename T> __device__ inline T rnew_of(const RobotDev& rb, int i);

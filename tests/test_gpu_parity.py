@@ -1011,3 +1011,38 @@ def test_small_batches_many_obstacles(oracle, engine, oriented):
     od, oprof, over, _ = oracle.distance(w.robot, oracle.scene_of(w.scene, oriented=oriented), w.q, 32)
     print(f"oriented={oriented}: collision-free {a[2].mean():.3f}")
     assert (a[2] == over).all() and ulps(a[0], od).max() <= 2 and ulps(a[1], oprof).max() <= 2
+
+
+@pytest.mark.parametrize("oriented", [False, True])
+@pytest.mark.parametrize("dofs,boxes,n", [(2, 0, 5), (6, 1, 1), (6, 16, 3), (6, 170, 67), (10, 102, 18), (10, 103, 18),
+                                          (22, 46, 33), (40, 7, 9)])
+def test_distances_by_pairs_sizes(engine, dofs, boxes, n, oriented):
+    """A few lanes per configuration against one lane, bit for bit, with and
+    without nearest points: from no obstacle to the row's 1,024 pairs and past
+    them (103 boxes of ten links: link by link), more segments than lanes,
+    ragged waves, contacts with several boxes, links that skip ground boxes,
+    finite tolerances, NaN and infinite joints."""
+    rng = np.random.default_rng(100 * dofs + boxes)
+    rb = {2: R.planar_2dof, 6: R.xarm6}.get(dofs, lambda: R.chain(rng.uniform(0.05, 0.2, dofs), radius=0.03,
+                                                                   ground_included=2))()
+    sc = W._boxes(rng, boxes, 0.02, 0.3, 1.5, rotated=oriented)
+    if boxes > 2:
+        gnd, tol = sc.is_ground.copy(), sc.min_dist_tol.copy()
+        gnd[::7] = 1
+        tol[1::5] = 0.1
+        sc = W.Scene(sc.dim, sc.pos, sc.quat, gnd, tol)
+    q = rng.uniform(-np.pi, np.pi, (n, rb.num_dofs)).astype(np.float32)
+    q[n // 2, 0] = np.nan
+    q[n - 1, 1] = np.inf
+    rid = engine.load_robot(rb)
+    eid = engine.create_env(sc, rvs.ENV_OBB if oriented else rvs.ENV_AABB)
+    try:
+        for near in ((False, True) if boxes else (False,)):
+            engine.set_small_batch(1 << 20)
+            a = engine.distance(rid, eid, q, want_nearest=near)
+            engine.set_small_batch(0)
+            b = engine.distance(rid, eid, q, want_nearest=near)
+            for x, y in zip(a, b):
+                assert (x is None and y is None) or np.array_equal(x, y, equal_nan=True)
+    finally:
+        engine.set_small_batch(16384)
