@@ -420,6 +420,21 @@ rvs_status rvs_robot_load(rvs_context* c, const rvs_robot_desc* d, int32_t* robo
         pairs.push_back(a);
         pairs.push_back(b);
     }
+    // the pairs as runs, for the queries whose answer is a minimum over them
+    std::vector<std::pair<int32_t, int32_t>> sorted;
+    for (size_t m = 0; m + 1 < pairs.size(); m += 2) sorted.emplace_back(pairs[m], pairs[m + 1]);
+    std::sort(sorted.begin(), sorted.end());
+    sorted.erase(std::unique(sorted.begin(), sorted.end()), sorted.end());
+    std::vector<PairRun> runs;
+    for (const auto& [a, b] : sorted) {
+        const float rs = rad[a] + rad[b];
+        if (!runs.empty() && runs.back().a == a && runs.back().b + runs.back().count == b) {
+            ++runs.back().count;
+            runs.back().rsum = std::max(runs.back().rsum, rs);
+        } else {
+            runs.push_back(PairRun{a, b, 1, rs});
+        }
+    }
     (void)hipSetDevice(c->opt.device);
     RobotRec r;
     hipError_t e = upload(r.allocs, seg.data(), seg.size(), &r.dev.seg);
@@ -429,6 +444,7 @@ rvs_status rvs_robot_load(rvs_context* c, const rvs_robot_desc* d, int32_t* robo
     if (e == hipSuccess) e = upload(r.allocs, rn32.data(), rn32.size(), &r.dev.rnew32);
     if (e == hipSuccess) e = upload(r.allocs, rn64.data(), rn64.size(), &r.dev.rnew64);
     if (e == hipSuccess) e = upload(r.allocs, pairs.data(), pairs.size(), &r.dev.pairs);
+    if (e == hipSuccess) e = upload(r.allocs, runs.data(), runs.size(), &r.dev.runs);
     if (e == hipSuccess) e = upload(r.allocs, renc.data(), renc.size(), &r.dev.rad_enc);
     if (e != hipSuccess) {
         for (void* p : r.allocs) (void)hipFree(p);
@@ -440,6 +456,7 @@ rvs_status rvs_robot_load(rvs_context* c, const rvs_robot_desc* d, int32_t* robo
     r.dev.num_links = L;
     r.dev.ground_included = d->ground_included;
     r.dev.num_pairs = (int32_t)pairs.size() / 2;
+    r.dev.num_runs = (int32_t)runs.size();
     r.num_dofs = ndof;
     r.num_links = L;
     r.num_pairs = r.dev.num_pairs;

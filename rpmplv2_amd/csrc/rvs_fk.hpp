@@ -65,6 +65,13 @@ struct PointDev {
     int32_t pad;
 };
 
+// Self pairs (a, b), (a, b + 1), ... (a, b + count - 1) of the sorted pair
+// list, and the largest radius sum among them (in float, as the pairs add it).
+struct alignas(16) PairRun {
+    int32_t a, b, count;
+    float rsum;
+};
+
 struct RobotDev {
     int32_t num_segments;
     int32_t num_dofs;
@@ -79,6 +86,8 @@ struct RobotDev {
     const float* rnew32;     // collision-tree inflated radius, float
     const double* rnew64;    // same in double
     const int32_t* pairs;    // self-collision pairs (a, b)
+    const PairRun* runs;     // the same pairs, each once, sorted, as runs of consecutive second links
+    int32_t num_runs;
     const float* rad_enc;    // radii added by computeEnclosingRadii (capsules_radius, or xArm6's capsules_radius_new)
 };
 

@@ -205,6 +205,39 @@ __device__ __attribute__((always_inline)) inline void flag_decode(const int32_t*
     }
 }
 
+// Bound of a self pair's computed distance by the bounding boxes of its
+// segments.  distanceLineSegToLineSeg (CollisionAndDistance.cpp:217-320)
+// returns 0 (below the equality threshold eq), max_distance (degenerate
+// input), or the float norm of p1 - p0 for points that are end points or
+// a + o (b - a) with o in [0, 1], each within 5 eps C of its segment
+// (eps = 2^-24, C the largest coordinate magnitude), so the returned distance
+// is at least (D - 21 eps C)(1 - 2 eps) with D the distance of the two
+// segments' bounding boxes.  A D, computed in float, above
+// R = max(lo + r_a + r_b, eq) by 4e-6 (C + R) (about 67 eps (C + R), which also
+// covers the rounding of D and of the radii's subtraction) therefore leaves
+// it at lo + r_a + r_b or more, provided max_distance is at least that bound.
+// apart_bound2 is the square of that bound (infinite when max_distance is
+// smaller, NaN when cmax is: nothing is ruled out then); a pair whose
+// boxes_gap2 exceeds it has a capsule distance of at least lo.
+__device__ __attribute__((always_inline)) inline float apart_bound2(float rsum, float lo, float cmax,
+                                                                    const Params<float>& p) {
+    const float R = fmaxf(lo + rsum, p.eq);
+    const float thr = R + 4e-6f * (cmax + R);
+    return thr <= p.maxd ? thr * thr : (thr == thr ? INFINITY : NAN);
+}
+struct SegBox {
+    float lx, ly, lz, hx, hy, hz;
+    __device__ SegBox(const Vec3<float>& A, const Vec3<float>& B)
+        : lx(fminf(A.x, B.x)), ly(fminf(A.y, B.y)), lz(fminf(A.z, B.z)),
+          hx(fmaxf(A.x, B.x)), hy(fmaxf(A.y, B.y)), hz(fmaxf(A.z, B.z)) {}
+};
+__device__ __attribute__((always_inline)) inline float boxes_gap2(const SegBox& a, const SegBox& c) {
+    const float gx = fmaxf(fmaxf(c.lx - a.hx, a.lx - c.hx), 0.0f);
+    const float gy = fmaxf(fmaxf(c.ly - a.hy, a.ly - c.hy), 0.0f);
+    const float gz = fmaxf(fmaxf(c.lz - a.hz, a.lz - c.hz), 0.0f);
+    return __builtin_fmaf(gz, gz, __builtin_fmaf(gy, gy, gx * gx));
+}
+
 template <typename T> __device__ inline T rnew_of(const RobotDev& rb, int i);
 template <> __device__ inline float rnew_of<float>(const RobotDev& rb, int i) { return rb.rnew32[i]; }
 template <> __device__ inline double rnew_of<double>(const RobotDev& rb, int i) { return rb.rnew64[i]; }

@@ -1046,3 +1046,31 @@ def test_distances_by_pairs_sizes(engine, dofs, boxes, n, oriented):
                 assert (x is None and y is None) or np.array_equal(x, y, equal_nan=True)
     finally:
         engine.set_small_batch(16384)
+
+
+@pytest.mark.parametrize("dofs,n,scale", [(6, 1, 1.0), (6, 63, 1.0), (3, 65, 1.0), (22, 200, 1.0), (40, 130, 1.0),
+                                          (14, 70, 300.0), (14, 70, 1e-3)])
+def test_self_collision_minimum_of_pairs(engine, dofs, n, scale):
+    """The smallest pair distance, found without most of the pairs, against
+    the smallest of all of them, bit for bit: one pair to 741, radii that
+    differ, pairs in no order and twice, long and tiny links (coordinates of a
+    kilometre, links below the equality threshold), NaN and infinite joints,
+    ragged waves."""
+    rng = np.random.default_rng(7 * dofs + n)
+    if dofs == 6:
+        rb = R.xarm6(radius=[0.08, 0.02, 0.05, 0.03, 0.06, 0.01])
+    else:
+        rb = R.chain(scale * rng.uniform(0.05, 0.3, dofs), radius=scale * rng.uniform(0.01, 0.06, dofs),
+                     self_collision=True)
+        pairs = [rb.self_pairs[k] for k in rng.permutation(len(rb.self_pairs))]
+        rb.self_pairs = pairs + pairs[: len(pairs) // 3]
+    q = rng.uniform(-np.pi, np.pi, (n, rb.num_dofs)).astype(np.float32)
+    if n > 60:
+        q[:20] *= 0.1
+        q[n // 2, 0] = np.nan
+        q[n - 1, 1] = np.inf
+    rid = engine.load_robot(rb)
+    lo, free = engine.self_collision(rid, q)
+    all_pairs = engine.self_distance(rid, q)
+    want = np.fmin.reduce(np.concatenate([np.full((n, 1), 1000.0, np.float32), all_pairs], 1), axis=1)
+    assert np.array_equal(lo, want) and np.array_equal(free, (want >= 0).astype(np.uint8))
