@@ -379,16 +379,13 @@ rvs_status rvs_edge_first_collision(rvs_context* ctx, int32_t env, const int32_t
  * broad phase together and every lane queueing its own (link, obstacle)
  * pairs, so that a wave evaluates one pair per lane per step, or one launch
  * per link over the configurations still alive at it, in the walk order,
- * with the same queues) and workgroup size.  The obstacle set is always staged whole in LDS (every lane walks
- * every obstacle of its current link, so a smaller obstacle tile would only
- * add reloads); it must fit the device's workgroup LDS.  Variants 0, 1 and 2
- * evaluate the same pairs and give the same results bit for bit.  Variants 3
- * and 4 search for the first hit in obstacle order among other candidates
- * (more of them, or the walk positions after the hit), so that their
- * screening flags, and with them the refined set, can differ: the same
- * verdicts, and distances within FP32 rounding (a few 1e-7 m) of the other
- * variants'.  Each variant's results do not depend on its block size,
- * workgroups per CU or walk order. */
+ * with the same queues) and workgroup size.  The obstacle set is always
+ * staged whole in LDS (every lane walks every obstacle of its current link, so
+ * a smaller obstacle tile would only add reloads); it must fit the device's
+ * workgroup LDS.  Every variant screens the same pairs and gives the same
+ * results bit for bit, whatever its block size, workgroups per CU or walk
+ * order.  Without a recorded shape a call chooses by links x obstacles, the
+ * obstacles and its batch: 0 for short walks, otherwise 1, 3 or 4. */
 typedef struct rvs_tuning {
     int32_t variant;        /* 0: one lane per configuration; 1: persistent lane refill; 2: one lane per
                                configuration in persistent waves over 64-configuration chunks;
@@ -396,7 +393,7 @@ typedef struct rvs_tuning {
                                broad-phase group tables, and the cull boxes and pair queues in LDS
                                beside the obstacles; runs as 1 otherwise); 4: one launch per link
                                over the configurations alive at it, each lane queueing its own pairs
-                               (the needs of 3 and 16 bytes of scratch per configuration; runs as 3
+                               (the needs of 3 and 128 bytes of scratch per configuration; runs as 3
                                in rvs_distance_async_static and served requests) */
     int32_t block;          /* threads per workgroup: 64, 128 or 256; variants 3 and 4: 256, 512 or 1024 */
     int32_t blocks_per_cu;  /* variants 1 to 4: resident workgroups per CU (0 = as many as fit) */

@@ -788,14 +788,24 @@ rvs_status rvs_distance(rvs_context* c, int32_t robot, int32_t env, const float*
     const bool sort_exact = prec != RVS_PREC_FP32_REFINE && n >= kExactSortMin && n <= INT32_MAX &&
                             (prec == RVS_PREC_FP64 || n > c->wave_max);
     const size_t coh_need = (prec == RVS_PREC_FP32_REFINE || sort_exact) ? coh_bytes(n, D) : 0;
-    const FastTuning ft = c->tuning_for(robot, env, L, M);
-    const size_t links_need = (prec == RVS_PREC_FP32_REFINE && ft.variant == 4) ? fast_links_bytes(n) : 0;
+    FastTuning ft = c->tuning_for(robot, env, L, M, n);
+    size_t links_need = (prec == RVS_PREC_FP32_REFINE && ft.variant == 4) ? fast_links_bytes(n) : 0;
+    // a link-major shape that nobody recorded gives way to lane refill (the
+    // same results) when its lists cannot be had
+    auto without_links = [&]() {
+        if (!links_need || c->tuned(robot, env)) return false;
+        ft.variant = 1;
+        ft.block = 256;
+        links_need = 0;
+        return true;
+    };
     int32_t* ridx = nullptr;
     uint32_t* rcount = nullptr;
     uint32_t* coh = nullptr;
     uint32_t* links = nullptr;
     if (flags & RVS_F_DEVICE) {
         e = c->arena.ensure(Carve::need({refine_bytes, coh_need, links_need}));
+        if (e != hipSuccess && without_links()) e = c->arena.ensure(Carve::need({refine_bytes, coh_need}));
         if (e != hipSuccess) return hip_fail(c, e, "rvs_distance: staging");
         Carve cv(c->arena.p);
         if (refine_bytes) { rcount = cv.take<uint32_t>(64); ridx = cv.take<int32_t>(n); }
@@ -803,10 +813,12 @@ rvs_status rvs_distance(rvs_context* c, int32_t robot, int32_t env, const float*
         if (links_need) links = cv.take<uint32_t>(links_need / 4);
         out.d = d; out.profile = profile; out.nearest = nearest; out.verdict = verdict;
     } else {
-        const size_t need = Carve::need({refine_bytes, coh_need, links_need, (size_t)n * D * 4, (size_t)n * 4,
-                                         profile ? (size_t)n * L * 4 : 0, nearest ? (size_t)n * M * L * 24 : 0,
-                                         (size_t)n});
-        e = c->arena.ensure(need);
+        auto need = [&]() {
+            return Carve::need({refine_bytes, coh_need, links_need, (size_t)n * D * 4, (size_t)n * 4,
+                                profile ? (size_t)n * L * 4 : 0, nearest ? (size_t)n * M * L * 24 : 0, (size_t)n});
+        };
+        e = c->arena.ensure(need());
+        if (e != hipSuccess && without_links()) e = c->arena.ensure(need());
         if (e != hipSuccess) return hip_fail(c, e, "rvs_distance: staging");
         Carve cv(c->arena.p);
         if (refine_bytes) { rcount = cv.take<uint32_t>(64); ridx = cv.take<int32_t>(n); }
@@ -845,7 +857,7 @@ rvs_status rvs_distance(rvs_context* c, int32_t robot, int32_t env, const float*
             if (e == hipSuccess && timing) e = hipEventRecord(c->ev[0], c->stream);
             const int32_t* perm = nullptr;
             if (e == hipSuccess && sort_exact)
-                e = launch_coherence_order(rb.dev, qd, n, c->tuning_for(robot, env, L, M), coh, &perm, c->stream);
+                e = launch_coherence_order(rb.dev, qd, n, c->tuning_for(robot, env, L, M, n), coh, &perm, c->stream);
             if (e == hipSuccess)
                 e = (prec == RVS_PREC_FP64)
                         ? launch_distance_fp64(rb.dev, ev.dev, qp, qd, n, out, c->stream, perm)
@@ -906,7 +918,7 @@ hipError_t async_exact_order(rvs_context* c, int32_t robot, int32_t env, const R
     if (e != hipSuccess) return e;
     Carve cv(c->arena.p);
     uint32_t* coh = cv.take<uint32_t>(coh_bytes(n, rb.num_dofs) / 4);
-    return launch_coherence_order(rb.dev, q, n, c->tuning_for(robot, env, rb.num_links, ev.dev.num_obj), coh, perm,
+    return launch_coherence_order(rb.dev, q, n, c->tuning_for(robot, env, rb.num_links, ev.dev.num_obj, n), coh, perm,
                                   st);
 }
 
@@ -934,11 +946,18 @@ rvs_status rvs_distance_async(rvs_context* c, int32_t robot, int32_t env, const 
     hipError_t e = async_begin(c, st);
     if (e == hipSuccess && n > 0) {
         if (prec == RVS_PREC_FP32_REFINE) {
-            const FastTuning ft = c->tuning_for(robot, env, L, M);
-            const size_t links_need = ft.variant == 4 ? fast_links_bytes(n) : 0;
+            FastTuning ft = c->tuning_for(robot, env, L, M, n);
+            size_t links_need = ft.variant == 4 ? fast_links_bytes(n) : 0;
             const size_t need = Carve::need({(size_t)n * 4 + 256, coh_bytes(n, D), links_need});
             if (need > c->arena.cap) c->drain_async();   // growing frees the block earlier calls use
             e = c->arena.ensure(need);
+            if (e != hipSuccess && links_need && !c->tuned(robot, env)) {
+                // a link-major shape that nobody recorded gives way to lane refill (the same results)
+                ft.variant = 1;
+                ft.block = 256;
+                links_need = 0;
+                e = c->arena.ensure(Carve::need({(size_t)n * 4 + 256, coh_bytes(n, D)}));
+            }
             if (e != hipSuccess) return hip_fail(c, e, "rvs_distance_async: staging");
             Carve cv(c->arena.p);
             uint32_t* rcount = cv.take<uint32_t>(64);
@@ -996,7 +1015,7 @@ rvs_status rvs_distance_async_static(rvs_context* c, int32_t robot, int32_t env,
     const QueryParams qp = params_of(c);
     DistOut out{};
     out.d = d; out.profile = profile; out.verdict = verdict;
-    const FastTuning ft = c->tuning_for(robot, env, L, M);
+    const FastTuning ft = c->tuning_for(robot, env, L, M, n);
     hipError_t e = async_begin(c, st);
     if (e == hipSuccess && n > 0) {
         Carve cv(base);
@@ -1008,7 +1027,7 @@ rvs_status rvs_distance_async_static(rvs_context* c, int32_t robot, int32_t env,
             // counters cleared by a kernel: the scratch keeps the last call's contents
             e = launch_zero_u32(rcount, 64, st);
             if (e == hipSuccess) e = launch_coherence_order(rb.dev, q, n, ft, coh, &perm, st);
-            // no links scratch in the static array: a link-major tuning runs as variant 3
+            // no links scratch in the static array: a link-major shape runs as variant 3
             if (e == hipSuccess)
                 e = launch_distance_fast(rb.dev, ev.dev, qp, q, n, out, ridx, rcount, ft, perm, nullptr, c->num_cus,
                                          st);
@@ -1217,7 +1236,7 @@ rvs_status rvs_get_tuning(rvs_context* c, int32_t robot, int32_t env, rvs_tuning
         if (robot_ok(c, robot)) L = c->robots[robot].num_links;
         if (env_ok(c, env)) M = c->envs[env].dev.num_obj;
     }
-    const FastTuning f = c->tuning_for(robot, env, L, M);
+    const FastTuning f = c->tuning_for(robot, env, L, M, 0);
     *t = rvs_tuning{f.variant, f.block, f.blocks_per_cu, f.coh_bits, 0.0f};
     return RVS_OK;
 }
@@ -1265,7 +1284,7 @@ rvs_status rvs_distance_f64(rvs_context* c, int32_t robot, int32_t env, const fl
     }
     const int32_t* perm = nullptr;
     if (e == hipSuccess && coh)
-        e = launch_coherence_order(rb.dev, qd, n, c->tuning_for(robot, env, L, ev.dev.num_obj), coh, &perm, c->stream);
+        e = launch_coherence_order(rb.dev, qd, n, c->tuning_for(robot, env, L, ev.dev.num_obj, n), coh, &perm, c->stream);
     if (e == hipSuccess) e = launch_distance_fp64(rb.dev, ev.dev, qp, qd, n, out, c->stream, perm);
     if (e == hipSuccess && !(flags & RVS_F_DEVICE)) {
         e = d2h(d, out.d64, (size_t)n * 8, c->stream);
@@ -1317,7 +1336,7 @@ rvs_status rvs_is_valid(rvs_context* c, int32_t robot, int32_t env, const float*
     const bool timing = (flags & RVS_F_TIMING) != 0;
     if (e == hipSuccess && timing) e = hipEventRecord(c->ev[0], c->stream);
     if (e == hipSuccess && coh)
-        e = launch_coherence_order(rb.dev, qd, n, c->tuning_for(robot, env, rb.num_links, ev.dev.num_obj), coh, &perm,
+        e = launch_coherence_order(rb.dev, qd, n, c->tuning_for(robot, env, rb.num_links, ev.dev.num_obj, n), coh, &perm,
                                    c->stream);
     if (e == hipSuccess && timing) e = hipEventRecord(c->ev[1], c->stream);
     if (e == hipSuccess) e = launch_is_valid(rb.dev, ev.dev, qp, qd, n, vd, fp64, c->stream, perm);

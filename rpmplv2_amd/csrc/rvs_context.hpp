@@ -111,8 +111,7 @@ struct rvs_context {
     int32_t nstages = 0;
     int32_t num_cus = 0;
     // FP32 bulk pass variant when no tuning is recorded: -1 = by walk length
-    // (lane refill when links x obstacles >= 1024), 0 = one lane per
-    // configuration, 1 = lane refill
+    // and batch (tuning_for), otherwise the variant
     int32_t fast_variant = -1;
     // reference-arithmetic distance batches up to this many configurations
     // run one wave per configuration (latency) instead of one lane
@@ -134,13 +133,35 @@ struct rvs_context {
     uint32_t* count_host = nullptr;   // pinned, coherent: refinement count the graphs' refinement stores
     uint32_t* count_dev = nullptr;    // the same word's device address
     std::mutex tuning_mu;
-    rvs::FastTuning tuning_for(int32_t robot, int32_t env, int32_t links, int32_t objects) {
+    // The launch shape of an RVS_PREC_FP32_REFINE batch of n configurations:
+    // the recorded one, else by the length of the walk and the batch (every
+    // shape gives the same bits, so the choice may follow n).
+    rvs::FastTuning tuning_for(int32_t robot, int32_t env, int32_t links, int32_t objects, int64_t n) {
         std::lock_guard<std::mutex> lk(tuning_mu);
         auto it = tuning.find({robot, env});
         if (it != tuning.end()) return it->second;
-        const int32_t v = fast_variant >= 0 ? fast_variant : ((int64_t)links * objects >= 1024 ? 1 : 0);
         // one lane per configuration: 64-thread workgroups measured fastest
-        return rvs::FastTuning{v, v == 0 ? 64 : 256, 0, 5};
+        if (fast_variant >= 0) return rvs::FastTuning{fast_variant, fast_variant == 0 ? 64 : 256, 0, 5};
+        if ((int64_t)links * objects < 1024) return rvs::FastTuning{0, 64, 0, 5};
+        // Long walks.  Link-major launches (4) against lane refill (1), 22-DOF
+        // chain: 512 boxes 5.9 against 11.7 ms for 2,097,152 configurations and
+        // 2.1 against 2.5 ms for 1,000; 256 boxes 3.5 against 5.0 ms for
+        // 1,000,000 and 1.2 against 1.6 for 1,000; 128 boxes 3.5 against 3.8 ms
+        // for 1,000,000 but 1.64 against 1.58 for 300,000; 96 boxes 3.4 against
+        // 3.2.  Their lists take 128 bytes a configuration: at most 2 GiB.
+        if (n > 0 && n <= (int64_t)1 << 24 && (objects >= 200 || (objects >= 128 && n >= (int64_t)1 << 19)))
+            return rvs::FastTuning{4, 512, 0, 5};
+        // Lane refill with pair queues (3) for small batches: 22-DOF chain and
+        // 96 boxes 0.64 against 0.77 ms for 1,000 and 0.73 against 0.85 for
+        // 30,000; 14-DOF chain and 65 boxes 0.40 against 0.46 for 100,000; but
+        // 18-DOF chain and 80 boxes 1.17 against 1.03 for 400,000.
+        if (n > 0 && n <= (int64_t)1 << 17) return rvs::FastTuning{3, 512, 0, 5};
+        return rvs::FastTuning{1, 256, 0, 5};
+    }
+    // Whether the launch shape of (robot, env) was recorded by a caller.
+    bool tuned(int32_t robot, int32_t env) {
+        std::lock_guard<std::mutex> lk(tuning_mu);
+        return tuning.find({robot, env}) != tuning.end();
     }
 };
 

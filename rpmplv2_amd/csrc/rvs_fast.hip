@@ -28,6 +28,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <climits>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -549,9 +550,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // queueing bound is never tighter than the walk's, a member's box lies
 // inside its group's, and every pair is tested again with exactly the bound
 // the walk has when it reaches it); the search evaluates every candidate
-// before the hit instead of stopping at the first, which can only add
-// screening flags.  The link's value, the warm pair of the next link and the
-// verdict are those of link_min.
+// before the hit instead of stopping at the first, and drops the screening
+// flags of candidates past the first hit, which link_min's search would not
+// have reached.  The link's value, the warm pair of the next link, the flags
+// and the verdict are those of link_min.
 constexpr int kLaneQueue = 16;         // pending pairs per lane (power of 2, > kGroupSize)
 constexpr int kDrainLanes = 40;        // an evaluation step once this many lanes hold a pair
 
@@ -627,15 +629,15 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
         Vec3<float> slo, shi;
         seg_bounds(P0, P1, slo, shi);
         const bool gnd_skip = i < rb.ground_included;
-        auto eval = [&](int j) {
-            return (s.gnd[j] && gnd_skip) ? p.maxd : flat_pair<OBB>(s, j, P0, P1, r, p, band, uncertain);
+        auto eval = [&](int j, bool& u) {
+            return (s.gnd[j] && gnd_skip) ? p.maxd : flat_pair<OBB>(s, j, P0, P1, r, p, band, u);
         };
         // 1. the warm pair
         float prof = p.maxd, vh = 0.0f;
         int best = -1, jh = -1;
         const int w = busy ? warm : -1;
         if (w >= 0) {
-            const float dw = eval(w);
+            const float dw = eval(w, uncertain);
             if (dw <= 0) {
                 jh = w;
                 vh = dw;
@@ -656,7 +658,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
                 if (!cull_fast(lcull + 6 * j, slo, shi, cull_bound2(prof, r, p.eq))) task = j;
             }
             if (task >= 0) {
-                const float dt = eval(task);
+                const float dt = eval(task, uncertain);
                 if (dt < prof) best = task;
                 prof = smin(prof, dt);
                 if (prof <= 0) {
@@ -691,13 +693,16 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
             const float bb0 = cull_bound2(0.0f, r, p.eq);
             int fj = jh;
             float fv = vh;
+            int uj = INT_MAX;   // smallest uncertain candidate
             auto search_step = [&]() {
                 if (qn > 0) {
                     const int j = ring[(qh & (kLaneQueue - 1)) * B];
                     ++qh;
                     --qn;
                     if (j < fj) {
-                        const float dt = eval(j);
+                        bool u = false;
+                        const float dt = eval(j, u);
+                        if (u) uj = min(uj, j);
                         if (dt <= 0) {
                             fj = j;
                             fv = dt;
@@ -721,7 +726,10 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
                 while (__ballot(qn > kLaneQueue - kGroupSize)) search_step();
             }
             while (__ballot(qn > 0)) search_step();
-            if (srch) vh = fv;
+            if (srch) {
+                vh = fv;
+                uncertain |= uj <= fj;
+            }
         }
         // the link's value
         bool finished = false;
@@ -783,20 +791,12 @@ __device__ __attribute__((always_inline)) inline uint32_t point_key(const Vec3<f
     return key;
 }
 
-// Set-up of the link-major walk (one workgroup of kBoxThreads):
-//   box[0..5]: the box quantizing the survivors' sort keys, the union of the
-//     scene's group boxes (finite coordinates only) as lo[3], 1024 /
-//     extent[3] (0 for an empty extent);
-//   warm0: the first link's warm pair, the obstacle whose cull box is nearest
-//     to configuration 0's first skeleton point (smallest index on ties; -1
-//     without obstacles).  Any obstacle gives the walk the same results; a
-//     near one gives the first link a tight bound from its first pair.
+// Set-up of the link-major walk (one workgroup of kBoxThreads): the box
+// quantizing the survivors' sort keys, the union of the scene's group boxes
+// (finite coordinates only) as lo[3], 1024 / extent[3] (0 for an empty extent).
 constexpr int kBoxThreads = 256;
-__global__ __launch_bounds__(kBoxThreads) void k_links_setup(RobotDev rb, EnvDev env, const float* __restrict__ q,
-                                                             float* __restrict__ box, int32_t* __restrict__ warm0) {
+__global__ __launch_bounds__(kBoxThreads) void k_links_setup(EnvDev env, float* __restrict__ box) {
     __shared__ float red[6][kBoxThreads];
-    __shared__ float bd[kBoxThreads];
-    __shared__ int bj[kBoxThreads];
     const int ng = num_groups(env.num_obj);
     float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
     for (int g = threadIdx.x; g < ng; g += kBoxThreads)
@@ -805,46 +805,18 @@ __global__ __launch_bounds__(kBoxThreads) void k_links_setup(RobotDev rb, EnvDev
             if (isfinite(l)) lo[a] = fminf(lo[a], l);
             if (isfinite(h)) hi[a] = fmaxf(hi[a], h);
         }
-    FKf fk;
-    fk.M = Mat3f{1.0f, 0.0f, 0.0f, 0.0f, 1.0f, 0.0f, 0.0f, 0.0f, 1.0f};
-    fk.px = fk.py = fk.pz = 0.0f;
-    fk.seg = 0;
-    fk.qi = 0;
-    const Vec3<float> P = skelf_point(fk, rb, q, 0);
-    float best = INFINITY;
-    int bestj = -1;
-    for (int j = threadIdx.x; j < env.num_obj; j += kBoxThreads) {
-        const float* cb = env.cull + 6 * j;
-        const float gx = fmaxf(fmaxf(cb[0] - P.x, P.x - cb[3]), 0.0f);
-        const float gy = fmaxf(fmaxf(cb[1] - P.y, P.y - cb[4]), 0.0f);
-        const float gz = fmaxf(fmaxf(cb[2] - P.z, P.z - cb[5]), 0.0f);
-        const float g2 = fmaf(gz, gz, fmaf(gy, gy, gx * gx));
-        if (g2 < best) {   // ascending j per thread: the first of equals stays
-            best = g2;
-            bestj = j;
-        }
-    }
     for (int a = 0; a < 3; ++a) {
         red[a][threadIdx.x] = lo[a];
         red[3 + a][threadIdx.x] = hi[a];
     }
-    bd[threadIdx.x] = best;
-    bj[threadIdx.x] = bestj;
     __syncthreads();
     for (int w = kBoxThreads / 2; w > 0; w >>= 1) {
         const int t = threadIdx.x;
-        if (t < w) {
+        if (t < w)
             for (int a = 0; a < 3; ++a) {
                 red[a][t] = fminf(red[a][t], red[a][t + w]);
                 red[3 + a][t] = fmaxf(red[3 + a][t], red[3 + a][t + w]);
             }
-            const float d2 = bd[t + w];
-            const int j2 = bj[t + w];
-            if (j2 >= 0 && (bj[t] < 0 || d2 < bd[t] || (d2 == bd[t] && j2 < bj[t]))) {
-                bd[t] = d2;
-                bj[t] = j2;
-            }
-        }
         __syncthreads();
     }
     if (threadIdx.x < 3) {
@@ -854,7 +826,6 @@ __global__ __launch_bounds__(kBoxThreads) void k_links_setup(RobotDev rb, EnvDev
         box[a] = ok ? l : 0.0f;
         box[3 + a] = ok ? 1024.0f / (h - l) : 0.0f;
     }
-    if (threadIdx.x == 0) *warm0 = bj[0];
 }
 
 // A round's cell counts and per-wave words (256 + 48 words) reuse the queue
@@ -870,8 +841,7 @@ static_assert(kLaneQueue * sizeof(int16_t) * 256 >= (256 + 48) * sizeof(uint32_t
 //      frame the previous link's launch left in the list entry (the same
 //      compositions in the same order as the incremental walk, so the same
 //      bits);
-//   2. the warm pair (the previous link's nearest obstacle; for the first
-//      link the obstacle nearest to the first skeleton point), all lanes in
+//   2. the warm pair (the previous link's nearest obstacle), all lanes in
 //      one step;
 //   3. the wave's candidate groups: 64 groups at a time, one per lane, tested
 //      against the union of the lanes' segment boxes with the largest of
@@ -890,14 +860,16 @@ static_assert(kLaneQueue * sizeof(int16_t) * 256 >= (256 + 48) * sizeof(uint32_t
 //      smaller index than the smallest hit found.  Every position before the
 //      hit held a pair evaluated above 0 or culled with a bound at least that
 //      of a minimum of 0, which never culls a pair whose distance can be
-//      <= 0: none of them can be an earlier hit.
-// The link's value (the value at the first hit in obstacle order, or the
-// minimum over the pairs, which no culled pair can lower) and the verdict
-// are those of link_min whatever the warm pair; the walk evaluates the pairs
-// of link_min's walk up to its hit in its order when their warm pairs agree
+//      <= 0: none of them can be an earlier hit.  Screening flags of
+//      candidates past the first hit are dropped: link_min's search, in
+//      obstacle order, stops at it.
+// The walk evaluates the pairs of link_min's walk up to its hit in its order
 // (the queueing bound is never tighter than the walk's, a member's box lies
 // inside its group's, and every pair is tested again with exactly the bound
-// the walk has when it reaches it).  A configuration that goes on keeps its
+// the walk has when it reaches it), and the search counts the pairs of
+// link_min's: the link's value, the flags and the verdict are its own, bit for
+// bit.  (A first link warmed by the obstacle nearest to the base, with other
+// flags, took 5% less time.)  A configuration that goes on keeps its
 // running minimum, warm pair, screening flag and walk state in its entry
 // of the next link's list; a round's survivors are ordered by the Morton code
 // (over box) of their next link's start point, at the resolution of 256 cells
@@ -913,7 +885,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
     RobotDev rb, EnvDev env, QueryParams qp, const float* __restrict__ q, int64_t n, DistOut out, int32_t* idx,
     uint32_t* count, int link, const int32_t* __restrict__ perm, const LinkEntry* __restrict__ in,
     const uint32_t* __restrict__ in_count, uint32_t* cursor, LinkEntry* __restrict__ next_list, uint32_t* next_count,
-    const float* __restrict__ box, const int32_t* __restrict__ warm0, size_t cull_off, size_t queue_off) {
+    const float* __restrict__ box, size_t cull_off, size_t queue_off) {
     // configurations at this link: the first takes all n (in the walk order
     // perm, or the order given), the others the previous link's list
     const int64_t cnt = link == 0 ? n : (int64_t)*in_count;
@@ -929,7 +901,6 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
     const const_ptr<float> ccull = as_const(env.cull);
     const const_ptr<int32_t> gorder = as_const(env.gorder);
     const float kbox[6] = {box[0], box[1], box[2], box[3], box[4], box[5]};
-    const int first_warm = link == 0 ? *warm0 : -1;
     const int M = env.num_obj;
     const int L = rb.num_links;
     const int D = rb.num_dofs;
@@ -951,7 +922,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
         const bool busy = e < cnt;
         int64_t c = 0;
         float d = p.maxd;
-        int warm = first_warm;
+        int warm = -1;
         int uk = -1;   // the first link with an uncertain decision
         bool uncertain = false;
         Vec3<float> P0{0.0f, 0.0f, 0.0f}, P1{0.0f, 0.0f, 0.0f};
@@ -986,15 +957,15 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
         }
         Vec3<float> slo, shi;
         seg_bounds(P0, P1, slo, shi);
-        auto eval = [&](int j) {
-            return (s.gnd[j] && gnd_skip) ? p.maxd : flat_pair<OBB>(s, j, P0, P1, r, p, band, uncertain);
+        auto eval = [&](int j, bool& u) {
+            return (s.gnd[j] && gnd_skip) ? p.maxd : flat_pair<OBB>(s, j, P0, P1, r, p, band, u);
         };
         // 2. the warm pair
         float prof = p.maxd, vh = 0.0f;
         int best = -1, jh = -1;   // jh: the smallest hit index found (-1: walking)
         const int w = busy ? warm : -1;
         if (w >= 0) {
-            const float dw = eval(w);
+            const float dw = eval(w, uncertain);
             if (dw <= 0) {
                 jh = w;
                 vh = dw;
@@ -1016,6 +987,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
         const float ubb = wave_max(bb);
         // 4-5. the walk, then the search, its pairs evaluated from the queues
         int qh = 0, qt = 0, qn = 0;   // ring head, tail and length
+        int uj = INT_MAX;             // smallest uncertain candidate of the search
         auto step = [&]() {   // one queued pair per lane
             int task = -1;
             while (qn > 0 && task < 0) {
@@ -1025,8 +997,10 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
                 if (j < lim && !cull_fast(lcull + 6 * j, slo, shi, bb)) task = j;
             }
             if (task >= 0) {
-                const float dt = eval(task);
+                bool u = false;
+                const float dt = eval(task, u);
                 if (jh < 0) {
+                    uncertain |= u;
                     if (dt < prof) best = task;
                     prof = smin(prof, dt);
                     if (prof <= 0) {
@@ -1037,10 +1011,13 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
                     } else {
                         bb = cull_bound2(prof, r, p.eq);
                     }
-                } else if (dt <= 0) {
-                    jh = task;
-                    vh = dt;
-                    lim = task;
+                } else {
+                    if (u) uj = min(uj, task);
+                    if (dt <= 0) {
+                        jh = task;
+                        vh = dt;
+                        lim = task;
+                    }
                 }
             }
         };
@@ -1077,8 +1054,9 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
         // the link's value
         bool finished = false;
         if (busy) {
-            if (uncertain && uk < 0) uk = i;
             const bool hit = jh >= 0;
+            uncertain |= hit && uj <= jh;
+            if (uncertain && uk < 0) uk = i;
             const float lp = hit ? vh : prof;
             if (out.profile) out.profile[c * L + i] = lp;
             if (hit) {
@@ -1503,14 +1481,14 @@ hipError_t launch_fast_shape(const RobotDev& rb, const EnvDev& env, const QueryP
             const dim3 g((unsigned)std::max<int64_t>(1, blocks)), b(BL);
             hipError_t e = launch_zero_u32(ll.count, kLinksCounters, st);
             if (e == hipSuccess) {
-                hipLaunchKernelGGL(k_links_setup, dim3(1), dim3(kBoxThreads), 0, st, rb, env, q, ll.box, ll.warm0);
+                hipLaunchKernelGGL(k_links_setup, dim3(1), dim3(kBoxThreads), 0, st, env, ll.box);
                 e = hipGetLastError();
             }
             for (int i = 0; i < rb.num_links && e == hipSuccess; ++i) {
                 const LinkEntry* in = i == 0 ? nullptr : ll.list[(i - 1) & 1];
                 hipLaunchKernelGGL((k_distance_fast_links<OBB>), g, b, lsm, st, rb, env, qp, q, n, out, idx, count, i,
                                    perm, in, ll.count + i, ll.cursor + i, ll.list[i & 1], ll.count + i + 1, ll.box,
-                                   ll.warm0, cull_off, queue_off);
+                                   cull_off, queue_off);
                 e = hipGetLastError();
             }
             return e;

@@ -204,8 +204,7 @@ hipError_t launch_coherence_order(const RobotDev& rb, const float* q, int64_t n,
 // (warm pair + 1) << 1 | screening flag and the forward-kinematics walk up to
 // the link's end point, so that the next link goes on from there; then the
 // lists' sizes per link and the round counters per link (kLinksCounters
-// words, cleared together), the box that quantizes the sort keys and the
-// first link's warm pair.
+// words, cleared together) and the box that quantizes the sort keys.
 struct alignas(16) LinkEntry {
     int32_t c;       // configuration
     float d;         // running minimum over the links before
@@ -222,7 +221,6 @@ struct LinksLayout {
     uint32_t* count;    // [kMaxLinks + 1] list sizes, then
     uint32_t* cursor;   // [kMaxLinks + 1] round counters
     float* box;         // lo[3], 1024 / extent[3]
-    int32_t* warm0;
 };
 inline size_t fast_links_bytes(int64_t n) {
     const size_t m = (size_t)std::max<int64_t>(n, 0);
@@ -236,7 +234,6 @@ inline LinksLayout links_layout(uint32_t* base, int64_t n) {
     L.count = base + 2 * lw;
     L.cursor = L.count + kMaxLinks + 1;
     L.box = reinterpret_cast<float*>(L.count + coh_words(kLinksCounters));
-    L.warm0 = reinterpret_cast<int32_t*>(L.box + 6);
     return L;
 }
 // The persistent variants (1: lane refill, 2: chunks, 3: per-lane queues)

@@ -129,3 +129,37 @@ def test_walk_order_covers_every_configuration(engine, case):
             else:
                 assert np.array_equal(got[2], ref[2]), (cb, variant)
                 assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1]), (cb, variant)
+
+
+@pytest.mark.parametrize("scene", ["obb512", "overlap200", "tolerances130"])
+def test_launch_shapes_same_bits(engine, scene):
+    """Every variant gives the same distances, profiles, verdicts and refined
+    set, bit for bit: among rotated boxes, among large overlapping boxes (first
+    hits in obstacle order behind the first hit found) and with finite
+    tolerances and ground boxes; and so does the shape a call chooses itself."""
+    if scene == "obb512":
+        w, sem = W.workload5(6000), rvs.ENV_OBB
+        rb, sc, q = w.robot, w.scene, w.q
+    else:
+        rng = np.random.default_rng(17)
+        m = 200 if scene == "overlap200" else 130
+        rb = R.chain(rng.uniform(0.1, 0.3, 10), radius=0.05, ground_included=2)
+        sc = W._boxes(rng, m, 0.05, 0.6 if scene == "overlap200" else 0.2, 1.5)
+        pos = sc.pos * np.where(np.linalg.norm(sc.pos[:, :2], axis=1) < 0.5, 2.0, 1.0)[:, None]
+        tol, gnd = sc.min_dist_tol.copy(), sc.is_ground.copy()
+        if scene != "overlap200":
+            tol[::3] = 0.07
+            gnd[::5] = 1
+        sc, sem = W.Scene(sc.dim, pos, sc.quat, gnd, tol), rvs.ENV_AABB
+        q = rng.uniform(-np.pi, np.pi, (6000, 10)).astype(np.float32)
+    rid = engine.load_robot(rb)
+    ref = engine.distance(rid, engine.create_env(sc, sem), q, precision=rvs.PREC_FP32_REFINE)
+    nref = engine.last_refined()
+    eid = engine.create_env(sc, sem)
+    for variant, block in ((0, 64), (1, 256), (2, 128), (3, 512), (4, 256), (4, 512)):
+        engine.set_tuning(rid, eid, variant, block, 0, 5)
+        got = engine.distance(rid, eid, q, precision=rvs.PREC_FP32_REFINE)
+        assert engine.last_refined() == nref, (variant, block)
+        for a, b in zip(got[:3], ref[:3]):
+            assert np.array_equal(a, b), (variant, block)
+    assert 0 < nref < len(q) and 0.01 < ref[2].mean() < 0.99
