@@ -204,6 +204,54 @@ __host__ __device__ __attribute__((always_inline)) inline Vec3<T> skel_point_sc(
     return P;
 }
 
+// The same kinematics with the lanes of a group sharing one configuration's
+// work, bit for bit: segment poses first (a segment a lane), then the frames'
+// product row by row (row r of the frame and coordinate r of its origin need
+// only themselves: lane r carries them, 21 operations a segment instead of
+// 133).  A segment's pose takes 12 doubles: rotation (row major), origin.
+__device__ __attribute__((always_inline)) inline void seg_pose_store(double* e, const SegDev& g, const float* q) {
+    Mat3 SM = mat_load(g.R);
+    if (g.rev) {
+        double st, ct;
+        sincos((double)q[g.joint], &st, &ct);
+        SM = mat_mul(rot2(g.axis, st, ct), SM);
+    }
+    e[0] = SM.m0; e[1] = SM.m1; e[2] = SM.m2;
+    e[3] = SM.m3; e[4] = SM.m4; e[5] = SM.m5;
+    e[6] = SM.m6; e[7] = SM.m7; e[8] = SM.m8;
+    e[9] = g.o[0]; e[10] = g.o[1]; e[11] = g.o[2];
+}
+// Coordinate r of skeleton points 0 .. L to skel[3 k + r] (write false: the
+// lane only follows), from the poses segs and the recipe pts.
+__device__ __attribute__((always_inline)) inline void skeleton_row(const double* segs, const PointDev* pts, int L,
+                                                                 int r, float* skel, bool write) {
+    double m0 = r == 0 ? 1.0 : 0.0, m1 = r == 1 ? 1.0 : 0.0, m2 = r == 2 ? 1.0 : 0.0, x = 0.0;
+    int seg = 0;
+    for (int k = 0; k <= L; ++k) {
+        const PointDev pt = pts[k];
+        for (; seg <= pt.frame; ++seg) {
+            const double* e = segs + 12 * seg;
+            x = m0 * e[9] + m1 * e[10] + m2 * e[11] + x;
+            const double n0 = m0 * e[0] + m1 * e[3] + m2 * e[6];
+            const double n1 = m0 * e[1] + m1 * e[4] + m2 * e[7];
+            const double n2 = m0 * e[2] + m1 * e[5] + m2 * e[8];
+            m0 = n0;
+            m1 = n1;
+            m2 = n2;
+        }
+        float P = 0.0f;
+        if (pt.frame >= 0) {
+            const double w0 = pt.axis == 0 ? 1.0 : 0.0, w1 = pt.axis == 1 ? 1.0 : 0.0, w2 = pt.axis == 2 ? 1.0 : 0.0;
+            const double a = m0 * w0 + m1 * w1 + m2 * w2;
+            double v = x;
+            if (pt.flags & 1) v = v + pt.pre * a;
+            P = (float)v;
+            if (pt.flags & 2) P = P - (float)pt.post * (float)a;
+        }
+        if (write) skel[3 * k + r] = P;
+    }
+}
+
 // Skeleton point k with the joint values read from q (joint m is
 // q[m * qstride]; points must be requested in increasing k).
 template <typename T>

@@ -73,13 +73,6 @@ inline PairLds pair_lds(const RobotDev& rb, const EnvDev& env, bool want_np, int
     return l;
 }
 
-// Orders the LDS accesses of a wave's lanes (a row belongs to one wave).
-__device__ __attribute__((always_inline)) inline void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // G lanes per configuration (16 or 64), 64 / G configurations per wave; a
 // workgroup is one wave.
 //   1. Lane m of the group works out segment m's rotation (and m + G's, ...),
@@ -145,20 +138,7 @@ __global__ __launch_bounds__(64) void k_distance_pairs(RobotDev rb, EnvDev env, 
         int k0 = 0;   // the first link to compute
         flag_decode(idx, live ? kb + grp : total - 1, qp, out, c, k0);
         const float* qc = q + c * D;
-        for (int m = t; m < S; m += G) {
-            const SegDev g = rb.seg[m];
-            Mat3 SM = mat_load(g.R);
-            if (g.rev) {
-                double st, ct;
-                sincos((double)qc[g.joint], &st, &ct);
-                SM = mat_mul(rot2(g.axis, st, ct), SM);
-            }
-            double* e = row.seg + 12 * m;
-            e[0] = SM.m0; e[1] = SM.m1; e[2] = SM.m2;
-            e[3] = SM.m3; e[4] = SM.m4; e[5] = SM.m5;
-            e[6] = SM.m6; e[7] = SM.m7; e[8] = SM.m8;
-            e[9] = g.o[0]; e[10] = g.o[1]; e[11] = g.o[2];
-        }
+        for (int m = t; m < S; m += G) seg_pose_store(row.seg + 12 * m, rb.seg[m], qc);
         for (int i = t; i < L; i += G) {
             row.near_key[i] = ~0ull;
             row.hit_key[i] = ~0ull;
@@ -166,37 +146,7 @@ __global__ __launch_bounds__(64) void k_distance_pairs(RobotDev rb, EnvDev env, 
         }
         if (t == 0) *row.first_link = L;
         wave_sync();
-        {
-            // row r of the frame and coordinate r of its origin (fk_advance_sc
-            // and skel_point_sc, one row of each); lanes 3 and up follow row 0
-            const int r = t < 3 ? t : 0;
-            double m0 = r == 0 ? 1.0 : 0.0, m1 = r == 1 ? 1.0 : 0.0, m2 = r == 2 ? 1.0 : 0.0, x = 0.0;
-            int seg = 0;
-            for (int k = 0; k <= L; ++k) {
-                const PointDev pt = pts[k];
-                for (; seg <= pt.frame; ++seg) {
-                    const double* e = row.seg + 12 * seg;
-                    x = m0 * e[9] + m1 * e[10] + m2 * e[11] + x;
-                    const double n0 = m0 * e[0] + m1 * e[3] + m2 * e[6];
-                    const double n1 = m0 * e[1] + m1 * e[4] + m2 * e[7];
-                    const double n2 = m0 * e[2] + m1 * e[5] + m2 * e[8];
-                    m0 = n0;
-                    m1 = n1;
-                    m2 = n2;
-                }
-                float P = 0.0f;
-                if (pt.frame >= 0) {
-                    const double w0 = pt.axis == 0 ? 1.0 : 0.0, w1 = pt.axis == 1 ? 1.0 : 0.0;
-                    const double w2 = pt.axis == 2 ? 1.0 : 0.0;
-                    const double a = m0 * w0 + m1 * w1 + m2 * w2;
-                    double v = x;
-                    if (pt.flags & 1) v = v + pt.pre * a;
-                    P = (float)v;
-                    if (pt.flags & 2) P = P - (float)pt.post * (float)a;
-                }
-                if (t < 3) row.skel[3 * k + r] = P;
-            }
-        }
+        skeleton_row(row.seg, pts, L, t < 3 ? t : 0, row.skel, t < 3);   // lanes 3 and up follow row 0
         wave_sync();
         // the loop's view of pair (i, j) of a row: min(MAX_DISTANCE, filtered
         // distance), MAX_DISTANCE for a NaN; and its place in the row

@@ -98,6 +98,13 @@ __device__ __attribute__((always_inline)) inline Vec3<T> from_box(const float* x
 // Compares squared values (no square root); a NaN end point never culls.
 constexpr float kCullMargin = 1e-5f;
 
+// Orders the LDS accesses of a wave's lanes (LDS that one wave alone uses).
+__device__ __attribute__((always_inline)) inline void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Squared gap between the segment's bounding box and the box cb (0 on an
 // axis where they overlap or a coordinate is NaN).
 template <typename T>

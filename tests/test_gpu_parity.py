@@ -1074,3 +1074,39 @@ def test_self_collision_minimum_of_pairs(engine, dofs, n, scale):
     all_pairs = engine.self_distance(rid, q)
     want = np.fmin.reduce(np.concatenate([np.full((n, 1), 1000.0, np.float32), all_pairs], 1), axis=1)
     assert np.array_equal(lo, want) and np.array_equal(free, (want >= 0).astype(np.uint8))
+
+
+@pytest.mark.parametrize("dofs,boxes,points,traj", [(6, 1, 1, 5), (6, 16, 64, 70), (6, 70, 65, 40), (10, 9, 130, 30),
+                                                    (22, 12, 20, 20), (2, 3, 1025, 9), (40, 5, 3, 7)])
+@pytest.mark.parametrize("self_collision", [False, True])
+def test_trajectory_is_safe_sizes(oracle, engine, dofs, boxes, points, traj, self_collision):
+    """Chunks of 64 points and their remainders, more points than the time
+    table holds, from two to forty joints (segments, radii rows and planes
+    beyond a wave's lanes), moving obstacles: equal to the oracle's walk."""
+    rng = np.random.default_rng(1000 * dofs + points)
+    if dofs == 6:
+        rb = R.xarm6()
+    elif dofs == 2:
+        rb = R.planar_2dof()
+    else:
+        rb = R.chain(rng.uniform(0.03, 0.1, dofs), radius=0.02, self_collision=True)
+    u = rng.normal(size=(boxes, 3))
+    sc = W._boxes(rng, boxes, 0.02, 0.1, 1.0)
+    sc = W.Scene(sc.dim, rng.uniform(1.2, 2.5, (boxes, 1)) * u / np.linalg.norm(u, axis=1, keepdims=True), sc.quat,
+                 sc.is_ground, sc.min_dist_tol)
+    osc = oracle.scene_of(sc)
+    root = np.zeros(dofs, np.float32)
+    _, p0, ok, np0 = oracle.distance(rb, osc, root[None], 32, want_np=True)
+    assert ok[0] == 1
+    v = rng.normal(size=(traj, dofs))
+    v /= np.linalg.norm(v, axis=1, keepdims=True)
+    s = np.linspace(0, 1, points + 1)[1:]
+    pts = (rng.uniform(0.05, 2.5, traj)[:, None, None] * s[None, :, None] * v[:, None, :]).astype(np.float32)
+    mv = rng.uniform(0, 0.05, boxes).astype(np.float32)
+    dt = 1.0 / points
+    rid, eid = engine.load_robot(rb), engine.create_env(sc)
+    safe = engine.trajectory_is_safe(rid, eid, pts, root, p0[0], np0[0], mv, t_iter=0.1, time_step=dt,
+                                     self_collision=self_collision)
+    osafe = oracle.traj_safe(rb, osc, pts, root, p0[0], np0[0], mv, 0.1, dt,
+                             pairs=rb.self_pairs if self_collision else None)
+    assert np.array_equal(safe, osafe)
