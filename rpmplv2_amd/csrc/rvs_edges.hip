@@ -171,10 +171,18 @@ __device__ inline SlabEntry load_entry(ConstPtr<SlabEntry> p) {
 // One link (P0, P1) of radius r against the obstacles of table tab, for the
 // lanes with act set: true where some obstacle collides
 // (collisionCapsuleToBox).  The table pointer and the loop counts are
-// uniform, so the entries, and the bounds of an obstacle that goes to the
-// full test, arrive through scalar loads.
+// uniform, so the entries arrive through scalar loads, kSlabBatch at a time so
+// that one wait covers a batch (an entry a wait left a wave idle for most of
+// the search: 16,384 planner-start edges of four chains 1.60 ms a call so, 1.10
+// ms with this and the joint values and self pairs fetched in batches; 65,536
+// xArm6 edges of ten states 200 against 159 us).  A lane marks the obstacles that its axis tests leave, 64 of the
+// walk order at a time, and then takes its own one after the other to the full
+// test: lanes near different obstacles share its steps, and the kernel holds
+// one copy of it.
+constexpr int kSlabBatch = 4;
+static_assert(kSlabGroup % kSlabBatch == 0 && 64 % kSlabGroup == 0, "whole batches and groups");
 __device__ inline bool link_hits(const Vec3<float>& P0, const Vec3<float>& P1, float r, float rn,
-                                 ConstPtr<SlabEntry> tab, int G, int M, ConstPtr<float> aabb,
+                                 ConstPtr<SlabEntry> tab, int G, int M, const float* __restrict__ aabb,
                                  const Params<float>& p, bool act) {
     // per axis, the larger and the smaller end point coordinate: "both below
     // L" is "the larger below L" unless a coordinate is NaN, and then every
@@ -188,17 +196,55 @@ __device__ inline bool link_hits(const Vec3<float>& P0, const Vec3<float>& P1, f
                (mnz > x.hi[2]);
     };
     bool hit = false;
-    for (int g = 0; g < G; ++g) {
-        const SlabEntry gx = load_entry(tab + g);
-        if (act && !hit && (exact || !apart(gx))) {
-            const int b1 = min(M, (g + 1) * kSlabGroup);
-            for (int b = g * kSlabGroup; b < b1; ++b) {
-                const SlabEntry x = load_entry(tab + G + b);
-                if (!hit && x.idx >= 0 && (exact || !apart(x))) {
-                    ConstPtr<float> o = aabb + 6 * x.idx;
-                    const Box<float> bx{{o[0], o[1], o[2]}, {o[3], o[4], o[5]}};
-                    if (collision_box(P0, P1, r, rn, bx, p)) hit = true;
+    for (int c0 = 0; c0 < M; c0 += 64) {   // positions c0 .. c0 + 63 of the walk order
+        uint32_t mark[2] = {0u, 0u};
+        const int g1 = min(G, c0 / kSlabGroup + 64 / kSlabGroup);
+        for (int g0 = c0 / kSlabGroup; g0 < g1; g0 += kSlabBatch) {
+            SlabEntry gx[kSlabBatch];
+#pragma unroll
+            for (int k = 0; k < kSlabBatch; ++k) gx[k] = load_entry(tab + min(g0 + k, G - 1));
+            uint32_t near = 0;   // the batch's groups that some lane is near
+            bool in[kSlabBatch];
+#pragma unroll
+            for (int k = 0; k < kSlabBatch; ++k) {
+                in[k] = g0 + k < g1 && act && !hit && (exact | !apart(gx[k]));
+                near |= __any(in[k]) ? 1u << k : 0u;
+            }
+            while (near) {   // uniform
+                const int k = __builtin_ctz(near);
+                near &= near - 1;
+                const bool mine = k == 0 ? in[0] : (k == 1 ? in[1] : (k == 2 ? in[2] : in[3]));
+                const int b0 = (g0 + k) * kSlabGroup;
+                uint32_t bits = 0;
+#pragma unroll
+                for (int m0 = 0; m0 < kSlabGroup; m0 += kSlabBatch) {
+                    SlabEntry x[kSlabBatch];
+#pragma unroll
+                    for (int m = 0; m < kSlabBatch; ++m) x[m] = load_entry(tab + G + min(b0 + m0 + m, M - 1));
+#pragma unroll
+                    for (int m = 0; m < kSlabBatch; ++m)
+                        bits |= ((exact | !apart(x[m])) & (x[m].idx >= 0) & (b0 + m0 + m < M)) ? 1u << (m0 + m) : 0u;
                 }
+                const int at = b0 - c0;   // 0, 8, ..., 56
+                const uint32_t put = mine ? bits << (at & 31) : 0u;
+                if (at < 32) mark[0] |= put;
+                else mark[1] |= put;
+            }
+        }
+#pragma clang loop unroll(disable)
+        while (__any(!hit && (mark[0] | mark[1]))) {
+            if (!hit && (mark[0] | mark[1])) {
+                int b;
+                if (mark[0]) {
+                    b = __builtin_ctz(mark[0]);
+                    mark[0] &= mark[0] - 1;
+                } else {
+                    b = 32 + __builtin_ctz(mark[1]);
+                    mark[1] &= mark[1] - 1;
+                }
+                const float* o = aabb + 6 * tab[G + c0 + b].idx;
+                const Box<float> bx{{o[0], o[1], o[2]}, {o[3], o[4], o[5]}};
+                hit = collision_box(P0, P1, r, rn, bx, p);
             }
         }
     }
@@ -237,6 +283,7 @@ __device__ inline bool link_hits_obb(const Vec3<float>& P0, const Vec3<float>& P
 // reference's interpolation is); LDS holds the queue and the skeletons for
 // the self pairs.
 constexpr int kQueue = 128;
+constexpr int kSelfBatch = 4;
 template <bool OBB>
 __global__ __launch_bounds__(64) void k_edge_first_q(EdgeGroups gr, EnvDev env, QueryParams qp,
                                                         const float* __restrict__ q1, const float* __restrict__ dir,
@@ -312,10 +359,17 @@ __global__ __launch_bounds__(64) void k_edge_first_q(EdgeGroups gr, EnvDev env, 
         const float* qa = q1 + (int64_t)e * row_stride;
         const float* qd = dir + (int64_t)e * row_stride;
         const float sk = step * (float)k;
-        auto sc = [&](int j, double* st, double* ct) {
-            const float qv = qa[j] + sk * qd[j];
-            sincos((double)qv, st, ct);
-        };
+        // the joint values up to the last skeleton point, at the end of the
+        // skeletons' LDS, so that the rows' loads are in flight together: the
+        // kinematics take joint j no later than they write skeleton point
+        // j - 1, whose place lies before it (point i ends at row 3 i + 2, and
+        // at most L - i joints are left then, from row 3 (L + 1) - (L - i) on)
+        const int last = rb.pts[rb.num_links].frame;
+        const int nq = last < 0 ? 0 : rb.seg[last].joint + rb.seg[last].rev;
+        float* qv = skel + (3 * (rb.num_links + 1) - nq) * 64 + lane;
+#pragma unroll 4
+        for (int j = 0; j < nq; ++j) qv[j * 64] = qa[j] + sk * qd[j];
+        auto sc = [&](int j, double* st, double* ct) { sincos((double)qv[j * 64], st, ct); };
         const bool pairs = rb.num_pairs > 0;
         FKStream fk;
         fk_init(fk);
@@ -346,7 +400,7 @@ __global__ __launch_bounds__(64) void k_edge_first_q(EdgeGroups gr, EnvDev env, 
                                   i < rb.ground_included, p, !done);
             } else {
                 ConstPtr<SlabEntry> tab = as_const(gr.slab) + (size_t)keys[i] * (G + M);
-                h = link_hits(P0, P1, rb.radius[i], rb.rnew32[i], tab, G, M, as_const(env.aabb), p, !done);
+                h = link_hits(P0, P1, rb.radius[i], rb.rnew32[i], tab, G, M, env.aabb, p, !done);
             }
             if (h) {
                 bad = true;
@@ -360,34 +414,47 @@ __global__ __launch_bounds__(64) void k_edge_first_q(EdgeGroups gr, EnvDev env, 
             if (!done && __atomic_load_n(&first[e], __ATOMIC_RELAXED) <= k) done = true;
             P0 = P1;
         }
-        const bool bound_ok = csum == csum;
-        for (int m = 0; m < rb.num_pairs; ++m) {
+        if (!(csum == csum)) cmax = NAN;
+        // self pairs, run by run, kSelfBatch at a time: the wave tests the
+        // bounding boxes (apart_bound2 with a distance of 0), and the pairs that
+        // do not settle every lane take the full test
+        auto pt = [&](int kk) {
+            return Vec3<float>{skel[(3 * kk) * 64 + lane], skel[(3 * kk + 1) * 64 + lane],
+                               skel[(3 * kk + 2) * 64 + lane]};
+        };
+        for (int m = 0; m < rb.num_runs; ++m) {
             if (!__any(!done)) break;
-            const int a = rb.pairs[2 * m], b = rb.pairs[2 * m + 1];
-            const float ra = rb.radius[a], rbb = rb.radius[b];
-            auto pt = [&](int kk) {
-                return Vec3<float>{skel[(3 * kk) * 64 + lane], skel[(3 * kk + 1) * 64 + lane],
-                                   skel[(3 * kk + 2) * 64 + lane]};
-            };
-            const Vec3<float> A = pt(a), B = pt(a + 1), C = pt(b), D = pt(b + 1);
-            // distance of the two bounding boxes, squared (self_pair_hits's
-            // bound, written out here: the whole wave tests it, and only the
-            // lanes that it does not settle take the full test)
-            const float gx = fmaxf(fmaxf(fminf(C.x, D.x) - fmaxf(A.x, B.x), fminf(A.x, B.x) - fmaxf(C.x, D.x)), 0.0f);
-            const float gy = fmaxf(fmaxf(fminf(C.y, D.y) - fmaxf(A.y, B.y), fminf(A.y, B.y) - fmaxf(C.y, D.y)), 0.0f);
-            const float gz = fmaxf(fmaxf(fminf(C.z, D.z) - fmaxf(A.z, B.z), fminf(A.z, B.z) - fmaxf(C.z, D.z)), 0.0f);
-            const float R = fmaxf(ra + rbb, p.eq);
-            const float thr = R + 4e-6f * (cmax + R);
-            const bool apart = bound_ok && thr <= p.maxd && (gx * gx + gy * gy) + gz * gz > thr * thr;
-            if (!done && !apart) {
-                const float sd = seg_seg<float, false>(A, B, C, D, p, nullptr);
-                if (sd - ra - rbb < 0) {
-                    bad = true;
-                    done = true;
-                    atomicMin(&first[e], k);
+            const PairRun run = rb.runs[m];
+            const Vec3<float> A = pt(run.a), B = pt(run.a + 1);
+            const SegBox box(A, B);
+            const float ra = rb.radius[run.a];
+            const float bound2 = apart_bound2(run.rsum, 0.0f, cmax, p);
+            Vec3<float> C0 = pt(run.b);
+            for (int k0 = 0; k0 < run.count; k0 += kSelfBatch) {
+                Vec3<float> D[kSelfBatch];
+#pragma unroll
+                for (int k2 = 0; k2 < kSelfBatch; ++k2) D[k2] = pt(run.b + min(k0 + k2, run.count - 1) + 1);
+                uint32_t mine = 0;   // this lane's pairs of the batch
+#pragma unroll
+                for (int k2 = 0; k2 < kSelfBatch; ++k2)
+                    mine |= (k0 + k2 < run.count &&
+                             !(boxes_gap2(box, SegBox(k2 ? D[k2 - 1] : C0, D[k2])) > bound2)) ? 1u << k2 : 0u;
+                C0 = D[kSelfBatch - 1];
+#pragma clang loop unroll(disable)
+                while (__any(!done && mine)) {
+                    if (!done && mine) {
+                        const int b = run.b + k0 + __builtin_ctz(mine);
+                        mine &= mine - 1;
+                        const float sd = seg_seg<float, false>(A, B, pt(b), pt(b + 1), p, nullptr);
+                        if (sd - ra - rb.radius[b] < 0) {
+                            bad = true;
+                            done = true;
+                            atomicMin(&first[e], k);
+                        }
+                    }
                 }
             }
-            if ((m & 15) == 15 && !done && __atomic_load_n(&first[e], __ATOMIC_RELAXED) <= k) done = true;
+            if (!done && __atomic_load_n(&first[e], __ATOMIC_RELAXED) <= k) done = true;
         }
     }
 }
@@ -395,9 +462,9 @@ __global__ __launch_bounds__(64) void k_edge_first_q(EdgeGroups gr, EnvDev env, 
 // isValid(q1, q2): one lane per (edge, state), the collision tree through
 // the axis-test tables (axis-aligned scenes) or every oriented box in its
 // frame (OBB), as in k_edge_first_q (uniform loops per wave, joint values
-// computed where the kinematics reads them), no LDS.
+// in LDS).
 template <bool OBB>
-__global__ __launch_bounds__(256) void k_edge_valid_q(RobotDev rb, EnvDev env, QueryParams qp,
+__global__ __launch_bounds__(64) void k_edge_valid_q(RobotDev rb, EnvDev env, QueryParams qp,
                                                          const float* __restrict__ q1, const float* __restrict__ q2,
                                                          int64_t n, uint8_t* __restrict__ valid,
                                                          const int32_t* __restrict__ link_key,
@@ -415,10 +482,12 @@ __global__ __launch_bounds__(256) void k_edge_valid_q(RobotDev rb, EnvDev env, Q
     // step = k / num_checks * dist
     const float step = (float)kk / (float)K * dist;
     const float f = dist > 0 ? step / dist : 0.0f;
-    auto sc = [&](int j, double* st, double* ct) {
-        const float qv = dist > 0 ? a[j] + (b[j] - a[j]) * f : b[j];
-        sincos((double)qv, st, ct);
-    };
+    // the joint values first, so that the rows' loads are in flight together
+    extern __shared__ __align__(16) unsigned char smem[];
+    float* qv = reinterpret_cast<float*>(smem) + threadIdx.x;   // [D] at stride 64
+#pragma unroll 4
+    for (int j = 0; j < D; ++j) qv[j * 64] = dist > 0 ? a[j] + (b[j] - a[j]) * f : b[j];
+    auto sc = [&](int j, double* st, double* ct) { sincos((double)qv[j * 64], st, ct); };
     const int M = env.num_obj, G = (M + kSlabGroup - 1) / kSlabGroup;
     const Params<float> p{qp.eq, qp.maxd};
     FKStream fk;
@@ -434,7 +503,7 @@ __global__ __launch_bounds__(256) void k_edge_valid_q(RobotDev rb, EnvDev env, Q
                               i < rb.ground_included, p, !done);
         } else {
             ConstPtr<SlabEntry> tab = as_const(slab) + (size_t)as_const(link_key)[i] * (G + M);
-            h = link_hits(P0, P1, rb.radius[i], rb.rnew32[i], tab, G, M, as_const(env.aabb), p, !done);
+            h = link_hits(P0, P1, rb.radius[i], rb.rnew32[i], tab, G, M, env.aabb, p, !done);
         }
         if (h) {
             valid[e] = 0;
@@ -458,10 +527,10 @@ hipError_t launch_edge_valid(const RobotDev& rb, const EnvDev& env, const QueryP
         if (nkeys > 0 && G > 0)
             hipLaunchKernelGGL(k_slab_build, dim3((unsigned)((G + 63) / 64), (unsigned)nkeys), dim3(64), 0, st, env,
                                keys, nkeys, slab);
-        hipLaunchKernelGGL(k_edge_valid_q<false>, blocks_for(n * qp.num_checks, 256), dim3(256), 0, st, rb, env, qp,
+        hipLaunchKernelGGL(k_edge_valid_q<false>, blocks_for(n * qp.num_checks, 64), dim3(64), (size_t)256 * rb.num_dofs, st, rb, env, qp,
                            q1, q2, n, valid, link_key, slab);
     } else {
-        hipLaunchKernelGGL(k_edge_valid_q<true>, blocks_for(n * qp.num_checks, 256), dim3(256), 0, st, rb, env, qp,
+        hipLaunchKernelGGL(k_edge_valid_q<true>, blocks_for(n * qp.num_checks, 64), dim3(64), (size_t)256 * rb.num_dofs, st, rb, env, qp,
                            q1, q2, n, valid, link_key, slab);
     }
     return hipGetLastError();
