@@ -117,7 +117,7 @@ struct rvs_context {
     // run one wave per configuration (latency) instead of one lane
     int64_t wave_max = 16384;
     int32_t edge_waves_per_cu = 16;   // persistent first-collision kernel: resident waves per CU
-    int32_t edge_spl = 1;             // ... and slots per lane in one 64-lane item
+    int32_t edge_spl = 0;             // ... and slots per lane in one 64-lane item (0: by the slots of the call)
     std::map<std::pair<int32_t, int32_t>, rvs::FastTuning> tuning;   // (robot, env) -> autotuned launch shape
     // captured FP32 + refinement pipelines of device-array rvs_distance calls
     struct Graph {

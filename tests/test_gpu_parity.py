@@ -1110,3 +1110,32 @@ def test_trajectory_is_safe_sizes(oracle, engine, dofs, boxes, points, traj, sel
     osafe = oracle.traj_safe(rb, osc, pts, root, p0[0], np0[0], mv, 0.1, dt,
                              pairs=rb.self_pairs if self_collision else None)
     assert np.array_equal(safe, osafe)
+
+
+@pytest.mark.parametrize("boxes", [1, 8, 9, 63, 64, 65, 130])
+@pytest.mark.parametrize("dofs", [1, 6, 22])
+def test_edge_first_collision_obstacle_marks(oracle, engine, boxes, dofs):
+    """Obstacle counts at the edges of the table's batches, groups and 64-bit
+    marks, robots of one joint to 22 with self pairs, ground boxes skipped by
+    the first links, NaN rows, ragged waves: first indices and edge validity
+    equal to the oracle's."""
+    rng = np.random.default_rng(10 * boxes + dofs)
+    rb = R.xarm6(ground_included=2) if dofs == 6 else R.chain(rng.uniform(0.1, 0.4, dofs), radius=0.03,
+                                                              ground_included=min(2, dofs), self_collision=dofs > 1)
+    sc = W._boxes(rng, boxes, 0.05, 0.3, 1.5)
+    gnd = (rng.random(boxes) < 0.2).astype(np.uint8)
+    sc = W.Scene(sc.dim, sc.pos * np.where(np.linalg.norm(sc.pos[:, :2], axis=1) < 0.4, 3.0, 1.0)[:, None], sc.quat,
+                 gnd, sc.min_dist_tol)
+    osc = oracle.scene_of(sc)
+    n = 67
+    q1 = rng.uniform(-0.5, 0.5, (n, dofs)).astype(np.float32)
+    u = rng.normal(size=(n, dofs))
+    u = (u / np.linalg.norm(u, axis=1, keepdims=True)).astype(np.float32)
+    K = rng.integers(0, 40, n).astype(np.int32)
+    q1[5, dofs - 1] = np.nan
+    rid, eid = engine.load_robot(rb), engine.create_env(sc)
+    got = engine.edge_first_collision(eid, np.full(n, rid, np.int32), q1, u, K)
+    want = oracle.edge_first_collision(rb, osc, q1, u, K, 0.05)
+    assert np.array_equal(got, want)
+    q2 = (q1 + 0.3 * u).astype(np.float32)
+    assert np.array_equal(engine.edge_is_valid(rid, eid, q1, q2), oracle.edge_valid(rb, osc, q1, q2))
