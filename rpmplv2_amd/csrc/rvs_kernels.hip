@@ -322,8 +322,14 @@ __global__ __launch_bounds__(kBlock) void k_distance64(RobotDev rb, EnvDev env, 
 
 // ---------------------------------------------------------------- isValid
 // RealVectorSpace::isValid(q) (RealVectorSpace.cpp:277-309): collision tree
-// per pair, ground skipped for the first ground_included links, stop on the
-// first hit.
+// per pair, ground skipped for the first ground_included links, free when no
+// pair collides.  Per link the wave runs over the obstacles together, each lane
+// marking those that the tree's rejecting test (both end points beyond one
+// face of the box grown by the radius, collision_box) leaves; then every lane
+// takes its own marked obstacles to the full test.  The test as a chain of
+// branches, taken where the wave's walk met a pair, spent as many scalar
+// instructions on masks as vector ones on arithmetic (1,000,003 xArm6
+// configurations, 17 boxes: 200 us so, 165 us with the marks).
 template <typename T, bool OBB>
 __global__ __launch_bounds__(kBlock) void k_valid(RobotDev rb, EnvDev env, QueryParams qp,
                                                   const float* __restrict__ q, int64_t n, uint8_t* valid,
@@ -341,20 +347,45 @@ __global__ __launch_bounds__(kBlock) void k_valid(RobotDev rb, EnvDev env, Query
     fk_init(fk);
     Vec3<T> P0 = skel_point<T>(fk, rb, qc, 0);
     bool ok = true;
-    for (int i = 0; i < L && ok; ++i) {
+    for (int i = 0; i < L; ++i) {
+        if (!__any(ok)) break;
         const Vec3<T> P1 = skel_point<T>(fk, rb, qc, i + 1);
         const T r = (T)rb.radius[i];
         const T rn = rnew_of<T>(rb, i);
-        for (int j = 0; j < M; ++j) {
-            if (s.gnd[j] && i < rb.ground_included) continue;
-            bool col;
-            if (OBB) {
-                const float* x = s.xf + 12 * j;
-                col = collision_box(to_box(x, P0), to_box(x, P1), r, rn, s.box[j], p);
-            } else {
-                col = collision_box(P0, P1, r, rn, s.box[j], p);
+        const bool gnd_skip = i < rb.ground_included;
+        const T sum = ((P0.x + P0.y) + (P0.z + P1.x)) + (P1.y + P1.z);
+        const bool exact = !(sum - sum == T(0));   // a non-finite coordinate: every obstacle to the full test
+        for (int j0 = 0; j0 < M; j0 += 32) {
+            uint32_t mark = 0;
+            const int cnt = min(32, M - j0);
+#pragma unroll 4
+            for (int k = 0; k < cnt; ++k) {
+                const int j = j0 + k;
+                const Box<T> b = s.box[j];
+                Vec3<T> A = P0, B = P1;
+                if (OBB) {
+                    A = to_box(s.xf + 12 * j, P0);
+                    B = to_box(s.xf + 12 * j, P1);
+                }
+                const bool apart = (fmax(A.x, B.x) < b.lo[0] - r) | (fmin(A.x, B.x) > b.hi[0] + r) |
+                                   (fmax(A.y, B.y) < b.lo[1] - r) | (fmin(A.y, B.y) > b.hi[1] + r) |
+                                   (fmax(A.z, B.z) < b.lo[2] - r) | (fmin(A.z, B.z) > b.hi[2] + r);
+                const bool skip = gnd_skip && s.gnd[j];
+                mark |= (!skip & (exact | !apart)) ? 1u << k : 0u;
             }
-            if (col) { ok = false; break; }
+#pragma clang loop unroll(disable)
+            while (__any(ok && mark)) {
+                if (ok && mark) {
+                    const int j = j0 + __builtin_ctz(mark);
+                    mark &= mark - 1;
+                    if (OBB) {
+                        const float* x = s.xf + 12 * j;
+                        ok = !collision_box(to_box(x, P0), to_box(x, P1), r, rn, s.box[j], p);
+                    } else {
+                        ok = !collision_box(P0, P1, r, rn, s.box[j], p);
+                    }
+                }
+            }
         }
         P0 = P1;
     }

@@ -1139,3 +1139,26 @@ def test_edge_first_collision_obstacle_marks(oracle, engine, boxes, dofs):
     assert np.array_equal(got, want)
     q2 = (q1 + 0.3 * u).astype(np.float32)
     assert np.array_equal(engine.edge_is_valid(rid, eid, q1, q2), oracle.edge_valid(rb, osc, q1, q2))
+
+
+@pytest.mark.parametrize("oriented", [False, True])
+@pytest.mark.parametrize("dofs,boxes,n", [(2, 0, 3), (6, 1, 65), (6, 31, 300), (10, 32, 257), (10, 33, 64), (22, 64, 90),
+                                          (6, 100, 513)])
+def test_is_valid_obstacle_marks(oracle, engine, dofs, boxes, n, oriented):
+    """Obstacle counts at the edges of the 32-bit marks and their remainders,
+    both precisions, ground boxes skipped by the first links, ragged waves,
+    NaN and infinite joints: flags equal to the oracle's."""
+    rng = np.random.default_rng(3 * boxes + dofs)
+    rb = {2: R.planar_2dof, 6: lambda: R.xarm6(ground_included=2)}.get(
+        dofs, lambda: R.chain(rng.uniform(0.1, 0.2, dofs), radius=0.03, ground_included=1))()
+    sc = W._boxes(rng, boxes, 0.05, 0.25, 1.5, rotated=oriented)
+    sc = W.Scene(sc.dim, sc.pos * np.where(np.linalg.norm(sc.pos[:, :2], axis=1) < 0.3, 3.0, 1.0)[:, None], sc.quat,
+                 (rng.random(boxes) < 0.2).astype(np.uint8), sc.min_dist_tol)
+    q = rng.uniform(-np.pi, np.pi, (n, rb.num_dofs)).astype(np.float32)
+    q[n // 2, 0] = np.nan
+    q[n - 1, 1] = np.inf
+    rid = engine.load_robot(rb)
+    eid = engine.create_env(sc, rvs.ENV_OBB if oriented else rvs.ENV_AABB)
+    osc = oracle.scene_of(sc, oriented=oriented)
+    assert np.array_equal(engine.is_valid(rid, eid, q), oracle.is_valid(rb, osc, q))
+    assert np.array_equal(engine.is_valid(rid, eid, q, precision=rvs.PREC_FP64), oracle.is_valid(rb, osc, q, 64))
