@@ -735,7 +735,7 @@ hipError_t fp32_graph_run(rvs_context* c, int32_t robot, int32_t env, const Robo
         // clear without it), and the refinement stores the flagged count in
         // the mapped host word: no copy node
         const int32_t* perm = nullptr;
-        hipError_t le = launch_coherence_order(rb, q, n, ft, coh, &perm, c->stream, rcount, 64);
+        hipError_t le = launch_coherence_order(rb, q, n, ft.coh_bits, coh, &perm, c->stream, rcount, 64);
         if (le == hipSuccess && !perm) le = launch_zero_u32(rcount, 64, c->stream);
         if (le == hipSuccess)
             le = launch_distance_fast(rb, ev, qp, q, n, out, ridx, rcount, ft, perm, links, c->num_cus, c->stream);
@@ -788,7 +788,7 @@ rvs_status rvs_distance(rvs_context* c, int32_t robot, int32_t env, const float*
     const bool sort_exact = prec != RVS_PREC_FP32_REFINE && n >= kExactSortMin && n <= INT32_MAX &&
                             (prec == RVS_PREC_FP64 || n > c->wave_max);
     const size_t coh_need = (prec == RVS_PREC_FP32_REFINE || sort_exact) ? coh_bytes(n, D) : 0;
-    FastTuning ft = c->tuning_for(robot, env, L, M, n);
+    FastTuning ft = c->tuning_for(robot, env, D, L, M, n);
     size_t links_need = (prec == RVS_PREC_FP32_REFINE && ft.variant == 4) ? fast_links_bytes(n) : 0;
     // a link-major shape that nobody recorded gives way to lane refill (the
     // same results) when its lists cannot be had
@@ -844,7 +844,7 @@ rvs_status rvs_distance(rvs_context* c, int32_t robot, int32_t env, const float*
             e = launch_zero_u32(rcount, 64, c->stream);
             const int32_t* perm = nullptr;
             if (e == hipSuccess && timing) e = hipEventRecord(c->ev[3], c->stream);
-            if (e == hipSuccess) e = launch_coherence_order(rb.dev, qd, n, ft, coh, &perm, c->stream);
+            if (e == hipSuccess) e = launch_coherence_order(rb.dev, qd, n, ft.coh_bits, coh, &perm, c->stream);
             if (e == hipSuccess && timing) e = hipEventRecord(c->ev[0], c->stream);
             if (e == hipSuccess)
                 e = launch_distance_fast(rb.dev, ev.dev, qp, qd, n, out, ridx, rcount, ft, perm, links, c->num_cus,
@@ -857,7 +857,7 @@ rvs_status rvs_distance(rvs_context* c, int32_t robot, int32_t env, const float*
             if (e == hipSuccess && timing) e = hipEventRecord(c->ev[0], c->stream);
             const int32_t* perm = nullptr;
             if (e == hipSuccess && sort_exact)
-                e = launch_coherence_order(rb.dev, qd, n, c->tuning_for(robot, env, L, M, n), coh, &perm, c->stream);
+                e = launch_coherence_order(rb.dev, qd, n, c->order_bits(robot, env), coh, &perm, c->stream);
             if (e == hipSuccess)
                 e = (prec == RVS_PREC_FP64)
                         ? launch_distance_fp64(rb.dev, ev.dev, qp, qd, n, out, c->stream, perm)
@@ -908,8 +908,8 @@ namespace {
 // Walk order for a large exact-path batch of an async call (nullptr below
 // kExactSortMin): the sort's scratch comes from the arena, which async calls
 // use one after another (async_begin orders each after the previous one).
-hipError_t async_exact_order(rvs_context* c, int32_t robot, int32_t env, const RobotRec& rb, const EnvRec& ev,
-                             const float* q, int64_t n, hipStream_t st, const int32_t** perm) {
+hipError_t async_exact_order(rvs_context* c, int32_t robot, int32_t env, const RobotRec& rb, const float* q, int64_t n,
+                             hipStream_t st, const int32_t** perm) {
     *perm = nullptr;
     if (n < kExactSortMin || n > INT32_MAX) return hipSuccess;
     const size_t need = Carve::need({coh_bytes(n, rb.num_dofs)});
@@ -918,8 +918,7 @@ hipError_t async_exact_order(rvs_context* c, int32_t robot, int32_t env, const R
     if (e != hipSuccess) return e;
     Carve cv(c->arena.p);
     uint32_t* coh = cv.take<uint32_t>(coh_bytes(n, rb.num_dofs) / 4);
-    return launch_coherence_order(rb.dev, q, n, c->tuning_for(robot, env, rb.num_links, ev.dev.num_obj, n), coh, perm,
-                                  st);
+    return launch_coherence_order(rb.dev, q, n, c->order_bits(robot, env), coh, perm, st);
 }
 
 }  // namespace
@@ -946,7 +945,7 @@ rvs_status rvs_distance_async(rvs_context* c, int32_t robot, int32_t env, const 
     hipError_t e = async_begin(c, st);
     if (e == hipSuccess && n > 0) {
         if (prec == RVS_PREC_FP32_REFINE) {
-            FastTuning ft = c->tuning_for(robot, env, L, M, n);
+            FastTuning ft = c->tuning_for(robot, env, D, L, M, n);
             size_t links_need = ft.variant == 4 ? fast_links_bytes(n) : 0;
             const size_t need = Carve::need({(size_t)n * 4 + 256, coh_bytes(n, D), links_need});
             if (need > c->arena.cap) c->drain_async();   // growing frees the block earlier calls use
@@ -966,14 +965,14 @@ rvs_status rvs_distance_async(rvs_context* c, int32_t robot, int32_t env, const 
             uint32_t* links = links_need ? cv.take<uint32_t>(links_need / 4) : nullptr;
             const int32_t* perm = nullptr;
             e = launch_zero_u32(rcount, 64, st);
-            if (e == hipSuccess) e = launch_coherence_order(rb.dev, q, n, ft, coh, &perm, st);
+            if (e == hipSuccess) e = launch_coherence_order(rb.dev, q, n, ft.coh_bits, coh, &perm, st);
             if (e == hipSuccess)
                 e = launch_distance_fast(rb.dev, ev.dev, qp, q, n, out, ridx, rcount, ft, perm, links, c->num_cus,
                                          st);
             if (e == hipSuccess) e = launch_distance_refine(rb.dev, ev.dev, qp, q, n, out, ridx, rcount, st);
         } else {
             const int32_t* perm = nullptr;
-            if (prec == RVS_PREC_FP64 || n > c->wave_max) e = async_exact_order(c, robot, env, rb, ev, q, n, st, &perm);
+            if (prec == RVS_PREC_FP64 || n > c->wave_max) e = async_exact_order(c, robot, env, rb, q, n, st, &perm);
             if (e == hipSuccess)
                 e = prec == RVS_PREC_FP64 ? launch_distance_fp64(rb.dev, ev.dev, qp, q, n, out, st, perm)
                                           : launch_distance_ref32_auto(rb.dev, ev.dev, qp, q, n, out, c->wave_max, st,
@@ -1015,7 +1014,7 @@ rvs_status rvs_distance_async_static(rvs_context* c, int32_t robot, int32_t env,
     const QueryParams qp = params_of(c);
     DistOut out{};
     out.d = d; out.profile = profile; out.verdict = verdict;
-    const FastTuning ft = c->tuning_for(robot, env, L, M, n);
+    const FastTuning ft = c->tuning_for(robot, env, D, L, M, n);
     hipError_t e = async_begin(c, st);
     if (e == hipSuccess && n > 0) {
         Carve cv(base);
@@ -1026,14 +1025,14 @@ rvs_status rvs_distance_async_static(rvs_context* c, int32_t robot, int32_t env,
         if (refine) {
             // counters cleared by a kernel: the scratch keeps the last call's contents
             e = launch_zero_u32(rcount, 64, st);
-            if (e == hipSuccess) e = launch_coherence_order(rb.dev, q, n, ft, coh, &perm, st);
+            if (e == hipSuccess) e = launch_coherence_order(rb.dev, q, n, ft.coh_bits, coh, &perm, st);
             // no links scratch in the static array: a link-major shape runs as variant 3
             if (e == hipSuccess)
                 e = launch_distance_fast(rb.dev, ev.dev, qp, q, n, out, ridx, rcount, ft, perm, nullptr, c->num_cus,
                                          st);
             if (e == hipSuccess) e = launch_distance_refine(rb.dev, ev.dev, qp, q, n, out, ridx, rcount, st);
         } else {
-            if (sort) e = launch_coherence_order(rb.dev, q, n, ft, coh, &perm, st);
+            if (sort) e = launch_coherence_order(rb.dev, q, n, c->order_bits(robot, env), coh, &perm, st);
             if (e == hipSuccess)
                 e = prec == RVS_PREC_FP64 ? launch_distance_fp64(rb.dev, ev.dev, qp, q, n, out, st, perm)
                                           : launch_distance_ref32_auto(rb.dev, ev.dev, qp, q, n, out, c->wave_max, st,
@@ -1061,7 +1060,8 @@ rvs_status rvs_is_valid_async(rvs_context* c, int32_t robot, int32_t env, const 
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c->stream;
     hipError_t e = async_begin(c, st);
     const int32_t* perm = nullptr;
-    if (e == hipSuccess && n > 0) e = async_exact_order(c, robot, env, rb, ev, q, n, st, &perm);
+    if (e == hipSuccess && n > 0 && c->order_valid(robot, env, n))
+        e = async_exact_order(c, robot, env, rb, q, n, st, &perm);
     if (e == hipSuccess && n > 0) e = launch_is_valid(rb.dev, ev.dev, params_of(c), q, n, valid, fp64, st, perm);
     if (e == hipSuccess) e = async_end(c, st, done);
     if (e != hipSuccess) return hip_fail(c, e, "rvs_is_valid_async");
@@ -1173,7 +1173,7 @@ rvs_status rvs_autotune(rvs_context* c, int32_t robot, int32_t env, const float*
             e = launch_zero_u32(count, 64, c->stream);
             const int32_t* perm = nullptr;
             if (e == hipSuccess) e = hipEventRecord(c->ev[0], c->stream);
-            if (e == hipSuccess) e = launch_coherence_order(rb.dev, qs, m, t, coh, &perm, c->stream);
+            if (e == hipSuccess) e = launch_coherence_order(rb.dev, qs, m, t.coh_bits, coh, &perm, c->stream);
             if (e == hipSuccess)
                 e = launch_distance_fast(rb.dev, ev.dev, qp, qs, m, out, idx, count, t, perm, links, c->num_cus,
                                          c->stream);
@@ -1236,7 +1236,7 @@ rvs_status rvs_get_tuning(rvs_context* c, int32_t robot, int32_t env, rvs_tuning
         if (robot_ok(c, robot)) L = c->robots[robot].num_links;
         if (env_ok(c, env)) M = c->envs[env].dev.num_obj;
     }
-    const FastTuning f = c->tuning_for(robot, env, L, M, 0);
+    const FastTuning f = c->tuning_for(robot, env, 0, L, M, 0);
     *t = rvs_tuning{f.variant, f.block, f.blocks_per_cu, f.coh_bits, 0.0f};
     return RVS_OK;
 }
@@ -1284,7 +1284,7 @@ rvs_status rvs_distance_f64(rvs_context* c, int32_t robot, int32_t env, const fl
     }
     const int32_t* perm = nullptr;
     if (e == hipSuccess && coh)
-        e = launch_coherence_order(rb.dev, qd, n, c->tuning_for(robot, env, L, ev.dev.num_obj, n), coh, &perm, c->stream);
+        e = launch_coherence_order(rb.dev, qd, n, c->order_bits(robot, env), coh, &perm, c->stream);
     if (e == hipSuccess) e = launch_distance_fp64(rb.dev, ev.dev, qp, qd, n, out, c->stream, perm);
     if (e == hipSuccess && !(flags & RVS_F_DEVICE)) {
         e = d2h(d, out.d64, (size_t)n * 8, c->stream);
@@ -1315,7 +1315,7 @@ rvs_status rvs_is_valid(rvs_context* c, int32_t robot, int32_t env, const float*
     const float* qd = q;
     uint8_t* vd = valid;
     // large batches run in the walk order (as rvs_distance's exact paths)
-    const size_t coh_need = (n >= kExactSortMin && n <= INT32_MAX) ? coh_bytes(n, D) : 0;
+    const size_t coh_need = c->order_valid(robot, env, n) ? coh_bytes(n, D) : 0;
     uint32_t* coh = nullptr;
     if (!(flags & RVS_F_DEVICE)) {
         e = c->arena.ensure(Carve::need({coh_need, (size_t)n * D * 4, (size_t)n}));
@@ -1336,8 +1336,7 @@ rvs_status rvs_is_valid(rvs_context* c, int32_t robot, int32_t env, const float*
     const bool timing = (flags & RVS_F_TIMING) != 0;
     if (e == hipSuccess && timing) e = hipEventRecord(c->ev[0], c->stream);
     if (e == hipSuccess && coh)
-        e = launch_coherence_order(rb.dev, qd, n, c->tuning_for(robot, env, rb.num_links, ev.dev.num_obj, n), coh, &perm,
-                                   c->stream);
+        e = launch_coherence_order(rb.dev, qd, n, c->order_bits(robot, env), coh, &perm, c->stream);
     if (e == hipSuccess && timing) e = hipEventRecord(c->ev[1], c->stream);
     if (e == hipSuccess) e = launch_is_valid(rb.dev, ev.dev, qp, qd, n, vd, fp64, c->stream, perm);
     if (e == hipSuccess && timing) e = hipEventRecord(c->ev[2], c->stream);

@@ -136,13 +136,24 @@ struct rvs_context {
     // The launch shape of an RVS_PREC_FP32_REFINE batch of n configurations:
     // the recorded one, else by the length of the walk and the batch (every
     // shape gives the same bits, so the choice may follow n).
-    rvs::FastTuning tuning_for(int32_t robot, int32_t env, int32_t links, int32_t objects, int64_t n) {
+    rvs::FastTuning tuning_for(int32_t robot, int32_t env, int32_t dofs, int32_t links, int32_t objects, int64_t n) {
         std::lock_guard<std::mutex> lk(tuning_mu);
         auto it = tuning.find({robot, env});
         if (it != tuning.end()) return it->second;
         // one lane per configuration: 64-thread workgroups measured fastest
         if (fast_variant >= 0) return rvs::FastTuning{fast_variant, fast_variant == 0 ? 64 : 256, 0, 5};
-        if ((int64_t)links * objects < 1024) return rvs::FastTuning{0, 64, 0, 5};
+        if ((int64_t)links * objects < 1024) {
+            // The walk order's four kernels (16 to 31 us) pay for themselves
+            // in large batches: xArm6 and 17 boxes 266 against 322 us for
+            // 1,000,003 configurations, 148 against 146 for 262,147, 114
+            // against 104 for 5,909 (10-DOF chain 405 / 423, 209 / 178 and 140
+            // / 125).  Where they order the whole pose (at most 3 joints) they
+            // pay early, unless the walk is short: planar arm, 40 boxes 108
+            // against 164 us for 65,536; 4 boxes 130 against 102 for 1,000,003.
+            // (n <= 0: the shape of a large batch, for rvs_get_tuning)
+            const int64_t from = (int64_t)links * objects < 32 ? INT64_MAX : (dofs <= 3 ? 1024 : 1 << 18);
+            return rvs::FastTuning{0, 64, 0, n <= 0 || n >= from ? 5 : 0};
+        }
         // Long walks.  Link-major launches (4) against lane refill (1), 22-DOF
         // chain: 512 boxes 5.9 against 11.7 ms for 2,097,152 configurations and
         // 2.1 against 2.5 ms for 1,000; 256 boxes 3.5 against 5.0 ms for
@@ -157,6 +168,21 @@ struct rvs_context {
         // 18-DOF chain and 80 boxes 1.17 against 1.03 for 400,000.
         if (n > 0 && n <= (int64_t)1 << 17) return rvs::FastTuning{3, 512, 0, 5};
         return rvs::FastTuning{1, 256, 0, 5};
+    }
+    // Walk-order bits of the exact paths: a recorded shape's, else 5.
+    int32_t order_bits(int32_t robot, int32_t env) {
+        std::lock_guard<std::mutex> lk(tuning_mu);
+        auto it = tuning.find({robot, env});
+        return it != tuning.end() ? it->second.coh_bits : 5;
+    }
+    // Whether an isValid batch of n configurations runs in the walk order:
+    // 16 to 31 us of sorting against fewer branches.  xArm6 and 17 boxes, REF32
+    // (FP64): 204 against 235 us (246 / 318) for 1,000,003 configurations, 146
+    // against 142 (174 / 193) for 524,288, 105 against 88 (126 / 124) for
+    // 262,147; the planar arm among 4 boxes 80 against 59 us for 1,000,003.
+    bool order_valid(int32_t robot, int32_t env, int64_t n) const {
+        return n >= 1 << 19 && n <= INT32_MAX &&
+               (int64_t)robots[robot].num_links * envs[env].dev.num_obj >= 32;
     }
     // Whether the launch shape of (robot, env) was recorded by a caller.
     bool tuned(int32_t robot, int32_t env) {

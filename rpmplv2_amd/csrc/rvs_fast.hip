@@ -1417,10 +1417,10 @@ hipError_t launch_zero_u32(uint32_t* p, int n, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t launch_coherence_order(const RobotDev& rb, const float* q, int64_t n, const FastTuning& t, uint32_t* coh,
+hipError_t launch_coherence_order(const RobotDev& rb, const float* q, int64_t n, int32_t coh_bits, uint32_t* coh,
                                   const int32_t** perm, hipStream_t st, uint32_t* zero, int nzero) {
     *perm = nullptr;
-    const int bits = std::min<int>(t.coh_bits, kCohKeyBits);
+    const int bits = std::min<int>(coh_bits, kCohKeyBits);
     if (n <= 0 || !coh || bits <= 0 || rb.num_dofs <= 0) return hipSuccess;
     const int nj = std::min(rb.num_dofs, kCohKeyBits / bits);
     if (n > INT32_MAX) return hipErrorInvalidValue;

@@ -189,13 +189,13 @@ inline CohLayout coh_layout(uint32_t* base, int64_t n) {
     L.key_lo = reinterpret_cast<uint16_t*>(L.perm + coh_words(m));
     return L;
 }
-// The walk order of the bulk pass: with t.coh_bits > 0 and coh scratch the
+// The walk order of the bulk pass: with coh_bits > 0 and coh scratch the
 // configurations are bucketed by their first joint angles (so that the lanes
 // of a wave hold similar poses) and *perm points at the order in coh;
 // otherwise *perm is null (the order given).  When it runs, its first kernel
 // also clears zero[0, nzero) (zero may be null); with *perm null nothing
 // was cleared.
-hipError_t launch_coherence_order(const RobotDev& rb, const float* q, int64_t n, const FastTuning& t, uint32_t* coh,
+hipError_t launch_coherence_order(const RobotDev& rb, const float* q, int64_t n, int32_t coh_bits, uint32_t* coh,
                                   const int32_t** perm, hipStream_t st, uint32_t* zero = nullptr, int nzero = 0);
 // Scratch of the link-major bulk pass (tuning variant 4), 256-byte aligned:
 // two lists of the configurations alive at a link, used in turn, whose

@@ -288,7 +288,7 @@ hipError_t issue(rvs_server* s, Batch& b, const Layout& lay) {
         out.verdict = flag;
         const int prec = s->opt.precision;
         if (prec == RVS_PREC_FP32_REFINE) {
-            const FastTuning ft = s->ctx->tuning_for(h.r.robot, h.r.env, L, M, N);
+            const FastTuning ft = s->ctx->tuning_for(h.r.robot, h.r.env, D, L, M, N);
             if (e == hipSuccess) e = launch_zero_u32(count, 64, st);
             if (e == hipSuccess)
                 // order given; no links scratch (a link-major shape runs as variant 3)
