@@ -104,7 +104,7 @@ inline PairLds pair_lds(const RobotDev& rb, const EnvDev& env, bool want_np, int
 // 44 us, 16,384 60 us (one wave per configuration with every pair evaluated:
 // 30, 60 and 121 us; the serial kinematics alone took 13,000 of a wave's 39,000
 // cycles, now 6,000), one state with its nearest points 76 us from host arrays
-// (90 us with a link at a time).
+// (90 us with a link at a time); 64 lanes a configuration: launch_distance_pairs.
 template <bool OBB, bool WANT_NP, int G>
 __global__ __launch_bounds__(64) void k_distance_pairs(RobotDev rb, EnvDev env, QueryParams qp,
                                                        const float* __restrict__ q, DistOut out,
@@ -317,12 +317,21 @@ bool pairs_fit(const RobotDev& rb, const EnvDev& env) {
 hipError_t launch_distance_pairs(const RobotDev& rb, const EnvDev& env, const QueryParams& qp, const float* q,
                                  const DistOut& out, const int32_t* idx, const uint32_t* count, int64_t n,
                                  int64_t max_waves, hipStream_t st, uint32_t* count_out) {
-    if (env.use_obb)
-        return out.nearest ? launch_shape<true, true, 64>(rb, env, qp, q, out, idx, count, n, max_waves, count_out, st)
-                           : launch_shape<true, false, 16>(rb, env, qp, q, out, idx, count, n, max_waves, count_out,
-                                                           st);
-    return out.nearest ? launch_shape<false, true, 64>(rb, env, qp, q, out, idx, count, n, max_waves, count_out, st)
-                       : launch_shape<false, false, 16>(rb, env, qp, q, out, idx, count, n, max_waves, count_out, st);
+    // Lanes per configuration.  64 leave a shorter chain, 16 fill the waves
+    // better once there are more waves than the SIMDs hold side by side.  Of
+    // a batch in reference arithmetic, 64 against 16 lanes a call: xArm6 and
+    // 40 boxes 1,000 configurations 42 / 58 us, 4,096 50 / 67, 8,192 70 / 74,
+    // 16,384 103 / 102; 17 boxes 4,096 43 / 47 and 8,192 55 / 47; spatial10
+    // and 28 boxes 16,384 113 / 116, 40 boxes 134 / 151: 64 lanes up to 4,096
+    // configurations, and from 256 pairs a configuration on at any size.  A
+    // bulk pass lists about one configuration in 60 to 300: a whole call on
+    // spatial10 and 40 boxes, 65,536 190 / 208 us, 1,000,003 641 / 617;
+    // 4 boxes 65,536 90 / 89, 200,000 119 / 113: 64 lanes up to 131,072.
+    const bool wide = idx ? n <= 131072 : n <= 4096 || rb.num_links * env.num_obj >= 256;
+    auto run = [&](auto shape) { return shape(rb, env, qp, q, out, idx, count, n, max_waves, count_out, st); };
+    if (out.nearest) return env.use_obb ? run(launch_shape<true, true, 64>) : run(launch_shape<false, true, 64>);
+    if (wide) return env.use_obb ? run(launch_shape<true, false, 64>) : run(launch_shape<false, false, 64>);
+    return env.use_obb ? run(launch_shape<true, false, 16>) : run(launch_shape<false, false, 16>);
 }
 
 }  // namespace rvs

@@ -1015,9 +1015,10 @@ def test_small_batches_many_obstacles(oracle, engine, oriented):
 
 @pytest.mark.parametrize("oriented", [False, True])
 @pytest.mark.parametrize("dofs,boxes,n", [(2, 0, 5), (6, 1, 1), (6, 16, 3), (6, 170, 67), (10, 102, 18), (10, 103, 18),
-                                          (22, 46, 33), (40, 7, 9)])
+                                          (22, 46, 33), (40, 7, 9), (2, 1, 4097), (6, 16, 4099), (6, 40, 4101),
+                                          (40, 6, 4098), (10, 25, 4097)])
 def test_distances_by_pairs_sizes(engine, dofs, boxes, n, oriented):
-    """A few lanes per configuration against one lane, bit for bit, with and
+    """16 or 64 lanes per configuration against one lane, bit for bit, with and
     without nearest points: from no obstacle to the row's 1,024 pairs and past
     them (103 boxes of ten links: link by link), more segments than lanes,
     ragged waves, contacts with several boxes, links that skip ground boxes,
