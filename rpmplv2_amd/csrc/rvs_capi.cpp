@@ -42,6 +42,23 @@ rvs_status hip_fail(rvs_context* c, hipError_t e, const char* what) {
 
 // exact-path batches of at least this many configurations run in the walk order
 constexpr int64_t kExactSortMin = 65536;
+// Host arrays of a distance or trajectory call up to this many bytes, inputs
+// and outputs together, go through pinned host memory that the kernels address:
+// a copy of an array costs about 10 us however small it is, the link carries
+// 1 MiB in about 25 us.  xArm6 in reference arithmetic, pinned against copies:
+// one state and 4 boxes with nearest points 30 / 93 us, 4,096 configurations 61
+// / 98, 16,384 (0.9 MB) 99 / 180; 40 boxes with nearest points, 170
+// configurations (1 MB), about 140 / 180.  The block itself is 1 MiB at least.
+constexpr size_t kPinnedIo = 1024 * 1024;
+// The device's address of the context's pinned block of kPinnedIo bytes;
+// nullptr when there is none to be had.
+void* pinned_io(rvs_context* c) {
+    void* dev = nullptr;
+    if (c->staging.ensure(kPinnedIo) == hipSuccess && hipHostGetDevicePointer(&dev, c->staging.p, 0) == hipSuccess)
+        return dev;
+    (void)hipGetLastError();   // the call goes on with copies
+    return nullptr;
+}
 
 // Scratch of rvs_distance_async_static: the refinement list and counters and
 // the walk-order sort of one call of up to kStaticMaxConfigs configurations
@@ -803,7 +820,11 @@ rvs_status rvs_distance(rvs_context* c, int32_t robot, int32_t env, const float*
     uint32_t* rcount = nullptr;
     uint32_t* coh = nullptr;
     uint32_t* links = nullptr;
-    if (flags & RVS_F_DEVICE) {
+    // small host arrays stay in a pinned block that the kernels read and write
+    const size_t io = Carve::need({(size_t)n * D * 4, (size_t)n * 4, profile ? (size_t)n * L * 4 : 0,
+                                   nearest ? (size_t)n * M * L * 24 : 0, (size_t)n});
+    void* const pinned = (flags & RVS_F_DEVICE) || io > kPinnedIo ? nullptr : pinned_io(c);
+    if ((flags & RVS_F_DEVICE) || pinned) {
         e = c->arena.ensure(Carve::need({refine_bytes, coh_need, links_need}));
         if (e != hipSuccess && without_links()) e = c->arena.ensure(Carve::need({refine_bytes, coh_need}));
         if (e != hipSuccess) return hip_fail(c, e, "rvs_distance: staging");
@@ -812,6 +833,15 @@ rvs_status rvs_distance(rvs_context* c, int32_t robot, int32_t env, const float*
         if (coh_need) coh = cv.take<uint32_t>(coh_need / 4);
         if (links_need) links = cv.take<uint32_t>(links_need / 4);
         out.d = d; out.profile = profile; out.nearest = nearest; out.verdict = verdict;
+        if (pinned) {
+            Carve io_cv(pinned);
+            std::memcpy(c->staging.p, q, (size_t)n * D * 4);
+            qd = io_cv.take<float>((size_t)n * D);   // at the block's start
+            out.d = io_cv.take<float>(n);
+            out.profile = profile ? io_cv.take<float>((size_t)n * L) : nullptr;
+            out.nearest = nearest ? io_cv.take<float>((size_t)n * M * L * 6) : nullptr;
+            out.verdict = io_cv.take<uint8_t>(n);
+        }
     } else {
         auto need = [&]() {
             return Carve::need({refine_bytes, coh_need, links_need, (size_t)n * D * 4, (size_t)n * 4,
@@ -865,7 +895,7 @@ rvs_status rvs_distance(rvs_context* c, int32_t robot, int32_t env, const float*
             if (e == hipSuccess && timing) e = hipEventRecord(c->ev[1], c->stream);
         }
     }
-    if (e == hipSuccess && !(flags & RVS_F_DEVICE)) {
+    if (e == hipSuccess && !(flags & RVS_F_DEVICE) && !pinned) {
         e = d2h(d, out.d, (size_t)n * 4, c->stream);
         if (e == hipSuccess) e = d2h(profile, out.profile, (size_t)n * L * 4, c->stream);
         if (e == hipSuccess) e = d2h(nearest, out.nearest, (size_t)n * M * L * 24, c->stream);
@@ -873,6 +903,17 @@ rvs_status rvs_distance(rvs_context* c, int32_t robot, int32_t env, const float*
     }
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "rvs_distance");
+    if (pinned) {
+        auto take = [&](void* dst, const void* dev, size_t bytes) {
+            if (dst && dev)
+                std::memcpy(dst, static_cast<char*>(c->staging.p) +
+                                     (static_cast<const char*>(dev) - static_cast<char*>(pinned)), bytes);
+        };
+        take(d, out.d, (size_t)n * 4);
+        take(profile, out.profile, (size_t)n * L * 4);
+        take(nearest, out.nearest, (size_t)n * M * L * 24);
+        take(verdict, out.verdict, (size_t)n);
+    }
     c->last_refined = (prec == RVS_PREC_FP32_REFINE) ? (int64_t)refined : 0;
     if (timing) {
         c->nstages = prec == RVS_PREC_FP32_REFINE ? 3 : 2;
@@ -1498,32 +1539,47 @@ rvs_status rvs_trajectory_is_safe(rvs_context* c, int32_t robot, int32_t env, co
     a.time_step = time_step;
     a.self_collision = self_collision ? 1 : 0;
     a.safe = safe;
-    hipError_t e = hipSuccess;
-    if (!(flags & RVS_F_DEVICE)) {
-        e = c->arena.ensure(Carve::need({pb, (size_t)D * 4, (size_t)L * 4, set * 4, (size_t)M * 4, (size_t)num_traj}));
-        if (e != hipSuccess) return hip_fail(c, e, "rvs_trajectory_is_safe: staging");
-        Carve cv(c->arena.p);
-        float* ps = cv.take<float>(pb / 4);
-        float* qs = cv.take<float>(D);
-        float* prs = cv.take<float>(L);
-        float* ns = cv.take<float>(set);
-        float* vs = cv.take<float>(M);
-        a.safe = cv.take<uint8_t>(num_traj);
-        e = h2d(ps, points, pb, c->stream);
-        if (e == hipSuccess) e = h2d(qs, q_current, (size_t)D * 4, c->stream);
-        if (e == hipSuccess) e = h2d(prs, profile_current, (size_t)L * 4, c->stream);
-        if (e == hipSuccess) e = h2d(ns, nearest_current, set * 4, c->stream);
-        if (e == hipSuccess) e = h2d(vs, max_vel, (size_t)M * 4, c->stream);
-        a.points = ps;
-        a.q_current = qs;
-        a.profile_current = prs;
-        a.nearest_current = ns;
-        a.max_vel = vs;
+    if (flags & RVS_F_DEVICE) {
+        hipError_t e = launch_traj_safe(rb.dev, qp, a, num_traj, c->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        if (e != hipSuccess) return hip_fail(c, e, "rvs_trajectory_is_safe");
+        return RVS_OK;
     }
+    // the current state's arrays are small: through a pinned mirror, in one
+    // copy; the points straight from the caller.  A small call stays in the
+    // mirror with all it reads and writes.
+    const size_t state = Carve::need({(size_t)D * 4, (size_t)L * 4, set * 4, (size_t)M * 4});
+    const size_t io = state + Carve::need({pb, (size_t)num_traj});
+    void* const pinned = io <= kPinnedIo ? pinned_io(c) : nullptr;
+    hipError_t e = pinned ? hipSuccess : c->arena.ensure(io);
+    if (e == hipSuccess && !pinned) e = c->staging.ensure(state);
+    if (e != hipSuccess) return hip_fail(c, e, "rvs_trajectory_is_safe: staging");
+    char* const mirror = static_cast<char*>(c->staging.p);
+    Carve cv(pinned ? pinned : c->arena.p);
+    auto put = [&](size_t bytes, const float* src) {
+        float* const dev = cv.take<float>(bytes / 4);
+        if (bytes) std::memcpy(mirror + (reinterpret_cast<char*>(dev) - cv.base), src, bytes);
+        return dev;
+    };
+    a.q_current = put((size_t)D * 4, q_current);
+    a.profile_current = put((size_t)L * 4, profile_current);
+    a.nearest_current = put(set * 4, nearest_current);
+    a.max_vel = put((size_t)M * 4, max_vel);
+    float* ps = nullptr;
+    if (pinned) {
+        ps = put(pb, points);
+    } else {
+        e = h2d(cv.base, mirror, cv.off, c->stream);
+        ps = cv.take<float>(pb / 4);
+        if (e == hipSuccess) e = h2d(ps, points, pb, c->stream);
+    }
+    a.points = ps;
+    a.safe = cv.take<uint8_t>(num_traj);
     if (e == hipSuccess) e = launch_traj_safe(rb.dev, qp, a, num_traj, c->stream);
-    if (e == hipSuccess && !(flags & RVS_F_DEVICE)) e = d2h(safe, a.safe, (size_t)num_traj, c->stream);
+    if (e == hipSuccess && !pinned) e = d2h(safe, a.safe, (size_t)num_traj, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "rvs_trajectory_is_safe");
+    if (pinned) std::memcpy(safe, mirror + (reinterpret_cast<char*>(a.safe) - cv.base), (size_t)num_traj);
     return RVS_OK;
 }
 

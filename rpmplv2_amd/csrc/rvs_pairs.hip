@@ -103,8 +103,8 @@ inline PairLds pair_lds(const RobotDev& rb, const EnvDev& env, bool want_np, int
 // steps the better.  xArm6 and 17 boxes, a call: 1 configuration 24 us, 4,096
 // 44 us, 16,384 60 us (one wave per configuration with every pair evaluated:
 // 30, 60 and 121 us; the serial kinematics alone took 13,000 of a wave's 39,000
-// cycles, now 6,000), one state with its nearest points 76 us from host arrays
-// (90 us with a link at a time); 64 lanes a configuration: launch_distance_pairs.
+// cycles, now 6,000), one state with its nearest points 75 us from copied host
+// arrays (90 us with a link at a time) and 30 us in place; 64 lanes a configuration: launch_distance_pairs.
 template <bool OBB, bool WANT_NP, int G>
 __global__ __launch_bounds__(64) void k_distance_pairs(RobotDev rb, EnvDev env, QueryParams qp,
                                                        const float* __restrict__ q, DistOut out,

@@ -1163,3 +1163,50 @@ def test_is_valid_obstacle_marks(oracle, engine, dofs, boxes, n, oriented):
     osc = oracle.scene_of(sc, oriented=oriented)
     assert np.array_equal(engine.is_valid(rid, eid, q), oracle.is_valid(rb, osc, q))
     assert np.array_equal(engine.is_valid(rid, eid, q, precision=rvs.PREC_FP64), oracle.is_valid(rb, osc, q, 64))
+
+
+@pytest.mark.parametrize("n", [1, 17, 3639, 3640, 3700, 21500, 22700])
+def test_host_arrays_in_place_and_copied(engine, n):
+    """Host arrays up to 1 MiB are used in place, larger ones copied: both give
+    the device arrays' bits, on each side of the line with the nearest points
+    (288 bytes a configuration here) and without (about 46)."""
+    import torch
+
+    rng = np.random.default_rng(n)
+    rb = R.xarm6()
+    sc = W._boxes(rng, 2, 0.05, 0.3, 0.9)
+    q = rng.uniform(-np.pi, np.pi, (n, 6)).astype(np.float32)
+    rid, eid = engine.load_robot(rb), engine.create_env(sc, rvs.ENV_AABB)
+    qd = torch.from_numpy(q).cuda()
+    for prec in (rvs.PREC_REF32, rvs.PREC_FP32_REFINE):
+        dd, pd, vd = (torch.empty(n, device="cuda"), torch.empty((n, 6), device="cuda"),
+                      torch.empty(n, dtype=torch.uint8, device="cuda"))
+        engine.distance_device(rid, eid, qd, dd, pd, vd, precision=prec)
+        d, prof, ver, _ = engine.distance(rid, eid, q, precision=prec)
+        assert np.array_equal(d, dd.cpu().numpy()) and np.array_equal(prof, pd.cpu().numpy())
+        assert np.array_equal(ver, vd.cpu().numpy())
+    m = min(n, 4000)
+    _, _, _, near = engine.distance(rid, eid, q[:m], want_nearest=True)
+    parts = [engine.distance(rid, eid, q[k:k + 500], want_nearest=True)[3] for k in range(0, m, 500)]
+    assert np.array_equal(near, np.concatenate(parts), equal_nan=True)
+
+
+def test_trajectories_in_place_and_copied(engine):
+    """4,500 trajectories of 10 points (1.1 MB, copied) against the same in parts
+    that are used in place."""
+    rng = np.random.default_rng(5)
+    rb = R.xarm6()
+    sc = W._boxes(rng, 12, 0.05, 0.2, 0.9)
+    rid, eid = engine.load_robot(rb), engine.create_env(sc, rvs.ENV_AABB)
+    q = rng.uniform(-1, 1, 6).astype(np.float32)
+    _, prof, _, near = engine.distance(rid, eid, q[None], want_nearest=True)
+    pts = (q + np.cumsum(rng.normal(0, 0.01, (4500, 10, 6)), axis=1)).astype(np.float32)
+    vel = np.full(12, 0.1, np.float32)
+
+    def safe(p):
+        return engine.trajectory_is_safe(rid, eid, p, q, prof[0], near[0], vel, time_step=0.01)
+
+    whole = safe(pts)
+    print(f"safe {whole.mean():.3f}")
+    assert np.array_equal(whole, np.concatenate([safe(pts[k:k + 900]) for k in range(0, 4500, 900)]))
+    assert np.array_equal(whole[:1], safe(pts[:1]))
