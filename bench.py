@@ -85,10 +85,10 @@ LINKS_TRAFFIC_PER_CONFIG = (2.0 * 1733610.1 + 1900112.3) * 1024 / 2097152
 # edges each, shape 8 waves per CU x 4 slots), per launch, from rocprofv3
 # counters (profiles/k_edge_first_chains_planner_starts.md): VALU wave
 # instructions, FP32 and FP64 operations executed (SQ_INSTS_VALU_FLOPS_FP32 /
-# _FP64 x 26.11 lanes active per VALU instruction) and HBM bytes (FETCH_SIZE
-# 38,058 KiB x 2.0 + WRITE_SIZE 2,540.1 KiB).
-EDGE_COUNTERS = {"valu_instr": 2.7824e8, "fp32_flop": 1.0554e8 * 26.11, "fp64_flop": 3.0155e7 * 26.11,
-                 "traffic_bytes": (2.0 * 38058.0 + 2540.1) * 1024,
+# _FP64 x 40.78 lanes active per VALU instruction) and HBM bytes (FETCH_SIZE
+# 36,718.9 KiB x 2.0 + WRITE_SIZE 2,500.3 KiB).
+EDGE_COUNTERS = {"valu_instr": 1.7790e8, "fp32_flop": 4.1102e7 * 40.78, "fp64_flop": 3.0050e7 * 40.78,
+                 "traffic_bytes": (2.0 * 36718.9 + 2500.3) * 1024,
                  "source": "profiles/k_edge_first_chains_planner_starts.md"}
 PEAK_FP64_TFLOPS = 78.6
 # HBM bytes per launch of the FP32 bulk kernel on the headline workload from
@@ -788,7 +788,7 @@ def main():
         "roofline": roof,
         "tuning": tune,
         "refine": {"configs": refined, "fraction": refined / n,
-                   "kernel": "k_distance_refine_pairs" if L * w.scene.num_obj <= 256 else "k_distance_refine",
+                   "kernel": "k_distance_pairs" if L * w.scene.num_obj <= 1024 else "k_distance_refine",
                    "kernel_ms": refine_ms},
         "walk_order": {"kernels": "k_coh_hist, k_coh_scan, k_coh_bucket, k_coh_lowsort "
                                   "(sort by the first joint angles)",

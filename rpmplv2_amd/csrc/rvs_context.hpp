@@ -114,7 +114,7 @@ struct rvs_context {
     // and batch (tuning_for), otherwise the variant
     int32_t fast_variant = -1;
     // reference-arithmetic distance batches up to this many configurations
-    // run one wave per configuration (latency) instead of one lane
+    // run 16 or 64 lanes per configuration (latency) instead of one
     int64_t wave_max = 16384;
     int32_t edge_waves_per_cu = 16;   // persistent first-collision kernel: resident waves per CU
     int32_t edge_spl = 0;             // ... and slots per lane in one 64-lane item (0: by the slots of the call)

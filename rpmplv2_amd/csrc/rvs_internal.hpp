@@ -276,8 +276,9 @@ hipError_t launch_distance_pairs(const RobotDev& rb, const EnvDev& env, const Qu
 // (a walk order from launch_coherence_order).
 hipError_t launch_distance_ref32(const RobotDev& rb, const EnvDev& env, const QueryParams& qp, const float* q,
                                  int64_t n, const DistOut& out, hipStream_t st, const int32_t* perm = nullptr);
-// The same results with one wave per configuration (lanes over obstacles):
-// the low-latency form for small batches.
+// The same results with 16 or 64 lanes per configuration (its pairs over
+// them; lanes over obstacles where the pairs do not fit): the low-latency form
+// for small batches.
 hipError_t launch_distance_ref32_waves(const RobotDev& rb, const EnvDev& env, const QueryParams& qp, const float* q,
                                        int64_t n, const DistOut& out, hipStream_t st);
 // Either form by batch size: waves up to wave_max configurations.

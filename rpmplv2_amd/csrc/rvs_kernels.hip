@@ -143,8 +143,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
     distance_body<float, WANT_NP, OBB>(rb, env, qp, q, n, out, perm);
 }
 
-// Exact recomputation of the configurations the FP32 bulk pass flagged: one
-// wave per configuration, one link at a time.  For link i, lane t evaluates
+// Exact recomputation of the configurations the FP32 bulk pass flagged, where
+// their pairs do not fit k_distance_pairs (rvs_pairs.hip): one wave per
+// configuration, one link at a time.  For link i, lane t evaluates
 // obstacles j = t, t + 64, ... with the exact tree; the wave then reduces the
 // smallest filtered distance and the first obstacle whose filtered distance
 // is <= 0.  That gives exactly what the reference's sequential loop gives:

@@ -104,7 +104,8 @@ inline PairLds pair_lds(const RobotDev& rb, const EnvDev& env, bool want_np, int
 // 44 us, 16,384 60 us (one wave per configuration with every pair evaluated:
 // 30, 60 and 121 us; the serial kinematics alone took 13,000 of a wave's 39,000
 // cycles, now 6,000), one state with its nearest points 75 us from copied host
-// arrays (90 us with a link at a time) and 30 us in place; 64 lanes a configuration: launch_distance_pairs.
+// arrays (90 us with a link at a time) and 30 us in place.  The times of both
+// widths stand at launch_distance_pairs.
 template <bool OBB, bool WANT_NP, int G>
 __global__ __launch_bounds__(64) void k_distance_pairs(RobotDev rb, EnvDev env, QueryParams qp,
                                                        const float* __restrict__ q, DistOut out,

@@ -424,7 +424,7 @@ class Engine:
         return out
 
     def set_small_batch(self, max_configs: int):
-        """Reference-arithmetic batches up to max_configs run one wave per configuration."""
+        """Reference-arithmetic batches up to max_configs run 16 or 64 lanes per configuration."""
         self._check(lib().rvs_set_small_batch(self._ctx, int(max_configs)), "rvs_set_small_batch")
 
     def set_motion_law(self, env: int, motion_type: int, vel, max_vel, ws_center=(0.0, 0.0, 0.0),
