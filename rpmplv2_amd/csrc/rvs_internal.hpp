@@ -49,6 +49,7 @@ struct QueryParams {
     float band;     // near-contact band of the FP32 path
     int32_t num_checks;
     int32_t flag_link;   // set by the FP32 path's launches: flag_entry carries the start link
+    const int32_t* first_warm;   // set by them too: the obstacle every first link starts its walk from (null: none)
 };
 
 // Entries of the FP32 path's list of configurations for the exact pass.  In
