@@ -64,7 +64,7 @@ PEAK_HBM_GBPS = 8000.0
 COUNTER_FLOP_PER_CONFIG = {
     ("xarm6_16aabb_ground", "k_distance_fast"): (2276.6, "profiles/k_distance_fast_xarm6_1M.md"),
     ("chain22_512rotated_boxes", "k_distance_fast_links"):
-        (20217.9, "profiles/k_distance_fast_links_chain22_512obb.md"),
+        (15224.3, "profiles/k_distance_fast_links_chain22_512obb.md"),
 }
 # VALU wave instructions per configuration of the same kernels (SQ_INSTS_VALU
 # / configurations, same profiles): the issue rate they reach against the
@@ -73,14 +73,14 @@ COUNTER_FLOP_PER_CONFIG = {
 # long before the FP32 peak.
 COUNTER_VALU_PER_CONFIG = {
     ("xarm6_16aabb_ground", "k_distance_fast"): 74.77,
-    ("chain22_512rotated_boxes", "k_distance_fast_links"): 950.54,
+    ("chain22_512rotated_boxes", "k_distance_fast_links"): 790.70,
 }
 PEAK_VALU_ISSUE_G = 1024 * 2.4 / 4
 # HBM bytes per configuration of the link-major bulk pass on the 22-DOF chain
-# with 512 rotated boxes (all 22 launches of a call): FETCH_SIZE 1,723,688.4
-# KiB x 2.0 + WRITE_SIZE 1,899,474.9 KiB x 1.0 per call on 2,097,152
+# with 512 rotated boxes (all 22 launches of a call): FETCH_SIZE 1,733,610.1
+# KiB x 2.0 + WRITE_SIZE 1,900,112.3 KiB x 1.0 per call on 2,097,152
 # configurations (profiles/k_distance_fast_links_chain22_512obb.md).
-LINKS_TRAFFIC_PER_CONFIG = (2.0 * 1723688.4 + 1899474.9) * 1024 / 2097152
+LINKS_TRAFFIC_PER_CONFIG = (2.0 * 1733610.1 + 1900112.3) * 1024 / 2097152
 # The first-collision search on the planner-start edges (four chains, 4,096
 # edges each, shape 8 waves per CU x 4 slots), per launch, from rocprofv3
 # counters (profiles/k_edge_first_chains_planner_starts.md): VALU wave
