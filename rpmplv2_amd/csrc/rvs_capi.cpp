@@ -36,6 +36,7 @@ rvs_status fail(rvs_context* c, rvs_status s, const std::string& msg) {
 }
 
 rvs_status hip_fail(rvs_context* c, hipError_t e, const char* what) {
+    (void)hipGetLastError();   // reported here: the next call's launches start without it
     return fail(c, e == hipErrorOutOfMemory ? RVS_ENOMEM : RVS_EDEVICE,
                 std::string(what) + ": " + hipGetErrorString(e));
 }

@@ -17,6 +17,9 @@
 
 namespace rvs {
 
+// A request that fails leaves no buffer and no error behind: the runtime keeps
+// a call's error for hipGetLastError across later calls that succeed, and the
+// launches that a caller goes on with, in less memory, report by it.
 struct DevBuf {
     void* p = nullptr;
     size_t cap = 0;
@@ -27,8 +30,13 @@ struct DevBuf {
         cap = 0;
         size_t want = std::max<size_t>(bytes, 1 << 20);
         hipError_t e = hipMalloc(&p, want);
-        if (e == hipSuccess) cap = want;
-        return e;
+        if (e != hipSuccess) {
+            p = nullptr;
+            (void)hipGetLastError();
+            return e;
+        }
+        cap = want;
+        return hipSuccess;
     }
     void release() {
         if (p) (void)hipFree(p);
@@ -49,8 +57,13 @@ struct PinnedBuf {
         cap = 0;
         size_t want = std::max<size_t>(bytes, 1 << 20);
         hipError_t e = hipHostMalloc(&p, want, hipHostMallocDefault);
-        if (e == hipSuccess) cap = want;
-        return e;
+        if (e != hipSuccess) {
+            p = nullptr;
+            (void)hipGetLastError();
+            return e;
+        }
+        cap = want;
+        return hipSuccess;
     }
     void release() {
         if (p) (void)hipHostFree(p);

@@ -62,7 +62,12 @@ class Pool {
         host_ = host;
         hipError_t e = host ? hipHostMalloc(reinterpret_cast<void**>(&base_), cap_, hipHostMallocDefault)
                             : hipMalloc(reinterpret_cast<void**>(&base_), cap_);
-        if (e == hipSuccess) free_[0] = cap_;
+        if (e == hipSuccess) {
+            free_[0] = cap_;
+        } else {
+            base_ = nullptr;
+            (void)hipGetLastError();   // (the staging pool is optional)
+        }
         return e;
     }
     void destroy() {
@@ -824,7 +829,11 @@ const char* rvs_server_last_error(rvs_server* s) {
 
 void* rvs_host_alloc(int64_t bytes) {
     void* p = nullptr;
-    if (bytes <= 0 || hipHostMalloc(&p, (size_t)bytes, hipHostMallocDefault) != hipSuccess) return nullptr;
+    if (bytes <= 0) return nullptr;
+    if (hipHostMalloc(&p, (size_t)bytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();   // the caller goes on with other memory
+        return nullptr;
+    }
     return p;
 }
 
