@@ -87,13 +87,6 @@ __global__ __launch_bounds__(64) void k_traj_safe(RobotDev rb, QueryParams qp, T
     const float* points = a.points + c * (int64_t)K * D;
     auto PA = [&](int k) { return Vec3<float>{ska[3 * k], ska[3 * k + 1], ska[3 * k + 2]}; };
     auto PL = [&](int k) { return Vec3<float>{skl[(3 * k) * 64 + t], skl[(3 * k + 1) * 64 + t], skl[(3 * k + 2) * 64 + t]}; };
-    // t_iter at point i: t_iter + time_step added i times, in order
-    auto time_at = [&](int i) {
-        if (table) return times[i];
-        float ti = a.t_iter;
-        for (int k = 0; k < i; ++k) ti += a.time_step;
-        return ti;
-    };
     float max_obs_vel = 0.0f;   // AbstractTrajectory.cpp:44-49
     for (int o = t; o < M; o += 64)
         if (a.max_vel[o] > max_obs_vel) max_obs_vel = a.max_vel[o];
@@ -148,6 +141,7 @@ __global__ __launch_bounds__(64) void k_traj_safe(RobotDev rb, QueryParams qp, T
     if (!unsafe) anchor();
     float t_init = 0.0f;
     int s = 0;
+    float ts = a.t_iter;   // time at point s
     while (!unsafe) {
         // radii of the reference state, a row a lane (D <= 64 rows)
         if (t < D) {
@@ -161,12 +155,25 @@ __global__ __launch_bounds__(64) void k_traj_safe(RobotDev rb, QueryParams qp, T
         }
         wave_sync();
         int f = K;
+        float tf = 0.0f;   // time at point f
+        float tb = ts;     // time at the chunk's first point
         for (int b = s; b < K; b += 64) {
             const int i = b + t;
             bool fail = false;
+            // time at point i: t_iter + time_step added i times, in order;
+            // without the table the additions go on from the chunk before
+            // (from t_iter each time a trajectory of 10,000 points took 20 ms
+            // instead of 0.8)
+            float ti = tb;
+            if (table) {
+                if (i < K) ti = times[i];
+            } else {
+                for (int k = 0; k < t; ++k) ti += a.time_step;
+                tb = __shfl(ti, 63) + a.time_step;
+            }
             if (i < K) {
                 const float* qf = points + (int64_t)i * D;
-                const float rho_obs = max_obs_vel * (time_at(i) - t_init);
+                const float rho_obs = max_obs_vel * (ti - t_init);
                 for (int k = 0; k < D; ++k) dq[k * 64 + t] = fabsf(qf[k] - qa[k]);
                 for (int j = 0; j < D && !fail; ++j) {
                     const float rho_robot =
@@ -176,13 +183,14 @@ __global__ __launch_bounds__(64) void k_traj_safe(RobotDev rb, QueryParams qp, T
             }
             const uint64_t m = __ballot(fail);
             if (m) {
-                f = b + __ffsll((unsigned long long)m) - 1;
+                const int lane = __ffsll((unsigned long long)m) - 1;
+                f = b + lane;
+                tf = __shfl(ti, lane);
                 break;
             }
         }
         if (f >= K) break;   // every remaining point inside the bubble
         // possible collision at point f: it becomes the reference state
-        const float tf = time_at(f);
         wave_sync();
         for (int k = t; k < D; k += 64) qa[k] = points[(int64_t)f * D + k];
         for (int l = t; l < L; l += 64) pr[l] = qp.maxd;
@@ -202,6 +210,7 @@ __global__ __launch_bounds__(64) void k_traj_safe(RobotDev rb, QueryParams qp, T
         if (__any(bad)) unsafe = true;
         t_init = tf;
         s = f + 1;
+        ts = tf + a.time_step;
         wave_sync();
     }
     if (t == 0) a.safe[c] = unsafe ? 0 : 1;

@@ -1113,6 +1113,75 @@ def test_trajectory_is_safe_sizes(oracle, engine, dofs, boxes, points, traj, sel
     assert np.array_equal(safe, osafe)
 
 
+def _boxes_around(rng, rb, count, side_lo, side_hi, reach, clearance=0.02):
+    """Boxes in a ball of `reach` around the middle of the zero pose's
+    skeleton, their bounding balls clear of it."""
+    P = R.skeleton_np(rb, np.zeros(rb.num_dofs))[0]
+    t = np.linspace(0.0, 1.0, 21)[:, None, None]
+    pts = (P[None, :-1] + t * (P[1:] - P[:-1])[None]).reshape(-1, 3)
+    gap = np.max(rb.radius) + clearance
+    rows = []
+    while len(rows) < count:
+        sc = W._boxes(rng, 4 * count + 8, side_lo, side_hi, reach, center=P.mean(0))
+        far = np.linalg.norm(sc.pos[:, None] - pts[None], axis=2).min(1) > 0.5 * np.linalg.norm(sc.dim, axis=1) + gap
+        rows += [k for k in zip(sc.dim[far], sc.pos[far])]
+    dim, pos = (np.array(x[:count]) for x in zip(*rows))
+    return W.Scene(dim, pos, np.tile([1.0, 0.0, 0.0, 0.0], (count, 1)), np.zeros(count, np.uint8),
+                   np.full(count, 1000.0, np.float32))
+
+
+@pytest.mark.parametrize("points", [1025, 2500])
+def test_trajectory_points_past_the_time_table(oracle, engine, points):
+    """More points than the time table holds, with reference states along the
+    way: equal to the oracle's walk, both outcomes among them."""
+    rng = np.random.default_rng(points)
+    rb = R.xarm6()
+    sc = _boxes_around(rng, rb, 12, 0.05, 0.2, 0.7)
+    osc = oracle.scene_of(sc)
+    root = np.zeros(6, np.float32)
+    _, p0, ok, np0 = oracle.distance(rb, osc, root[None], 32, want_np=True)
+    assert ok[0] == 1
+    v = rng.normal(size=(40, 6))
+    v /= np.linalg.norm(v, axis=1, keepdims=True)
+    s = np.linspace(0, 1, points + 1)[1:]
+    pts = (rng.uniform(0.05, 2.5, 40)[:, None, None] * s[None, :, None] * v[:, None, :]).astype(np.float32)
+    mv = rng.uniform(0, 0.05, 12).astype(np.float32)
+    dt = 1.0 / points
+    rid, eid = engine.load_robot(rb), engine.create_env(sc)
+    safe = engine.trajectory_is_safe(rid, eid, pts, root, p0[0], np0[0], mv, t_iter=0.1, time_step=dt)
+    osafe = oracle.traj_safe(rb, osc, pts, root, p0[0], np0[0], mv, 0.1, dt)
+    assert 0.1 < osafe.mean() < 0.9
+    assert np.array_equal(safe, osafe)
+
+
+def test_trajectory_cost_grows_with_its_points(engine):
+    """Eight times the points of a trajectory that stays near its reference
+    state take at most twenty times as long (64 times if every chunk added its
+    times up from the start)."""
+    import time
+
+    rb = R.xarm6()
+    sc = W._boxes(np.random.default_rng(3), 4, 0.05, 0.1, 0.2, center=(0.0, 0.0, 3.0))
+    rid, eid = engine.load_robot(rb), engine.create_env(sc)
+    root = np.zeros(6, np.float32)
+    _, p0, _, np0 = engine.distance(rid, eid, root[None], want_nearest=True)
+
+    def cost(points):
+        pts = np.zeros((1, points, 6), np.float32)
+        best = float("inf")
+        for _ in range(4):
+            t0 = time.perf_counter()
+            safe = engine.trajectory_is_safe(rid, eid, pts, root, p0[0], np0[0], np.zeros(4, np.float32),
+                                             time_step=1e-4)
+            best = min(best, time.perf_counter() - t0)
+            assert safe[0] == 1
+        return best
+
+    short, long = cost(4096), cost(32768)
+    print(f"4,096 points {1e6 * short:.0f} us, 32,768 points {1e6 * long:.0f} us")
+    assert long < 20 * short
+
+
 @pytest.mark.parametrize("boxes", [1, 8, 9, 63, 64, 65, 130])
 @pytest.mark.parametrize("dofs", [1, 6, 22])
 def test_edge_first_collision_obstacle_marks(oracle, engine, boxes, dofs):
