@@ -46,11 +46,24 @@ constexpr int64_t kExactSortMin = 65536;
 // Host arrays of a distance or trajectory call up to this many bytes, inputs
 // and outputs together, go through pinned host memory that the kernels address:
 // a copy of an array costs about 10 us however small it is, the link carries
-// 1 MiB in about 25 us.  xArm6 in reference arithmetic, pinned against copies:
-// one state and 4 boxes with nearest points 30 / 93 us, 4,096 configurations 61
-// / 98, 16,384 (0.9 MB) 99 / 180; 40 boxes with nearest points, 170
-// configurations (1 MB), about 140 / 180.  The block itself is 1 MiB at least.
+// 1 MiB in about 25 us.  In place against copies: xArm6, one state and 16 boxes
+// with nearest points 33 / 82 us, reference arithmetic 6,573 configurations 56
+// / 226, 19,720 170 / 210, FP64 174 / 214, FP32 with refinement 123 / 190;
+// 22-DOF chain and 64 boxes, 5,729 configurations 347 / 400 (FP32 638 / 647);
+// 512 boxes 838 / 907.  The block itself is 1 MiB at least.  Not in place: the
+// FP32 link-major launches, which read a configuration's row again at every
+// link and write its profile a word at a time (5,729 configurations among 512
+// boxes 2,420 / 2,190 us).
 constexpr size_t kPinnedIo = 1024 * 1024;
+// Trajectories: a wave reads the current state's arrays again for each of its
+// reference states, so above this many bytes they are copied to the device
+// (xArm6, 100 trajectories of 60 points, in place against copies: 120 boxes 70
+// / 83 us, 240 boxes 92 / 95, 1,000 boxes 232 / 176; 500 trajectories 93 / 98,
+// 116 / 110); and it goes through its points 64 at a time, one read over the
+// link after the other, so long trajectories are copied (40 of 1,000 points 132
+// / 154 us, 4 of 10,000 840 / 790).
+constexpr size_t kPinnedState = 16 * 1024;
+constexpr int32_t kPinnedPoints = 1024;
 // The device's address of the context's pinned block of kPinnedIo bytes;
 // nullptr when there is none to be had.
 void* pinned_io(rvs_context* c) {
@@ -824,7 +837,7 @@ rvs_status rvs_distance(rvs_context* c, int32_t robot, int32_t env, const float*
     // small host arrays stay in a pinned block that the kernels read and write
     const size_t io = Carve::need({(size_t)n * D * 4, (size_t)n * 4, profile ? (size_t)n * L * 4 : 0,
                                    nearest ? (size_t)n * M * L * 24 : 0, (size_t)n});
-    void* const pinned = (flags & RVS_F_DEVICE) || io > kPinnedIo ? nullptr : pinned_io(c);
+    void* const pinned = (flags & RVS_F_DEVICE) || io > kPinnedIo || links_need ? nullptr : pinned_io(c);
     if ((flags & RVS_F_DEVICE) || pinned) {
         e = c->arena.ensure(Carve::need({refine_bytes, coh_need, links_need}));
         if (e != hipSuccess && without_links()) e = c->arena.ensure(Carve::need({refine_bytes, coh_need}));
@@ -1547,32 +1560,35 @@ rvs_status rvs_trajectory_is_safe(rvs_context* c, int32_t robot, int32_t env, co
         return RVS_OK;
     }
     // the current state's arrays are small: through a pinned mirror, in one
-    // copy; the points straight from the caller.  A small call stays in the
-    // mirror with all it reads and writes.
+    // copy (one by one where there is no mirror to be had); the points straight
+    // from the caller.  A small call stays in the mirror with all it reads and
+    // writes, but for a state above kPinnedState.
     const size_t state = Carve::need({(size_t)D * 4, (size_t)L * 4, set * 4, (size_t)M * 4});
     const size_t io = state + Carve::need({pb, (size_t)num_traj});
-    void* const pinned = io <= kPinnedIo ? pinned_io(c) : nullptr;
-    hipError_t e = pinned ? hipSuccess : c->arena.ensure(io);
-    if (e == hipSuccess && !pinned) e = c->staging.ensure(state);
+    void* const pinned = io <= kPinnedIo && num_points <= kPinnedPoints ? pinned_io(c) : nullptr;
+    const bool state_in_place = pinned && state <= kPinnedState;
+    hipError_t e = state_in_place ? hipSuccess : c->arena.ensure(pinned ? state : io);
     if (e != hipSuccess) return hip_fail(c, e, "rvs_trajectory_is_safe: staging");
-    char* const mirror = static_cast<char*>(c->staging.p);
-    Carve cv(pinned ? pinned : c->arena.p);
+    char* const mirror = pinned || c->staging.ensure(state) == hipSuccess ? static_cast<char*>(c->staging.p) : nullptr;
+    Carve sv(state_in_place ? pinned : c->arena.p);
     auto put = [&](size_t bytes, const float* src) {
-        float* const dev = cv.take<float>(bytes / 4);
-        if (bytes) std::memcpy(mirror + (reinterpret_cast<char*>(dev) - cv.base), src, bytes);
+        float* const dev = sv.take<float>(bytes / 4);
+        if (mirror && bytes) std::memcpy(mirror + (reinterpret_cast<char*>(dev) - sv.base), src, bytes);
+        else if (e == hipSuccess) e = h2d(dev, src, bytes, c->stream);
         return dev;
     };
     a.q_current = put((size_t)D * 4, q_current);
     a.profile_current = put((size_t)L * 4, profile_current);
     a.nearest_current = put(set * 4, nearest_current);
     a.max_vel = put((size_t)M * 4, max_vel);
-    float* ps = nullptr;
-    if (pinned) {
-        ps = put(pb, points);
-    } else {
-        e = h2d(cv.base, mirror, cv.off, c->stream);
-        ps = cv.take<float>(pb / 4);
+    if (mirror && !state_in_place) e = h2d(sv.base, mirror, sv.off, c->stream);
+    Carve cv(pinned ? pinned : c->arena.p);
+    cv.off = sv.off;
+    float* const ps = cv.take<float>(pb / 4);
+    if (!pinned) {
         if (e == hipSuccess) e = h2d(ps, points, pb, c->stream);
+    } else if (pb) {
+        std::memcpy(mirror + (reinterpret_cast<char*>(ps) - cv.base), points, pb);
     }
     a.points = ps;
     a.safe = cv.take<uint8_t>(num_traj);

@@ -1260,22 +1260,52 @@ def test_host_arrays_in_place_and_copied(engine, n):
     assert np.array_equal(near, np.concatenate(parts), equal_nan=True)
 
 
-def test_trajectories_in_place_and_copied(engine):
-    """4,500 trajectories of 10 points (1.1 MB, copied) against the same in parts
-    that are used in place."""
+@pytest.mark.parametrize("n", [17, 100, 3000, 5700])
+def test_link_major_batches_of_host_arrays(engine, n):
+    """Host arrays below 1 MiB of a batch that runs link by link: the device
+    arrays' bits."""
+    import torch
+
+    rng = np.random.default_rng(n)
+    rb = R.chain(rng.uniform(0.1, 0.3, 22), radius=0.04)
+    sc = _boxes_around(rng, rb, 300, 0.02, 0.2, 2.0)
+    q = rng.uniform(-np.pi, np.pi, (n, 22)).astype(np.float32)
+    rid, eid = engine.load_robot(rb), engine.create_env(sc, rvs.ENV_AABB)
+    out = (torch.empty(n, device="cuda"), torch.empty((n, 22), device="cuda"),
+           torch.empty(n, dtype=torch.uint8, device="cuda"))
+    engine.distance_device(rid, eid, torch.from_numpy(q).cuda(), *out, precision=rvs.PREC_FP32_REFINE)
+    got = engine.distance(rid, eid, q, precision=rvs.PREC_FP32_REFINE)
+    for a, b in zip(got, out):
+        assert np.array_equal(a, b.cpu().numpy())
+
+
+@pytest.mark.parametrize("boxes,points,parts", [(12, 10, 900), (200, 10, 900), (12, 1025, 9)])
+def test_trajectories_in_place_and_copied(oracle, engine, boxes, points, parts):
+    """4,500 trajectories of 10 points (1.1 MB, copied) against the same in
+    parts that are used in place, with the current state's arrays in place (12
+    boxes) and copied (200 boxes, 29 KB); long trajectories, copied whole: the
+    oracle's walk, both outcomes among them."""
     rng = np.random.default_rng(5)
     rb = R.xarm6()
-    sc = W._boxes(rng, 12, 0.05, 0.2, 0.9)
+    sc = _boxes_around(rng, rb, boxes, 0.05, 0.2, 0.7)
+    osc = oracle.scene_of(sc)
     rid, eid = engine.load_robot(rb), engine.create_env(sc, rvs.ENV_AABB)
-    q = rng.uniform(-1, 1, 6).astype(np.float32)
-    _, prof, _, near = engine.distance(rid, eid, q[None], want_nearest=True)
-    pts = (q + np.cumsum(rng.normal(0, 0.01, (4500, 10, 6)), axis=1)).astype(np.float32)
-    vel = np.full(12, 0.1, np.float32)
+    q = np.zeros(6, np.float32)
+    _, prof, ok, near = oracle.distance(rb, osc, q[None], 32, want_np=True)
+    assert ok[0] == 1
+    n = 5 * parts
+    u = rng.normal(size=(n, 6))
+    u = rng.uniform(0.05, 2.5, (n, 1)) * u / np.linalg.norm(u, axis=1, keepdims=True)
+    pts = (np.linspace(0, 1, points + 1)[1:, None] * u[:, None]).astype(np.float32)
+    vel = np.full(boxes, 0.1, np.float32)
+    dt = 0.1 / points
 
     def safe(p):
-        return engine.trajectory_is_safe(rid, eid, p, q, prof[0], near[0], vel, time_step=0.01)
+        return engine.trajectory_is_safe(rid, eid, p, q, prof[0], near[0], vel, time_step=dt)
 
-    whole = safe(pts)
-    print(f"safe {whole.mean():.3f}")
-    assert np.array_equal(whole, np.concatenate([safe(pts[k:k + 900]) for k in range(0, 4500, 900)]))
-    assert np.array_equal(whole[:1], safe(pts[:1]))
+    want = oracle.traj_safe(rb, osc, pts, q, prof[0], near[0], vel, 0.0, dt)
+    print(f"safe {want.mean():.3f}")
+    assert 0.05 < want.mean() < 0.95
+    assert np.array_equal(safe(pts), want)
+    assert np.array_equal(np.concatenate([safe(pts[k:k + parts]) for k in range(0, n, parts)]), want)
+    assert np.array_equal(safe(pts[:1]), want[:1])
