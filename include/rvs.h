@@ -410,6 +410,9 @@ typedef struct rvs_tuning {
 rvs_status rvs_autotune(rvs_context* ctx, int32_t robot, int32_t env, const float* q, int64_t n, uint32_t flags,
                         rvs_tuning* best);
 rvs_status rvs_set_tuning(rvs_context* ctx, int32_t robot, int32_t env, const rvs_tuning* tuning);
+/* The recorded shape; without one the shape that an RVS_PREC_FP32_REFINE call
+ * of 1,048,576 configurations chooses (other batches may choose others).  ms is
+ * 0. */
 rvs_status rvs_get_tuning(rvs_context* ctx, int32_t robot, int32_t env, rvs_tuning* tuning);
 
 /* Batches of reference-arithmetic distances (RVS_PREC_REF32 calls, calls

@@ -1285,13 +1285,16 @@ rvs_status rvs_set_small_batch(rvs_context* c, int64_t max_configs) {
 
 rvs_status rvs_get_tuning(rvs_context* c, int32_t robot, int32_t env, rvs_tuning* t) {
     if (!c || !t) return fail(c, RVS_EINVAL, "rvs_get_tuning: null argument");
-    int32_t L = 0, M = 0;
+    int32_t D = 0, L = 0, M = 0;
     {
         CtxLock lk(c);
-        if (robot_ok(c, robot)) L = c->robots[robot].num_links;
+        if (robot_ok(c, robot)) {
+            D = c->robots[robot].num_dofs;
+            L = c->robots[robot].num_links;
+        }
         if (env_ok(c, env)) M = c->envs[env].dev.num_obj;
     }
-    const FastTuning f = c->tuning_for(robot, env, 0, L, M, 0);
+    const FastTuning f = c->tuning_for(robot, env, D, L, M, (int64_t)1 << 20);
     *t = rvs_tuning{f.variant, f.block, f.blocks_per_cu, f.coh_bits, 0.0f};
     return RVS_OK;
 }

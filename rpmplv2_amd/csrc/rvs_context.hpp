@@ -163,9 +163,8 @@ struct rvs_context {
             // / 125).  Where they order the whole pose (at most 3 joints) they
             // pay early, unless the walk is short: planar arm, 40 boxes 108
             // against 164 us for 65,536; 4 boxes 130 against 102 for 1,000,003.
-            // (n <= 0: the shape of a large batch, for rvs_get_tuning)
             const int64_t from = (int64_t)links * objects < 32 ? INT64_MAX : (dofs <= 3 ? 1024 : 1 << 18);
-            return rvs::FastTuning{0, 64, 0, n <= 0 || n >= from ? 5 : 0};
+            return rvs::FastTuning{0, 64, 0, n >= from ? 5 : 0};
         }
         // Long walks.  Link-major launches (4) against lane refill (1), 22-DOF
         // chain: 512 boxes 5.9 against 11.7 ms for 2,097,152 configurations and
@@ -173,13 +172,13 @@ struct rvs_context {
         // 1,000,000 and 1.2 against 1.6 for 1,000; 128 boxes 3.5 against 3.8 ms
         // for 1,000,000 but 1.64 against 1.58 for 300,000; 96 boxes 3.4 against
         // 3.2.  Their lists take 128 bytes a configuration: at most 2 GiB.
-        if (n > 0 && n <= (int64_t)1 << 24 && (objects >= 200 || (objects >= 128 && n >= (int64_t)1 << 19)))
+        if (n <= (int64_t)1 << 24 && (objects >= 200 || (objects >= 128 && n >= (int64_t)1 << 19)))
             return rvs::FastTuning{4, 512, 0, 5};
         // Lane refill with pair queues (3) for small batches: 22-DOF chain and
         // 96 boxes 0.64 against 0.77 ms for 1,000 and 0.73 against 0.85 for
         // 30,000; 14-DOF chain and 65 boxes 0.40 against 0.46 for 100,000; but
         // 18-DOF chain and 80 boxes 1.17 against 1.03 for 400,000.
-        if (n > 0 && n <= (int64_t)1 << 17) return rvs::FastTuning{3, 512, 0, 5};
+        if (n <= (int64_t)1 << 17) return rvs::FastTuning{3, 512, 0, 5};
         return rvs::FastTuning{1, 256, 0, 5};
     }
     // Walk-order bits of the exact paths: a recorded shape's, else 5.

@@ -163,3 +163,27 @@ def test_launch_shapes_same_bits(engine, scene):
         for a, b in zip(got[:3], ref[:3]):
             assert np.array_equal(a, b), (variant, block)
     assert 0 < nref < len(q) and 0.01 < ref[2].mean() < 0.99
+
+
+def test_unrecorded_shape_is_that_of_a_large_batch(engine):
+    """get_tuning without a recorded shape names what a call of 2^20
+    configurations runs, in the form that set_tuning takes; recording it
+    changes no result."""
+    rng = np.random.default_rng(4)
+    for rb, boxes, want in ((R.planar_2dof(), 4, {"variant": 0, "block": 64, "coherence_bits": 0}),
+                            (R.xarm6(), 17, {"variant": 0, "block": 64, "coherence_bits": 5}),
+                            (R.chain(rng.uniform(0.1, 0.3, 22), radius=0.04), 60,
+                             {"variant": 1, "block": 256, "coherence_bits": 5}),
+                            (R.chain(rng.uniform(0.1, 0.3, 22), radius=0.04), 512,
+                             {"variant": 4, "block": 512, "coherence_bits": 5})):
+        sc = W._boxes(rng, boxes, 0.02, 0.2, 2.0)
+        q = rng.uniform(-np.pi, np.pi, (3000, rb.num_dofs)).astype(np.float32)
+        rid, eid = engine.load_robot(rb), engine.create_env(sc)
+        got = engine.get_tuning(rid, eid)
+        assert {k: got[k] for k in want} == want, (boxes, got)
+        ref = engine.distance(rid, eid, q, precision=rvs.PREC_FP32_REFINE)
+        engine.set_tuning(rid, eid, **got)
+        again = engine.distance(rid, eid, q, precision=rvs.PREC_FP32_REFINE)
+        assert engine.get_tuning(rid, eid) == got
+        for a, b in zip(ref[:3], again[:3]):
+            assert np.array_equal(a, b)
