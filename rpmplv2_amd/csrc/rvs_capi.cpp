@@ -821,12 +821,11 @@ rvs_status rvs_distance(rvs_context* c, int32_t robot, int32_t env, const float*
     const size_t coh_need = (prec == RVS_PREC_FP32_REFINE || sort_exact) ? coh_bytes(n, D) : 0;
     FastTuning ft = c->tuning_for(robot, env, D, L, M, n);
     size_t links_need = (prec == RVS_PREC_FP32_REFINE && ft.variant == 4) ? fast_links_bytes(n) : 0;
-    // a link-major shape that nobody recorded gives way to lane refill (the
-    // same results) when its lists cannot be had
+    // a link-major shape that nobody recorded gives way (to the same results)
+    // when its lists cannot be had
     auto without_links = [&]() {
         if (!links_need || c->tuned(robot, env)) return false;
-        ft.variant = 1;
-        ft.block = 256;
+        ft = c->tuning_for(robot, env, D, L, M, n, false);
         links_need = 0;
         return true;
     };
@@ -1006,9 +1005,8 @@ rvs_status rvs_distance_async(rvs_context* c, int32_t robot, int32_t env, const 
             if (need > c->arena.cap) c->drain_async();   // growing frees the block earlier calls use
             e = c->arena.ensure(need);
             if (e != hipSuccess && links_need && !c->tuned(robot, env)) {
-                // a link-major shape that nobody recorded gives way to lane refill (the same results)
-                ft.variant = 1;
-                ft.block = 256;
+                // a link-major shape that nobody recorded gives way (to the same results)
+                ft = c->tuning_for(robot, env, D, L, M, n, false);
                 links_need = 0;
                 e = c->arena.ensure(Carve::need({(size_t)n * 4 + 256, coh_bytes(n, D)}));
             }
@@ -1069,7 +1067,7 @@ rvs_status rvs_distance_async_static(rvs_context* c, int32_t robot, int32_t env,
     const QueryParams qp = params_of(c);
     DistOut out{};
     out.d = d; out.profile = profile; out.verdict = verdict;
-    const FastTuning ft = c->tuning_for(robot, env, D, L, M, n);
+    const FastTuning ft = c->tuning_for(robot, env, D, L, M, n, false);   // the static array has no room for lists
     hipError_t e = async_begin(c, st);
     if (e == hipSuccess && n > 0) {
         Carve cv(base);
@@ -1081,7 +1079,7 @@ rvs_status rvs_distance_async_static(rvs_context* c, int32_t robot, int32_t env,
             // counters cleared by a kernel: the scratch keeps the last call's contents
             e = launch_zero_u32(rcount, 64, st);
             if (e == hipSuccess) e = launch_coherence_order(rb.dev, q, n, ft.coh_bits, coh, &perm, st);
-            // no links scratch in the static array: a link-major shape runs as variant 3
+            // (a recorded link-major shape runs as variant 3)
             if (e == hipSuccess)
                 e = launch_distance_fast(rb.dev, ev.dev, qp, q, n, out, ridx, rcount, ft, perm, nullptr, c->num_cus,
                                          st);

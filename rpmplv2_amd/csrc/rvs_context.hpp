@@ -91,6 +91,44 @@ struct EnvRec {
     EnvStepDev step{};                    // motion-law state on the device
 };
 
+// The launch shape of an RVS_PREC_FP32_REFINE batch of n configurations that
+// nobody recorded one for: by the length of the walk and the batch (every shape
+// gives the same bits, so the choice may follow n).  lists: whether the call
+// can have the link-major pass's scratch (fast_links_bytes).
+inline FastTuning default_shape(int32_t dofs, int32_t links, int32_t objects, int64_t n, bool lists) {
+    if ((int64_t)links * objects < 1024) {
+        // The walk order's four kernels (16 to 31 us) pay for themselves
+        // in large batches: xArm6 and 17 boxes 266 against 322 us for
+        // 1,000,003 configurations, 148 against 146 for 262,147, 114
+        // against 104 for 5,909 (10-DOF chain 405 / 423, 209 / 178 and 140
+        // / 125).  Where they order the whole pose (at most 3 joints) they
+        // pay early, unless the walk is short: planar arm, 40 boxes 108
+        // against 164 us for 65,536; 4 boxes 130 against 102 for 1,000,003.
+        const int64_t from = (int64_t)links * objects < 32 ? INT64_MAX : (dofs <= 3 ? 1024 : 1 << 18);
+        return FastTuning{0, 64, 0, n >= from ? 5 : 0};
+    }
+    // Long walks.  Link-major launches (4) against lane refill (1), 22-DOF
+    // chain: 512 boxes 5.9 against 11.7 ms for 2,097,152 configurations and
+    // 2.1 against 2.5 ms for 1,000; 256 boxes 3.5 against 5.0 ms for
+    // 1,000,000 and 1.2 against 1.6 for 1,000; 128 boxes 3.5 against 3.8 ms
+    // for 1,000,000 but 1.64 against 1.58 for 300,000; 96 boxes 3.4 against
+    // 3.2.  Their lists take 128 bytes a configuration: at most 2 GiB.
+    if (lists && n <= (int64_t)1 << 24 && (objects >= 200 || (objects >= 128 && n >= (int64_t)1 << 19)))
+        return FastTuning{4, 512, 0, 5};
+    // Lane refill with pair queues (3) for small batches: 22-DOF chain and
+    // 96 boxes 0.64 against 0.77 ms for 1,000 and 0.73 against 0.85 for
+    // 30,000; 14-DOF chain and 65 boxes 0.40 against 0.46 for 100,000; but
+    // 18-DOF chain and 80 boxes 1.17 against 1.03 for 400,000.
+    // Where the lists cannot be had (the static and served calls hold none),
+    // the queues also serve larger batches of long chains among many
+    // obstacles: 22-DOF chain and 200 boxes 4.3 against 5.2 ms for 1,000,000,
+    // 512 boxes 8.2 against 8.9; but 6-DOF arm and 600 boxes 1.59 against 1.35
+    // ms, 10-DOF chain and 160 boxes 1.18 against 1.09, 12-DOF chain and 280
+    // boxes 1.42 against 1.32 for 400,000.
+    if (n <= (int64_t)1 << 17 || (!lists && links >= 14 && objects >= 200)) return FastTuning{3, 512, 0, 5};
+    return FastTuning{1, 256, 0, 5};
+}
+
 }  // namespace rvs
 
 // The opaque handle of include/rvs.h.
@@ -147,39 +185,15 @@ struct rvs_context {
     uint32_t* count_dev = nullptr;    // the same word's device address
     std::mutex tuning_mu;
     // The launch shape of an RVS_PREC_FP32_REFINE batch of n configurations:
-    // the recorded one, else by the length of the walk and the batch (every
-    // shape gives the same bits, so the choice may follow n).
-    rvs::FastTuning tuning_for(int32_t robot, int32_t env, int32_t dofs, int32_t links, int32_t objects, int64_t n) {
+    // the recorded one, else default_shape's.
+    rvs::FastTuning tuning_for(int32_t robot, int32_t env, int32_t dofs, int32_t links, int32_t objects, int64_t n,
+                               bool lists = true) {
         std::lock_guard<std::mutex> lk(tuning_mu);
         auto it = tuning.find({robot, env});
         if (it != tuning.end()) return it->second;
         // one lane per configuration: 64-thread workgroups measured fastest
         if (fast_variant >= 0) return rvs::FastTuning{fast_variant, fast_variant == 0 ? 64 : 256, 0, 5};
-        if ((int64_t)links * objects < 1024) {
-            // The walk order's four kernels (16 to 31 us) pay for themselves
-            // in large batches: xArm6 and 17 boxes 266 against 322 us for
-            // 1,000,003 configurations, 148 against 146 for 262,147, 114
-            // against 104 for 5,909 (10-DOF chain 405 / 423, 209 / 178 and 140
-            // / 125).  Where they order the whole pose (at most 3 joints) they
-            // pay early, unless the walk is short: planar arm, 40 boxes 108
-            // against 164 us for 65,536; 4 boxes 130 against 102 for 1,000,003.
-            const int64_t from = (int64_t)links * objects < 32 ? INT64_MAX : (dofs <= 3 ? 1024 : 1 << 18);
-            return rvs::FastTuning{0, 64, 0, n >= from ? 5 : 0};
-        }
-        // Long walks.  Link-major launches (4) against lane refill (1), 22-DOF
-        // chain: 512 boxes 5.9 against 11.7 ms for 2,097,152 configurations and
-        // 2.1 against 2.5 ms for 1,000; 256 boxes 3.5 against 5.0 ms for
-        // 1,000,000 and 1.2 against 1.6 for 1,000; 128 boxes 3.5 against 3.8 ms
-        // for 1,000,000 but 1.64 against 1.58 for 300,000; 96 boxes 3.4 against
-        // 3.2.  Their lists take 128 bytes a configuration: at most 2 GiB.
-        if (n <= (int64_t)1 << 24 && (objects >= 200 || (objects >= 128 && n >= (int64_t)1 << 19)))
-            return rvs::FastTuning{4, 512, 0, 5};
-        // Lane refill with pair queues (3) for small batches: 22-DOF chain and
-        // 96 boxes 0.64 against 0.77 ms for 1,000 and 0.73 against 0.85 for
-        // 30,000; 14-DOF chain and 65 boxes 0.40 against 0.46 for 100,000; but
-        // 18-DOF chain and 80 boxes 1.17 against 1.03 for 400,000.
-        if (n <= (int64_t)1 << 17) return rvs::FastTuning{3, 512, 0, 5};
-        return rvs::FastTuning{1, 256, 0, 5};
+        return rvs::default_shape(dofs, links, objects, n, lists);
     }
     // Walk-order bits of the exact paths: a recorded shape's, else 5.
     int32_t order_bits(int32_t robot, int32_t env) {

@@ -293,10 +293,10 @@ hipError_t issue(rvs_server* s, Batch& b, const Layout& lay) {
         out.verdict = flag;
         const int prec = s->opt.precision;
         if (prec == RVS_PREC_FP32_REFINE) {
-            const FastTuning ft = s->ctx->tuning_for(h.r.robot, h.r.env, D, L, M, N);
+            const FastTuning ft = s->ctx->tuning_for(h.r.robot, h.r.env, D, L, M, N, false);
             if (e == hipSuccess) e = launch_zero_u32(count, 64, st);
             if (e == hipSuccess)
-                // order given; no links scratch (a link-major shape runs as variant 3)
+                // order given; no lists (a recorded link-major shape runs as variant 3)
                 e = launch_distance_fast(rb, env, s->qp, q, N, out, idx, count, ft, nullptr, nullptr, s->ctx->num_cus,
                                          st);
             if (e == hipSuccess) e = launch_distance_refine(rb, env, s->qp, q, N, out, idx, count, st);

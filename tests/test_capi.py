@@ -76,6 +76,17 @@ def test_device_geometry_source_matches_oracle_on_host():
     assert "flat=0 " in r.stdout
 
 
+def test_default_launch_shapes():
+    """Shapes chosen without a recorded one: their needs can be met, and the
+    measured points get the shape that was faster there."""
+    exe = os.path.join(ROOT, "tests", "host", "_build", "shape_check")
+    if not os.path.exists(exe):
+        subprocess.run(["make", "-C", os.path.join(ROOT, "tests", "host")], check=True, capture_output=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    print(r.stdout)
+    assert r.returncode == 0 and "shape_check: 0 wrong" in r.stdout
+
+
 def test_workloads_deterministic_and_in_spec():
     a, b = W.workload2(5000), W.workload2(5000)
     assert np.array_equal(a.q, b.q) and np.array_equal(a.scene.aabb, b.scene.aabb)
