@@ -107,26 +107,52 @@ inline FastTuning default_shape(int32_t dofs, int32_t links, int32_t objects, in
         const int64_t from = (int64_t)links * objects < 32 ? INT64_MAX : (dofs <= 3 ? 1024 : 1 << 18);
         return FastTuning{0, 64, 0, n >= from ? 5 : 0};
     }
-    // Long walks.  Link-major launches (4) against lane refill (1), 22-DOF
-    // chain: 512 boxes 5.9 against 11.7 ms for 2,097,152 configurations and
-    // 2.1 against 2.5 ms for 1,000; 256 boxes 3.5 against 5.0 ms for
-    // 1,000,000 and 1.2 against 1.6 for 1,000; 128 boxes 3.5 against 3.8 ms
-    // for 1,000,000 but 1.64 against 1.58 for 300,000; 96 boxes 3.4 against
-    // 3.2.  Their lists take 128 bytes a configuration: at most 2 GiB.
-    if (lists && n <= (int64_t)1 << 24 && (objects >= 200 || (objects >= 128 && n >= (int64_t)1 << 19)))
-        return FastTuning{4, 512, 0, 5};
-    // Lane refill with pair queues (3) for small batches: 22-DOF chain and
-    // 96 boxes 0.64 against 0.77 ms for 1,000 and 0.73 against 0.85 for
-    // 30,000; 14-DOF chain and 65 boxes 0.40 against 0.46 for 100,000; but
-    // 18-DOF chain and 80 boxes 1.17 against 1.03 for 400,000.
-    // Where the lists cannot be had (the static and served calls hold none),
-    // the queues also serve larger batches of long chains among many
-    // obstacles: 22-DOF chain and 200 boxes 4.3 against 5.2 ms for 1,000,000,
-    // 512 boxes 8.2 against 8.9; but 6-DOF arm and 600 boxes 1.59 against 1.35
-    // ms, 10-DOF chain and 160 boxes 1.18 against 1.09, 12-DOF chain and 280
-    // boxes 1.42 against 1.32 for 400,000.
-    if (n <= (int64_t)1 << 17 || (!lists && links >= 14 && objects >= 200)) return FastTuning{3, 512, 0, 5};
-    return FastTuning{1, 256, 0, 5};
+    // Long walks: lane refill (1), the same with pair queues (3), or link-major
+    // launches (4), whose lists take 128 bytes a configuration, at most 2 GiB.
+    // A handful of configurations share nothing: lane refill for 1 and 10
+    // among fewer than 400 boxes (or without lists) 133 and 187 against 164 and
+    // 209 us with queues (10-DOF chain, 130 boxes), 257 and 607 against 288 and
+    // 846 link by link (22-DOF chain, 256 boxes); among 512 boxes 427 and 1,340
+    // against 344 and 1,260 link by link.
+    const FastTuning refill{1, 256, 0, 5}, queues{3, 512, 0, 5}, by_link{4, 512, 0, 5};
+    lists = lists && n <= (int64_t)1 << 24;
+    if (n <= 16 && (objects < 400 || !lists)) return refill;
+    // Refill, queues and link by link, us a call.  Arms of up to 7 links (6-DOF
+    // arm): 200 boxes 307, 278 and 254 for 1,000 configurations, 482, 513 and
+    // 506 for 400,000; 300 boxes 321, 337 and 282, and 941, 1,075 and 921 for
+    // 1,000,000 (200,000: 467 and 441); 1,000 boxes 2,524, 2,672 and 969.
+    if (links < 8) {
+        if (lists && (objects >= 320 || (objects >= 200 && n < (int64_t)1 << 18))) return by_link;
+        return n < (int64_t)1 << 18 ? queues : refill;
+    }
+    // 8 to 11 links (10-DOF chain): 130 boxes 229, 244 and 307 for 1,000, 957,
+    // 1,042 and 1,224 for 1,000,000; 200 boxes 445, 420 and 395 for 30,000; 256
+    // boxes 378, 464 and 419, and 1,331, 1,534 and 1,340 for 1,000,000; 700
+    // boxes 972, 860 and 436 for 1,000, 3,372, 3,455 and 1,657 for 1,000,000.
+    if (links < 12) {
+        if (lists && objects >= 200) return by_link;
+        return objects >= 600 && n < (int64_t)1 << 19 ? queues : refill;
+    }
+    // Longer chains:
+    //                     1,000               130,000             400,000             1,000,000
+    //   14 DOF,  80 boxes   389   331   452     502   449   636     845   791 1,126   1,574 1,639 1,937
+    //   14 DOF, 160 boxes   628   540   617     752   653   790   1,238 1,145 1,379   2,403 2,287 2,401
+    //   14 DOF, 256 boxes   763   678   647     952   850   889   1,490 1,517 1,484   3,068 2,961 2,484
+    //   22 DOF,  96 boxes   830   633   804   1,038   835 1,116   1,614 1,433 1,932   3,269 3,279 3,491
+    //   22 DOF, 128 boxes   855   748   902     976   899 1,146   1,620 1,623 2,008   3,383 3,519 3,578
+    //   22 DOF, 200 boxes 1,319 1,128 1,111   1,420 1,234 1,403   2,240 2,157 2,297   4,742 4,128 3,865
+    //   22 DOF, 512 boxes 2,770 2,287 1,922   2,974 2,503 2,405   5,516 4,579 3,657  10,955 8,794 6,458
+    //   40 DOF, 256 boxes 2,475 2,225 2,172   2,801 2,519 2,834   4,540 4,148 4,029
+    //   40 DOF, 400 boxes 3,703 3,148 2,958   3,863 3,422 3,617   6,443 5,577 4,881
+    // so link by link from more obstacles on the longer the chain, and earlier
+    // in batches that are large or too small to fill the card with queues (200
+    // boxes, 300 configurations: 14 DOF 722, 589 and 556, 22 DOF 1,303, 1,012
+    // and 956); queues in small batches and from 160 boxes on.
+    if (lists && (objects >= 100 + 8 * links || (objects >= 176 && n >= (int64_t)1 << 19) ||
+                  (objects >= 240 && n >= (int64_t)1 << 18) || (objects >= 200 && n <= 1024)))
+        return by_link;
+    if (n <= (int64_t)1 << 17 || objects >= 160) return queues;
+    return refill;
 }
 
 }  // namespace rvs

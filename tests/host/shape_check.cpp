@@ -42,10 +42,17 @@ int main() {
         {40, 200, 400000, false, 3}, {22, 200, 30000, false, 3}, {22, 128, 30000, false, 3},
         // ... and lane refill for short ones, and among fewer obstacles
         {6, 200, 400000, false, 1}, {6, 600, 1000000, false, 1}, {10, 160, 1000000, false, 1},
-        {12, 280, 400000, false, 1}, {22, 128, 1000000, false, 1}, {14, 130, 1000000, false, 1},
+        {22, 128, 1000000, false, 1}, {14, 130, 1000000, false, 1},
         // link-major launches
-        {22, 512, 1000, true, 4}, {22, 512, 2097152, true, 4}, {22, 128, 1000000, true, 4}, {14, 512, 30000, true, 4},
-        {6, 1000, 1000000, true, 4},
+        {22, 512, 1000, true, 4}, {22, 512, 2097152, true, 4}, {22, 200, 1000000, true, 4}, {14, 512, 30000, true, 4},
+        {6, 1000, 1000000, true, 4}, {6, 200, 1000, true, 4}, {10, 400, 1000000, true, 4}, {14, 256, 1000, true, 4},
+        {40, 400, 400000, true, 4}, {22, 512, 1, true, 4},
+        // ... not for short chains or few obstacles
+        {10, 130, 1000000, true, 1}, {10, 300, 30000, false, 1}, {10, 700, 30000, false, 3}, {6, 200, 1000000, true, 1}, {22, 200, 30000, true, 3},
+        {40, 256, 30000, true, 3}, {22, 96, 400000, true, 1}, {22, 128, 1000000, true, 1}, {22, 96, 30000, true, 3}, {14, 160, 1000000, true, 3},
+        // a handful of configurations
+        {22, 256, 1, true, 1}, {22, 256, 10, true, 1}, {10, 130, 10, true, 1}, {40, 150, 10, true, 1},
+        {22, 512, 1, false, 1}, {6, 1000, 10, false, 1},
     };
     for (const auto& p : point) {
         const FastTuning t = default_shape(p.links, p.links, p.objects, p.n, p.lists);
