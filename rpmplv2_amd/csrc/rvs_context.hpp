@@ -97,14 +97,27 @@ struct EnvRec {
 // can have the link-major pass's scratch (fast_links_bytes).
 inline FastTuning default_shape(int32_t dofs, int32_t links, int32_t objects, int64_t n, bool lists) {
     if ((int64_t)links * objects < 1024) {
-        // The walk order's four kernels (16 to 31 us) pay for themselves
-        // in large batches: xArm6 and 17 boxes 266 against 322 us for
-        // 1,000,003 configurations, 148 against 146 for 262,147, 114
-        // against 104 for 5,909 (10-DOF chain 405 / 423, 209 / 178 and 140
-        // / 125).  Where they order the whole pose (at most 3 joints) they
-        // pay early, unless the walk is short: planar arm, 40 boxes 108
-        // against 164 us for 65,536; 4 boxes 130 against 102 for 1,000,003.
-        const int64_t from = (int64_t)links * objects < 32 ? INT64_MAX : (dofs <= 3 ? 1024 : 1 << 18);
+        // The walk order's four kernels (16 to 31 us) pay for themselves in
+        // large batches, the earlier the longer the walk.  Sorted against
+        // unsorted, us a call: xArm6 and 17 boxes 266 / 322 for 1,000,003
+        // configurations, 120 / 101 for 260,000, 88 / 72 for 4,000; 80 boxes 233
+        // / 228 for 260,000, 177 / 177 for 80,000; 120 boxes 189 / 197 for
+        // 16,000, 242 / 282 for 200,000; 160 boxes 243 / 254 for 130,000; 14-DOF
+        // chain and 70 boxes 412 / 419 and 473 / 546 for 130,000 and 200,000;
+        // 10-DOF chain and 100 boxes 274 / 251 and 319 / 328.  Fewer than 32
+        // pairs: never (xArm6 and 5 boxes 553 / 375 for 4,000,000, 22-DOF chain
+        // and one box 737 / 533 for 1,000,000).
+        // Where they order the whole pose (at most 3 joints) they pay early,
+        // unless the walk is short: planar arm, 40 boxes 108 / 164 for 65,536;
+        // 15 boxes 83 / 75 for 300,000 and 123 / 138 for 1,000,000; 4 boxes 130
+        // / 102 for 1,000,003.
+        const int64_t pairs = (int64_t)links * objects;
+        int64_t from = INT64_MAX;
+        if (dofs <= 3) {
+            if (pairs >= 24) from = pairs >= 32 ? 1024 : 1 << 19;
+        } else if (pairs >= 32) {
+            from = objects >= 112 ? 1 << 14 : (pairs >= 700 ? 5 << 15 : 1 << 18);
+        }
         return FastTuning{0, 64, 0, n >= from ? 5 : 0};
     }
     // Long walks: lane refill (1), the same with pair queues (3), or link-major

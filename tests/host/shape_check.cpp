@@ -58,6 +58,20 @@ int main() {
         const FastTuning t = default_shape(p.links, p.links, p.objects, p.n, p.lists);
         need(t.variant == p.variant, "measured faster", p.links, p.objects, p.n, p.lists, t);
     }
+    const struct {
+        int dofs, links, objects;
+        long n;
+        bool sorted;
+    } order[] = {
+        {6, 6, 17, 1000003, true}, {6, 6, 17, 260000, false}, {6, 6, 17, 4000, false}, {10, 10, 60, 200000, false},
+        {6, 6, 120, 40000, true}, {6, 6, 160, 200000, true}, {14, 14, 70, 200000, true}, {14, 14, 40, 200000, false},
+        {22, 22, 1, 1000000, false}, {6, 6, 5, 4000000, false},
+        {2, 2, 40, 65536, true}, {2, 2, 15, 1000000, true}, {2, 2, 15, 130000, false}, {2, 2, 4, 1000003, false},
+    };
+    for (const auto& p : order) {
+        const FastTuning t = default_shape(p.dofs, p.links, p.objects, p.n, true);
+        need((t.coh_bits > 0) == p.sorted, "measured faster", p.links, p.objects, p.n, true, t);
+    }
     printf("shape_check: %d wrong\n", bad);
     return bad ? 1 : 0;
 }
