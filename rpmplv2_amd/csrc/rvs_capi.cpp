@@ -1745,7 +1745,7 @@ rvs_status rvs_extend_spines(rvs_context* c, int32_t robot, const float* q, cons
         a.profile = np ? ps : ds;
         a.q_e = es;
     }
-    if (e == hipSuccess) e = launch_spines(rb.dev, a, n, c->stream);
+    if (e == hipSuccess) e = launch_spines(rb.dev, a, n, c->num_cus, c->stream);
     if (e == hipSuccess && !(flags & RVS_F_DEVICE)) {
         e = d2h(q_new, a.q_new, (size_t)n * D * 4, c->stream);
         if (e == hipSuccess) e = d2h(status, a.status, (size_t)n * 4, c->stream);
@@ -1827,7 +1827,7 @@ rvs_status rvs_extend_gen_spines(rvs_context* c, int32_t robot, int32_t env, con
         g.expanded = use_expanded_bubble ? 1 : 0;
         g.d_crit = d_crit;
         g.maxd = qp.maxd;
-        if (e == hipSuccess) e = launch_gen_spines_under(rb.dev, g, n, c->stream);
+        if (e == hipSuccess) e = launch_gen_spines_under(rb.dev, g, n, c->num_cus, c->stream);
     } else if (e == hipSuccess) {
         e = launch_fill_u8(active, n, 1, c->stream);
     }
@@ -1848,7 +1848,7 @@ rvs_status rvs_extend_gen_spines(rvs_context* c, int32_t robot, int32_t env, con
         a.status = st;
         a.num_iter = num_iter;
         a.expanded = use_expanded_bubble ? 1 : 0;
-        e = launch_spines(rb.dev, a, n, c->stream);
+        e = launch_spines(rb.dev, a, n, c->num_cus, c->stream);
         if (e != hipSuccess) break;
         e = launch_distance_ref32_auto(rb.dev, ev.dev, qp, qn, n, lo, c->wave_max, c->stream);
         if (e == hipSuccess) e = launch_gen_layer(n, layer, d_root, d_layer, st, active, dd, d_crit, c->stream);

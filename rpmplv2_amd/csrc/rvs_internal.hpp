@@ -372,7 +372,7 @@ struct SpineArgs {
     int32_t num_iter;
     int32_t expanded;
 };
-hipError_t launch_spines(const RobotDev& rb, const SpineArgs& a, int64_t n, hipStream_t st);
+hipError_t launch_spines(const RobotDev& rb, const SpineArgs& a, int64_t n, int num_cus, hipStream_t st);
 // Generalized spines with underestimation layers, fused (device pointers):
 // root state, its distance [1], profile [L] and nearest points [M][L][6];
 // targets q_e [N][n]; outputs q_new [N][n], status [N], d_out [N].
@@ -392,7 +392,8 @@ struct GenSpineArgs {
     float d_crit;
     float maxd;
 };
-hipError_t launch_gen_spines_under(const RobotDev& rb, const GenSpineArgs& g, int64_t n, hipStream_t st);
+hipError_t launch_gen_spines_under(const RobotDev& rb, const GenSpineArgs& g, int64_t n, int num_cus,
+                                   hipStream_t st);
 // Between layers of generalized spines: d_out = d_layer and deactivation of
 // spines with d_layer < d_crit or status != advanced (layer 0: a root in
 // contact stops every spine with the root's distance).

@@ -32,6 +32,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "rvs_fk.hpp"
 #include "rvs_geometry.hpp"
@@ -47,8 +48,8 @@ constexpr int32_t kAdvanced = 1, kTrapped = 2, kReached = 3;
 
 // Floats of one lane's LDS slice: skeleton of the start state and of the
 // current state (3 (D+1) each), radii column, current state, clearance
-// losses, joint distances to the target (D each).
-__host__ __device__ inline int spine_slice(int D) { return 6 * (D + 1) + 4 * D; }
+// losses (D each), and with `dl` the joint distances to the target (D).
+__host__ __device__ inline int spine_slice(int D, bool dl) { return 6 * (D + 1) + (dl ? 4 : 3) * D; }
 
 // One lane's view of its LDS slice.
 struct SpineLane {
@@ -84,7 +85,7 @@ struct SpineLane {
 // extendSpine from the state in the lane's Q, whose skeleton is in sk0
 // (distance dq, link profile pc(i)), towards qe; Q holds q_new afterwards.
 // Returns the status.
-template <typename PC>
+template <bool DL, typename PC>
 __device__ int32_t spine_run(const RobotDev& rb, const SpineLane& s, float dq, PC pc, const float* qe,
                              int num_iter, int expanded) {
     const int D = rb.num_dofs;
@@ -100,11 +101,11 @@ __device__ int32_t spine_run(const RobotDev& rb, const SpineLane& s, float dq, P
     for (int it = 1;; ++it) {
         for (int i = 0; i < D; ++i) {
             s.acc(i) = 0.0f;
-            s.DL(i) = fabsf(qe[i] - s.Q(i));
+            if (DL) s.DL(i) = fabsf(qe[i] - s.Q(i));
         }
         // covered distance of skeleton point j: R.col(j).dot(|q_e - q_temp|)
         auto covered = [&]() {
-            return eigen_dyn_sum([&](int i) { return s.acc(i) * s.DL(i); }, D);
+            return eigen_dyn_sum([&](int i) { return s.acc(i) * (DL ? s.DL(i) : fabsf(qe[i] - s.Q(i))); }, D);
         };
         float step = INFINITY;
         for (int j = 1; j <= D; ++j) {
@@ -137,6 +138,7 @@ __device__ int32_t spine_run(const RobotDev& rb, const SpineLane& s, float dq, P
     return status;
 }
 
+template <bool DL>
 __global__ __launch_bounds__(64) void k_spines(RobotDev rb, SpineArgs a, int64_t n) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int D = rb.num_dofs;
@@ -152,7 +154,7 @@ __global__ __launch_bounds__(64) void k_spines(RobotDev rb, SpineArgs a, int64_t
     fk_init(fk);
     for (int k = 0; k <= D; ++k) s.set_P(s.sk0, k, skel_point<float>(fk, rb, s.qt + s.t, k, s.B));
     const int32_t status =
-        spine_run(rb, s, a.d[c * a.d_stride], [&](int i) { return pc[i]; }, a.q_e + c * D, a.num_iter, a.expanded);
+        spine_run<DL>(rb, s, a.d[c * a.d_stride], [&](int i) { return pc[i]; }, a.q_e + c * D, a.num_iter, a.expanded);
     float* qn = a.q_new + c * D;
     for (int k = 0; k < D; ++k) qn[k] = s.Q(k);
     a.status[c] = status;
@@ -175,6 +177,7 @@ __global__ __launch_bounds__(64) void k_spines(RobotDev rb, SpineArgs a, int64_t
 // distance included: 354 to 153 us a call).
 // A workgroup is one wave; its lanes go through the layers together, finished
 // ones masked off, so that all of them stage.
+template <bool DL>
 __global__ __launch_bounds__(64) void k_gen_spines_under(RobotDev rb, GenSpineArgs g, int64_t n, int tile) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int D = rb.num_dofs, L = rb.num_links, M = g.num_obj;
@@ -182,7 +185,7 @@ __global__ __launch_bounds__(64) void k_gen_spines_under(RobotDev rb, GenSpineAr
     Plane* planes = reinterpret_cast<Plane*>(smem);   // [tile][M]
     float* base = reinterpret_cast<float*>(smem + (size_t)tile * M * sizeof(Plane));
     const SpineLane s(base, D, B, t);
-    float* pr = base + (size_t)spine_slice(D) * B;    // [L][B]
+    float* pr = base + (size_t)spine_slice(D, DL) * B;    // [L][B]
     auto PR = [&](int k) -> float& { return pr[k * B + t]; };
     const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = c < n;
@@ -205,7 +208,7 @@ __global__ __launch_bounds__(64) void k_gen_spines_under(RobotDev rb, GenSpineAr
     }
     for (int layer = 0; layer < g.num_layers; ++layer) {
         if (!__any(on)) break;   // uniform: the workgroup is one wave
-        if (on) status = spine_run(rb, s, d_out, [&](int i) { return PR(i); }, qe, g.num_iter, g.expanded);
+        if (on) status = spine_run<DL>(rb, s, d_out, [&](int i) { return PR(i); }, qe, g.num_iter, g.expanded);
         // computeDistanceUnderestimation(q_new, root nearest points)
         FKStream fk;
         fk_init(fk);
@@ -384,35 +387,70 @@ __global__ __launch_bounds__(64) void k_edge_self(RobotDev rb, QueryParams qp, c
 
 }  // namespace
 
-size_t spine_lds_per_lane(const RobotDev& rb) { return (size_t)spine_slice(rb.num_dofs) * sizeof(float); }
+namespace {
 
-int spine_block(const RobotDev& rb) {
-    const size_t per = spine_lds_per_lane(rb);
-    int B = 64;
-    while (B > 16 && per * B > 64 * 1024) B /= 2;
-    return B;
+// Rounds of workgroups that n lanes take, B lanes and `bytes` of LDS to a
+// workgroup (a CU has 160 KB, handed out in pieces of 1,280 bytes); whole ones
+// up to two, after which the workgroups no longer end together.
+double spine_rounds(int64_t n, int B, size_t bytes, int num_cus) {
+    const size_t held = std::max<size_t>(1, (size_t)160 * 1024 / ((bytes + 1279) / 1280 * 1280));
+    const double r = (double)n / ((double)held * B * std::max(1, num_cus));
+    return r > 2 ? r : std::ceil(r);
 }
 
-hipError_t launch_spines(const RobotDev& rb, const SpineArgs& a, int64_t n, hipStream_t st) {
+}  // namespace
+
+// The joint distances to the target kept in LDS instead of worked out at each
+// use save 4 to 7% (65,536 xArm6 spines of 5 iterations 67 against 69 us, 22-DOF
+// chains 784 against 828), unless their share of LDS costs a CU a workgroup
+// that the batch needs (16-DOF chains, 65,536: 459 against 262 us; 22-DOF,
+// 45,000: 757 against 433; 32-DOF, 30,000: 1,514 against 766; xArm6, 600,000:
+// 357 against 341).  Two workgroups of 80 KB fill a CU as well as four of half
+// the lanes (30-DOF chains, 30,000: 658 against 669 us).
+hipError_t launch_spines(const RobotDev& rb, const SpineArgs& a, int64_t n, int num_cus, hipStream_t st) {
     if (n <= 0) return hipSuccess;
-    const int B = spine_block(rb);
-    const size_t sm = spine_lds_per_lane(rb) * B;
-    hipLaunchKernelGGL(k_spines, dim3((unsigned)((n + B - 1) / B)), dim3(B), sm, st, rb, a, n);
+    const size_t room = std::min<size_t>(80 * 1024, device_lds_limit());
+    int B[2];
+    size_t bytes[2];
+    double rounds[2];
+    for (int dl = 0; dl < 2; ++dl) {
+        const size_t per = (size_t)spine_slice(rb.num_dofs, dl) * sizeof(float);
+        B[dl] = 64;
+        while (B[dl] > 16 && per * B[dl] > room) B[dl] /= 2;
+        bytes[dl] = per * B[dl];
+        rounds[dl] = spine_rounds(n, B[dl], bytes[dl], num_cus);
+    }
+    const int dl = rounds[1] <= rounds[0] ? 1 : 0;
+    const dim3 grid((unsigned)((n + B[dl] - 1) / B[dl])), block(B[dl]);
+    if (dl) hipLaunchKernelGGL(k_spines<true>, grid, block, bytes[dl], st, rb, a, n);
+    else hipLaunchKernelGGL(k_spines<false>, grid, block, bytes[dl], st, rb, a, n);
     return hipGetLastError();
 }
 
-hipError_t launch_gen_spines_under(const RobotDev& rb, const GenSpineArgs& g, int64_t n, hipStream_t st) {
+// The same choice (64-DOF chains, 5 boxes, 65,536 spines 28.1 ms with the joint
+// distances, 19.2 without; 22-DOF chains, 100 boxes 5.5 and 2.8 ms).
+hipError_t launch_gen_spines_under(const RobotDev& rb, const GenSpineArgs& g, int64_t n, int num_cus,
+                                   hipStream_t st) {
     if (n <= 0) return hipSuccess;
     // 64 KB of LDS: the lanes' slices (fewer lanes for long chains), beside
     // at least one link's planes and as many links' as fit
-    const size_t per = spine_lds_per_lane(rb) + (size_t)rb.num_links * sizeof(float);
     const size_t link = (size_t)std::max(1, (int)g.num_obj) * sizeof(Plane);
     const size_t room = 64 * 1024;
-    int B = 64;
-    while (B > 1 && per * B + link > room) B /= 2;
-    const int tile = (int)std::min<size_t>((size_t)rb.num_links, std::max<size_t>(1, (room - per * B) / link));
-    hipLaunchKernelGGL(k_gen_spines_under, dim3((unsigned)((n + B - 1) / B)), dim3(B),
-                       (size_t)tile * g.num_obj * sizeof(Plane) + per * B, st, rb, g, n, tile);
+    int B[2], tile[2];
+    size_t bytes[2];
+    double rounds[2];
+    for (int dl = 0; dl < 2; ++dl) {
+        const size_t per = ((size_t)spine_slice(rb.num_dofs, dl) + (size_t)rb.num_links) * sizeof(float);
+        B[dl] = 64;
+        while (B[dl] > 1 && per * B[dl] + link > room) B[dl] /= 2;
+        tile[dl] = (int)std::min<size_t>((size_t)rb.num_links, std::max<size_t>(1, (room - per * B[dl]) / link));
+        bytes[dl] = (size_t)tile[dl] * g.num_obj * sizeof(Plane) + per * B[dl];
+        rounds[dl] = spine_rounds(n, B[dl], bytes[dl], num_cus);
+    }
+    const int dl = rounds[1] <= rounds[0] ? 1 : 0;
+    const dim3 grid((unsigned)((n + B[dl] - 1) / B[dl])), block(B[dl]);
+    if (dl) hipLaunchKernelGGL(k_gen_spines_under<true>, grid, block, bytes[dl], st, rb, g, n, tile[dl]);
+    else hipLaunchKernelGGL(k_gen_spines_under<false>, grid, block, bytes[dl], st, rb, g, n, tile[dl]);
     return hipGetLastError();
 }
 

@@ -114,6 +114,23 @@ def test_underestimation(oracle, engine):
     assert ulps(d2, ud2).max() <= 2
 
 
+def _boxes_around(rng, rb, count, side_lo, side_hi, reach, clearance=0.02):
+    """Boxes in a ball of `reach` around the middle of the zero pose's
+    skeleton, their bounding balls clear of it."""
+    P = R.skeleton_np(rb, np.zeros(rb.num_dofs))[0]
+    t = np.linspace(0.0, 1.0, 21)[:, None, None]
+    pts = (P[None, :-1] + t * (P[1:] - P[:-1])[None]).reshape(-1, 3)
+    gap = np.max(rb.radius) + clearance
+    rows = []
+    while len(rows) < count:
+        sc = W._boxes(rng, 4 * count + 8, side_lo, side_hi, reach, center=P.mean(0))
+        far = np.linalg.norm(sc.pos[:, None] - pts[None], axis=2).min(1) > 0.5 * np.linalg.norm(sc.dim, axis=1) + gap
+        rows += [k for k in zip(sc.dim[far], sc.pos[far])]
+    dim, pos = (np.array(x[:count]) for x in zip(*rows))
+    return W.Scene(dim, pos, np.tile([1.0, 0.0, 0.0, 0.0], (count, 1)), np.zeros(count, np.uint8),
+                   np.full(count, 1000.0, np.float32))
+
+
 @pytest.mark.parametrize("dofs,boxes,n,far", [(6, 1, 1, False), (6, 16, 255, False), (10, 40, 257, False),
                                               (22, 100, 300, False), (22, 1000, 65, False), (6, 17, 257, True),
                                               (22, 100, 300, True), (22, 1000, 65, True)])
@@ -769,6 +786,50 @@ def test_extend_spines(oracle, engine, which, num_iter, expanded):
     assert (st == 2).any() and (st == 1).any()
 
 
+@pytest.mark.parametrize("dofs,n", [(16, 60001), (26, 1000), (30, 20000), (32, 30000), (64, 20000)])
+def test_extend_spines_batch_forms(oracle, engine, dofs, n):
+    """The joint distances in LDS (small batches) or worked out at each use
+    (where they would cost resident workgroups), 64, 32 and 16 lanes a
+    workgroup: a batch equals its parts bit for bit, and its head the oracle."""
+    rng = np.random.default_rng(dofs)
+    rb = R.chain(rng.uniform(0.05, 0.2, dofs), radius=0.03)
+    q = rng.uniform(-0.5, 0.5, (n, dofs)).astype(np.float32)
+    v = rng.normal(size=(n, dofs))
+    q_e = (q + 2.0 * v / np.linalg.norm(v, axis=1, keepdims=True)).astype(np.float32)
+    d = rng.uniform(0.005, 0.5, n).astype(np.float32)
+    prof = (d[:, None] + rng.uniform(0, 0.3, (n, dofs))).astype(np.float32)
+    rid = engine.load_robot(rb)
+    qn, st = engine.extend_spines(rid, q, d, prof, q_e, num_iter=3)
+    parts = [engine.extend_spines(rid, q[k:k + 1900], d[k:k + 1900], prof[k:k + 1900], q_e[k:k + 1900], num_iter=3)
+             for k in range(0, n, 1900)]
+    assert np.array_equal(qn, np.concatenate([p[0] for p in parts]))
+    assert np.array_equal(st, np.concatenate([p[1] for p in parts]))
+    oqn, ost = oracle.extend_spines(rb, q[:300], d[:300], prof[:300], q_e[:300], num_iter=3)
+    assert np.array_equal(qn[:300], oqn) and np.array_equal(st[:300], ost)
+    assert (qn != q).any()
+
+
+@pytest.mark.parametrize("dofs,boxes,n", [(16, 20, 60001), (22, 100, 40000), (64, 5, 20000)])
+def test_extend_gen_spines_batch_forms(oracle, engine, dofs, boxes, n):
+    """The same for underestimation layers."""
+    rng = np.random.default_rng(dofs + boxes)
+    rb = R.chain(rng.uniform(0.05, 0.2, dofs), radius=0.02)
+    sc = _boxes_around(rng, rb, boxes, 0.05, 0.3, 0.08 * dofs, clearance=0.1)
+    root = np.zeros(dofs, np.float32)
+    v = rng.normal(size=(n, dofs))
+    q_e = (np.pi * v / np.linalg.norm(v, axis=1, keepdims=True)).astype(np.float32)
+    rid, eid = engine.load_robot(rb), engine.create_env(sc)
+    kw = dict(num_layers=3, num_iter=2, d_crit=0.01)
+    got = engine.extend_gen_spines(rid, eid, root, q_e, **kw)
+    parts = [engine.extend_gen_spines(rid, eid, root, q_e[k:k + 3900], **kw) for k in range(0, n, 3900)]
+    for i in range(3):
+        assert np.array_equal(got[i], np.concatenate([p[i] for p in parts]))
+    want = oracle.extend_gen_spines(rb, oracle.scene_of(sc), root, q_e[:200], **kw)
+    for g, o in zip(got, want):
+        assert np.array_equal(g[:200], o)
+    assert (got[2] > 0).any() and (got[0] != root).any()
+
+
 @pytest.mark.parametrize("use_real_dist", [False, True])
 @pytest.mark.parametrize("num_iter", [1, 5])
 def test_extend_gen_spines(oracle, engine, use_real_dist, num_iter):
@@ -1111,23 +1172,6 @@ def test_trajectory_is_safe_sizes(oracle, engine, dofs, boxes, points, traj, sel
     osafe = oracle.traj_safe(rb, osc, pts, root, p0[0], np0[0], mv, 0.1, dt,
                              pairs=rb.self_pairs if self_collision else None)
     assert np.array_equal(safe, osafe)
-
-
-def _boxes_around(rng, rb, count, side_lo, side_hi, reach, clearance=0.02):
-    """Boxes in a ball of `reach` around the middle of the zero pose's
-    skeleton, their bounding balls clear of it."""
-    P = R.skeleton_np(rb, np.zeros(rb.num_dofs))[0]
-    t = np.linspace(0.0, 1.0, 21)[:, None, None]
-    pts = (P[None, :-1] + t * (P[1:] - P[:-1])[None]).reshape(-1, 3)
-    gap = np.max(rb.radius) + clearance
-    rows = []
-    while len(rows) < count:
-        sc = W._boxes(rng, 4 * count + 8, side_lo, side_hi, reach, center=P.mean(0))
-        far = np.linalg.norm(sc.pos[:, None] - pts[None], axis=2).min(1) > 0.5 * np.linalg.norm(sc.dim, axis=1) + gap
-        rows += [k for k in zip(sc.dim[far], sc.pos[far])]
-    dim, pos = (np.array(x[:count]) for x in zip(*rows))
-    return W.Scene(dim, pos, np.tile([1.0, 0.0, 0.0, 0.0], (count, 1)), np.zeros(count, np.uint8),
-                   np.full(count, 1000.0, np.float32))
 
 
 @pytest.mark.parametrize("points", [1025, 2500])
