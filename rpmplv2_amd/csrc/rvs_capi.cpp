@@ -1157,7 +1157,7 @@ rvs_status rvs_self_collision_async(rvs_context* c, int32_t robot, const float* 
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c->stream;
     hipError_t e = async_begin(c, st);
     if (e == hipSuccess && n > 0)
-        e = launch_self_distance(rb.dev, params_of(c), q, n, nullptr, nullptr, min_dist, free_flag, st);
+        e = launch_self_distance(rb.dev, params_of(c), q, n, nullptr, min_dist, free_flag, st);
     if (e == hipSuccess) e = async_end(c, st, done);
     if (e != hipSuccess) return hip_fail(c, e, "rvs_self_collision_async");
     return RVS_OK;
@@ -1623,7 +1623,7 @@ rvs_status rvs_self_distance(rvs_context* c, int32_t robot, const float* q, int6
         e = h2d(qs, q, (size_t)n * D * 4, c->stream);
         qd = qs;
     }
-    if (e == hipSuccess) e = launch_self_distance(rb.dev, qp, qd, n, od, nullptr, nullptr, nullptr, c->stream);
+    if (e == hipSuccess) e = launch_self_distance(rb.dev, qp, qd, n, od, nullptr, nullptr, c->stream);
     if (e == hipSuccess && !(flags & RVS_F_DEVICE)) e = d2h(dist, od, (size_t)n * P * 4, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "rvs_self_distance");
@@ -1655,7 +1655,7 @@ rvs_status rvs_self_collision(rvs_context* c, int32_t robot, const float* q, int
         e = h2d(qs, q, (size_t)n * D * 4, c->stream);
         qd = qs;
     }
-    if (e == hipSuccess) e = launch_self_distance(rb.dev, qp, qd, n, nullptr, nullptr, md, fd, c->stream);
+    if (e == hipSuccess) e = launch_self_distance(rb.dev, qp, qd, n, nullptr, md, fd, c->stream);
     if (e == hipSuccess && !(flags & RVS_F_DEVICE)) {
         e = d2h(min_dist, md, min_dist ? (size_t)n * 4 : 0, c->stream);
         if (e == hipSuccess) e = d2h(free_flag, fd, free_flag ? (size_t)n : 0, c->stream);

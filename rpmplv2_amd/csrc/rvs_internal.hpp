@@ -425,9 +425,9 @@ size_t traj_lds_bytes(const RobotDev& rb);   // LDS of one trajectory's workgrou
 hipError_t launch_edge_self(const RobotDev& rb, const QueryParams& qp, const float* q1, const float* q2, int64_t n,
                             float eps_step, uint8_t* collide, float* q_out, hipStream_t st);
 
-// Per-pair distances (dist / dist64, [N][pairs]) and/or the per-configuration
-// minimum and collision-free flag (min_out / free_out); null outputs are skipped.
+// Per-pair distances (dist, [N][pairs]) and/or the per-configuration minimum
+// and collision-free flag (min_out / free_out); null outputs are skipped.
 hipError_t launch_self_distance(const RobotDev& rb, const QueryParams& qp, const float* q, int64_t n, float* dist,
-                                double* dist64, float* min_out, uint8_t* free_out, hipStream_t st);
+                                float* min_out, uint8_t* free_out, hipStream_t st);
 
 }  // namespace rvs

@@ -515,38 +515,36 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
 // distanceLineSegToLineSeg - r_a - r_b (xArm6::computeCapsulesDistance,
 // xArm6.cpp:417-424).  The skeleton of each lane is kept in LDS, one column
 // per lane.
-template <typename T>
 __global__ __launch_bounds__(128) void k_self(RobotDev rb, QueryParams qp, const float* __restrict__ q, int64_t n,
-                                              float* dist, double* dist64, float* min_out, uint8_t* free_out) {
+                                              float* dist, float* min_out, uint8_t* free_out) {
     extern __shared__ __align__(16) unsigned char smem[];
-    T* sk = reinterpret_cast<T*>(smem);
+    float* sk = reinterpret_cast<float*>(smem);
     const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= n) return;
     const int L = rb.num_links;
     const int B = blockDim.x, t = threadIdx.x;
     const float* qc = q + c * rb.num_dofs;
-    const Params<T> p{(T)qp.eq, (T)qp.maxd};
+    const Params<float> p{qp.eq, qp.maxd};
     FKStream fk;
     fk_init(fk);
     for (int k = 0; k <= L; ++k) {
-        const Vec3<T> P = skel_point<T>(fk, rb, qc, k);
+        const Vec3<float> P = skel_point<float>(fk, rb, qc, k);
         sk[(3 * k + 0) * B + t] = P.x;
         sk[(3 * k + 1) * B + t] = P.y;
         sk[(3 * k + 2) * B + t] = P.z;
     }
-    auto pt = [&](int k) { return Vec3<T>{sk[(3 * k) * B + t], sk[(3 * k + 1) * B + t], sk[(3 * k + 2) * B + t]}; };
+    auto pt = [&](int k) { return Vec3<float>{sk[(3 * k) * B + t], sk[(3 * k + 1) * B + t], sk[(3 * k + 2) * B + t]}; };
     // smallest pair distance in std::min order from MAX_DISTANCE (a NaN pair
     // distance never replaces the running minimum); colliding = some pair < 0
-    T lo = p.maxd;
+    float lo = p.maxd;
     for (int m = 0; m < rb.num_pairs; ++m) {
         const int a = rb.pairs[2 * m], b = rb.pairs[2 * m + 1];
-        const T sd = seg_seg<T, false>(pt(a), pt(a + 1), pt(b), pt(b + 1), p, nullptr);
-        const T v = sd - (T)rb.radius[a] - (T)rb.radius[b];
-        if (dist) dist[c * rb.num_pairs + m] = (float)v;
-        if (dist64) dist64[c * rb.num_pairs + m] = (double)v;
+        const float sd = seg_seg<float, false>(pt(a), pt(a + 1), pt(b), pt(b + 1), p, nullptr);
+        const float v = sd - rb.radius[a] - rb.radius[b];
+        if (dist) dist[c * rb.num_pairs + m] = v;
         lo = smin(lo, v);
     }
-    if (min_out) min_out[c] = (float)lo;
+    if (min_out) min_out[c] = lo;
     if (free_out) free_out[c] = lo < 0 ? 0 : 1;
 }
 
@@ -1005,23 +1003,27 @@ hipError_t launch_env_motion(const MotionDev& m, int64_t tick, float tick_second
     return hipGetLastError();
 }
 
+// The smallest pairs alone: k_self_min rules most pairs out but takes a wave
+// through its queue, so with few pairs k_self measures every one.  k_self
+// against k_self_min, us a call for 1,000 and 1,000,000 configurations: 4 pairs
+// (xArm6) 26.8 / 27.8 and 88 / 98, 10 pairs 32 / 38 and 132 / 155, 21 pairs 44
+// / 51 and 220 / 234, 36 pairs 60 / 67 and 353 / 338 (65,536: 75 / 71), 55 pairs
+// 79 / 79 and 503 / 449.  A few lanes rule out nearly all pairs, as none holds
+// up another: 16 configurations, 21 pairs 45 / 43, 36 pairs 62 / 59, one
+// configuration 44 / 31 and 59 / 35.
 hipError_t launch_self_distance(const RobotDev& rb, const QueryParams& qp, const float* q, int64_t n, float* dist,
-                                double* dist64, float* min_out, uint8_t* free_out, hipStream_t st) {
+                                float* min_out, uint8_t* free_out, hipStream_t st) {
     if (n <= 0) return hipSuccess;
-    if (!dist && !dist64) {
+    const int pairs = rb.num_pairs;
+    const bool every = dist || pairs < 8 ||
+                       (n > 16 && (pairs < 28 || (pairs < 48 && n > 64 && n < 65536)));
+    if (every) {
+        const int B = 128;
+        hipLaunchKernelGGL(k_self, grid_for(n, B), dim3(B), (size_t)3 * (rb.num_links + 1) * B * sizeof(float), st, rb,
+                           qp, q, n, dist, min_out, free_out);
+    } else {
         hipLaunchKernelGGL(k_self_min, grid_for(n, 64), dim3(64), self_min_lds(rb.num_links), st, rb, qp, q, n,
                            min_out, free_out);
-        return hipGetLastError();
-    }
-    const int B = 128;
-    if (dist64) {
-        const size_t sm = (size_t)3 * (rb.num_links + 1) * B * sizeof(double);
-        hipLaunchKernelGGL((k_self<double>), grid_for(n, B), dim3(B), sm, st, rb, qp, q, n, dist, dist64, min_out,
-                           free_out);
-    } else {
-        const size_t sm = (size_t)3 * (rb.num_links + 1) * B * sizeof(float);
-        hipLaunchKernelGGL((k_self<float>), grid_for(n, B), dim3(B), sm, st, rb, qp, q, n, dist, dist64, min_out,
-                           free_out);
     }
     return hipGetLastError();
 }

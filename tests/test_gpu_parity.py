@@ -1111,10 +1111,12 @@ def test_distances_by_pairs_sizes(engine, dofs, boxes, n, oriented):
 
 
 @pytest.mark.parametrize("dofs,n,scale", [(6, 1, 1.0), (6, 63, 1.0), (3, 65, 1.0), (22, 200, 1.0), (40, 130, 1.0),
-                                          (14, 70, 300.0), (14, 70, 1e-3)])
+                                          (14, 70, 300.0), (14, 70, 1e-3), (7, 16, 1.0), (7, 17, 1.0), (9, 64, 1.0),
+                                          (9, 65, 1.0), (9, 65536, 1.0)])
 def test_self_collision_minimum_of_pairs(engine, dofs, n, scale):
-    """The smallest pair distance, found without most of the pairs, against
-    the smallest of all of them, bit for bit: one pair to 741, radii that
+    """The smallest pair distance, found without most of the pairs (or, with
+    few, from every one: both sides of that rule's lines), against the
+    smallest of all of them, bit for bit: one pair to 741, radii that
     differ, pairs in no order and twice, long and tiny links (coordinates of a
     kilometre, links below the equality threshold), NaN and infinite joints,
     ragged waves."""
