@@ -424,8 +424,9 @@ rvs_status rvs_robot_load(rvs_context* c, const rvs_robot_desc* d, int32_t* robo
         pts[3].frame = 3; pts[3].axis = 2; pts[3].pre = -0.25; pts[3].flags = 1;
         pts[4].frame = 4;
         pts[5].frame = 4; pts[5].axis = 0; pts[5].pre = 0.076; pts[5].flags = 1;
-        pts[6].frame = 5; pts[6].axis = 2;
-        if (g != 0) { pts[6].pre = g; pts[6].post = 0.3 * g; pts[6].flags = 3; }
+        // the shift along the gripper's axis also without one, as the reference
+        // adds it: point 6 then takes joint 6 into account where that is no number
+        pts[6].frame = 5; pts[6].axis = 2; pts[6].pre = g; pts[6].post = 0.3 * g; pts[6].flags = 3;
     } else {
         return fail(c, RVS_EINVAL, "rvs_robot_load: unknown skeleton kind");
     }

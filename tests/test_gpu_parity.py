@@ -1280,6 +1280,34 @@ def test_is_valid_obstacle_marks(oracle, engine, dofs, boxes, n, oriented):
     assert np.array_equal(engine.is_valid(rid, eid, q, precision=rvs.PREC_FP64), oracle.is_valid(rb, osc, q, 64))
 
 
+@pytest.mark.parametrize("gripper", [0.0, 0.12])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_joint_that_is_no_number(oracle, engine, gripper, bad):
+    """One joint of an xArm6 NaN or infinite, each in turn: verdicts, flags and
+    first hits equal to the oracle's in every arithmetic."""
+    rng = np.random.default_rng(77)
+    rb = R.xarm6(gripper_length=gripper)
+    sc = _boxes_around(rng, rb, 40, 0.05, 0.3, 0.8)
+    osc = oracle.scene_of(sc)
+    n = 600
+    q = rng.uniform(-1.0, 1.0, (n, 6)).astype(np.float32)
+    q[np.arange(n), np.arange(n) % 6] = bad
+    rid, eid = engine.load_robot(rb), engine.create_env(sc, rvs.ENV_AABB)
+    od, oprof, over, _ = oracle.distance(rb, osc, q, 32)
+    assert all(0 < over[j::6].mean() < 1 for j in (4, 5))
+    for prec in (rvs.PREC_REF32, rvs.PREC_FP64, rvs.PREC_FP32_REFINE):
+        d, prof, ver, _ = engine.distance(rid, eid, q, precision=prec)
+        assert np.array_equal(ver, over), prec
+    assert np.array_equal(engine.is_valid(rid, eid, q), oracle.is_valid(rb, osc, q))
+    u = rng.normal(size=(n, 6))
+    u = (u / np.linalg.norm(u, axis=1, keepdims=True)).astype(np.float32)
+    K = np.full(n, 20, np.int32)
+    want = oracle.edge_first_collision(rb, osc, q, u, K, 0.05)
+    assert np.array_equal(engine.edge_first_collision(eid, np.full(n, rid, np.int32), q, u, K), want)
+    q2 = (q + 0.5 * u).astype(np.float32)
+    assert np.array_equal(engine.edge_is_valid(rid, eid, q, q2), oracle.edge_valid(rb, osc, q, q2))
+
+
 @pytest.mark.parametrize("n", [1, 17, 3639, 3640, 3700, 21500, 22700])
 def test_host_arrays_in_place_and_copied(engine, n):
     """Host arrays up to 1 MiB are used in place, larger ones copied: both give
