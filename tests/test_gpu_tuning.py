@@ -1,9 +1,7 @@
 """Autotuner of the FP32 bulk pass: every launch shape (one lane per
 configuration, lane refill, persistent chunks) and walk order gives the same
 per-configuration results (they only change which lane evaluates a
-configuration); the per-lane walks, which evaluate pairs without the case
-tree, give the same verdicts and distances within FP32 rounding; and
-rvs_autotune keeps one of the candidate shapes."""
+configuration), and rvs_autotune keeps one of the candidate shapes."""
 import numpy as np
 import pytest
 
@@ -23,8 +21,8 @@ def test_launch_shapes_agree(engine, wl):
     rid = engine.load_robot(w.robot)
     eid = engine.create_env(w.scene, sem)
     # bit-identical within a first-hit search: in obstacle order (variants
-    # 0-2), among all candidates in walk order (3), from the hit on (4); the
-    # searches evaluate different pairs, so their screening flags differ
+    # 0-2), among all candidates in walk order (3), from the hit on (4)
+    # (test_launch_shapes_same_bits holds all of them to the same bits)
     refs = {}
     form_of = lambda v: "ordered" if v < 3 else v
     for coh in (0, 5, 3):
