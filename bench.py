@@ -85,10 +85,10 @@ LINKS_TRAFFIC_PER_CONFIG = (2.0 * 1733610.1 + 1900112.3) * 1024 / 2097152
 # edges each, shape 8 waves per CU x 4 slots), per launch, from rocprofv3
 # counters (profiles/k_edge_first_chains_planner_starts.md): VALU wave
 # instructions, FP32 and FP64 operations executed (SQ_INSTS_VALU_FLOPS_FP32 /
-# _FP64 x 40.78 lanes active per VALU instruction) and HBM bytes (FETCH_SIZE
-# 36,718.9 KiB x 2.0 + WRITE_SIZE 2,500.3 KiB).
-EDGE_COUNTERS = {"valu_instr": 1.7790e8, "fp32_flop": 4.1102e7 * 40.78, "fp64_flop": 3.0050e7 * 40.78,
-                 "traffic_bytes": (2.0 * 36718.9 + 2500.3) * 1024,
+# _FP64 x 41.23 lanes active per VALU instruction) and HBM bytes (FETCH_SIZE
+# 37,134.6 KiB x 2.0 + WRITE_SIZE 2,597.6 KiB).
+EDGE_COUNTERS = {"valu_instr": 1.7659e8, "fp32_flop": 4.1225e7 * 41.23, "fp64_flop": 3.0058e7 * 41.23,
+                 "traffic_bytes": (2.0 * 37134.6 + 2597.6) * 1024,
                  "source": "profiles/k_edge_first_chains_planner_starts.md"}
 PEAK_FP64_TFLOPS = 78.6
 # HBM bytes per launch of the FP32 bulk kernel on the headline workload from
@@ -544,7 +544,7 @@ def underestimation_section(eng, cores: int) -> dict:
     ia, ib = gd.view(np.int32).astype(np.int64), ud.view(np.int32).astype(np.int64)
     ulp = int(np.abs(np.where(ia < 0, -(ia & 0x7FFFFFFF), ia) - np.where(ib < 0, -(ib & 0x7FFFFFFF), ib)).max())
     return {"workload": "xarm6_16aabb_ground", "configs": n, "ms": ms, "kernel_ms": float(np.min(ks)),
-            "configs_per_s": n / (ms * 1e-3), "kernel": "k_under", "stored_fraction": float(gst.mean()),
+            "configs_per_s": n / (ms * 1e-3), "kernel": "k_under_shared", "stored_fraction": float(gst.mean()),
             "stored_mismatch_vs_oracle": int((~same).sum()), "max_ulp_d_vs_oracle": ulp,
             "cpu_baseline": {"value": n / cpu_s, "unit": "configs/s", "cores": cores, "kind": "port",
                              "sample": "the same 1,048,576 configurations"}}

@@ -384,8 +384,9 @@ rvs_status rvs_edge_first_collision(rvs_context* ctx, int32_t env, const int32_t
  * a smaller obstacle tile would only add reloads); it must fit the device's
  * workgroup LDS.  Every variant screens the same pairs and gives the same
  * results bit for bit, whatever its block size, workgroups per CU or walk
- * order.  Without a recorded shape a call chooses by links x obstacles, the
- * obstacles and its batch: 0 for short walks, otherwise 1, 3 or 4. */
+ * order.  Without a recorded shape a call chooses by links, obstacles, joints,
+ * its batch and whether it can have the scratch of 4: 0 for short walks
+ * (links x obstacles below 1,024), otherwise 1, 3 or 4. */
 typedef struct rvs_tuning {
     int32_t variant;        /* 0: one lane per configuration; 1: persistent lane refill; 2: one lane per
                                configuration in persistent waves over 64-configuration chunks;
@@ -423,13 +424,19 @@ rvs_status rvs_get_tuning(rvs_context* ctx, int32_t robot, int32_t env, rvs_tuni
  * Larger batches run one lane per configuration.  0 disables; default
  * 16384 (MI355X, xArm6 and 17 boxes, spread against one lane: 1 configuration
  * 24 us vs 78 us per call, 4096: 46 us vs 294 us, 16384: 67 us vs 255 us,
- * 65536: 149 us vs 203 us, 131072: 257 us vs 202 us).  No counterpart in the
- * reference (a launch-shape choice). */
+ * 65536: 149 us vs 203 us, 131072: 257 us vs 202 us).  The two meet earlier on
+ * other scenes (planar arm, 4 boxes, 16384: 46 us vs 56 us, 32768: 60 us vs 53
+ * us; 22-DOF chain, 100 boxes, 16384: 0.94 ms vs 2.14 ms, 65536: 3.30 ms vs
+ * 1.88 ms), and the default lies below all of them; a program whose batches lie
+ * between can raise it.  No counterpart in the reference (a launch-shape
+ * choice). */
 rvs_status rvs_set_small_batch(rvs_context* ctx, int64_t max_configs);
 
 /* Launch shape of the persistent first-collision kernel: resident waves per
  * CU, and slots (edge states) per lane in one 64-lane work item, i.e. 64 *
- * slots_per_lane configurations per wavefront item. */
+ * slots_per_lane configurations per wavefront item.  Without a recorded shape
+ * 16 waves per CU, and by the slots of the call one or (from 400,000 on) two
+ * per lane. */
 typedef struct rvs_edge_tuning {
     int32_t waves_per_cu;
     int32_t slots_per_lane;
